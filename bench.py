@@ -484,10 +484,10 @@ def bench_vendor():
 
 
 def gemm_kernel_name(m, n, k, ta, tb):
-    """The kernel libhk.so runs for this shape (hk_gemm.hip's selection on 256 CUs)."""
+    """The kernel libhk.so runs for this shape: full grids of 256x256 tiles on 256 CUs, else smaller tiles."""
     if ((m + 255) // 256) * ((n + 255) // 256) >= 256 and k % 64 == 0:
         return "gemm_nt_m16_kernel"
-    return "gemm_nt_dma_kernel"
+    return "gemm_mid_kernel"
 
 
 def c4_tables(S=4096, D=128, theta=5e5):

@@ -20,6 +20,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -266,6 +267,30 @@ hk_status ensure_workspace(Ctx* c, size_t bytes) {
     return HK_OK;
 }
 
+// Workspace of an op that takes `fixed` bytes and then GEMM scratch: grows to the scratch the products
+// want, or, where that cannot be had (the workspace limit, device memory, a capturing stream, on
+// which nothing may be allocated), to what they need. *gemm_bytes: the scratch they may use.
+hk_status ensure_gemm_workspace(Ctx* c, size_t fixed, std::initializer_list<hk::GemmWorkspace> products,
+                                size_t* gemm_bytes) {
+    size_t need = 0, want = 0;
+    for (const hk::GemmWorkspace& w : products) {
+        need = std::max(need, w.need);
+        want = std::max(want, w.want);
+    }
+    hk_status st = HK_OK;
+    if (fixed + want > c->ws_bytes) {
+        bool grow = want == need;
+        if (!grow) {
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            grow = hipStreamIsCapturing(c->stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+        }
+        st = grow ? ensure_workspace(c, fixed + want) : HK_HIP_ERROR;
+        if (st == HK_HIP_ERROR && want > need) st = ensure_workspace(c, fixed + need);
+    }
+    *gemm_bytes = st == HK_OK ? c->ws_bytes - fixed : 0;
+    return st;
+}
+
 // Frees the workspace when it holds more than keep bytes (after the queued work that may use it).
 hk_status trim_workspace(Ctx* c, size_t keep) {
     if (!c->workspace || c->ws_bytes <= keep) return HK_OK;
@@ -427,10 +452,22 @@ bool out_matches(const GemmSpec& s, const hk_tensor* out) {
 }
 
 hk_status run_gemm(Ctx* c, const GemmSpec& s, const void* a, const void* b, void* out, int ta, int tb,
-                   void* ws, hipError_t* err) {
-    *err = hk::gemm_bf16(a, b, out, s.out_dtype == HK_BF16, s.batch, s.m, s.n, s.k, ta, tb, ws, c->num_cus,
-                         c->stream);
+                   void* ws, size_t ws_bytes, hipError_t* err) {
+    *err = hk::gemm_bf16(a, b, out, s.out_dtype == HK_BF16, s.batch, s.m, s.n, s.k, ta, tb, ws, ws_bytes,
+                         c->num_cus, c->stream);
     return HK_OK;
+}
+
+bool aligned16(std::initializer_list<const void*> ptrs) {
+    for (const void* p : ptrs)
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+    return true;
+}
+
+// Scratch of run_gemm with these operands (pieces of the workspace are 256-byte aligned: null here).
+hk::GemmWorkspace gemm_scratch(const Ctx* c, const GemmSpec& s, int ta, int tb, const void* a, const void* b,
+                               const void* out) {
+    return hk::gemm_workspace(s.batch, s.m, s.n, s.k, ta, tb, s.out_dtype == HK_BF16, aligned16({a, b, out}), c->num_cus);
 }
 
 // The reference's FP32-storage wrappers take F32 A/B; the GEMM runs on BF16 copies.
@@ -684,10 +721,11 @@ hk_status hk_gemm_into(hk_context* h, const hk_tensor* a, const hk_tensor* b, in
     if (!disjoint({out}, {a, b})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    st = ensure_workspace(g.c, hk::gemm_workspace_bytes(s.batch, s.m, s.n, s.k, ta, tb));
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a->data, b->data, out->data)}, &gb);
     if (st != HK_OK) return st;
     hipError_t e;
-    run_gemm(g.c, s, a->data, b->data, out->data, ta, tb, g.c->workspace, &e);
+    run_gemm(g.c, s, a->data, b->data, out->data, ta, tb, g.c->workspace, gb, &e);
     return complete(g.c, e, "gemm", 1);
 }
 
@@ -1335,12 +1373,13 @@ hk_status hk_linear_nt_backward(hk_context* h, const hk_tensor* x, const hk_tens
     if (!disjoint({dx, dw}, {x, w, dy})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    size_t ws = std::max(hk::gemm_workspace_bytes(1, sdx.m, sdx.n, sdx.k, HK_NO, HK_NO),
-                         hk::gemm_workspace_bytes(1, sdw.m, sdw.n, sdw.k, HK_YES, HK_NO));
-    if ((st = ensure_workspace(g.c, ws)) != HK_OK) return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, dy->data, w->data, dx->data),
+                                        gemm_scratch(g.c, sdw, HK_YES, HK_NO, dy->data, x->data, dw->data)}, &gb);
+    if (st != HK_OK) return st;
     hipError_t e;
-    run_gemm(g.c, sdx, dy->data, w->data, dx->data, HK_NO, HK_NO, g.c->workspace, &e);
-    if (e == hipSuccess) run_gemm(g.c, sdw, dy->data, x->data, dw->data, HK_YES, HK_NO, g.c->workspace, &e);
+    run_gemm(g.c, sdx, dy->data, w->data, dx->data, HK_NO, HK_NO, g.c->workspace, gb, &e);
+    if (e == hipSuccess) run_gemm(g.c, sdw, dy->data, x->data, dw->data, HK_YES, HK_NO, g.c->workspace, gb, &e);
     return complete(g.c, e, "linear_nt_backward", 2);
 }
 
@@ -1357,10 +1396,12 @@ hk_status hk_gemm_bf16_fp32(hk_context* h, const hk_tensor* a, const hk_tensor* 
     if (!disjoint({out, a_bf16, b_bf16}, {a, b})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, hk::gemm_workspace_bytes(s.batch, s.m, s.n, s.k, ta, tb))) != HK_OK) return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a_bf16->data, b_bf16->data, out->data)}, &gb);
+    if (st != HK_OK) return st;
     hipError_t e = hk::cast_apply(1, a->data, a_bf16->data, numel(a), g.c->stream);
     if (e == hipSuccess) e = hk::cast_apply(1, b->data, b_bf16->data, numel(b), g.c->stream);
-    if (e == hipSuccess) run_gemm(g.c, s, a_bf16->data, b_bf16->data, out->data, ta, tb, g.c->workspace, &e);
+    if (e == hipSuccess) run_gemm(g.c, s, a_bf16->data, b_bf16->data, out->data, ta, tb, g.c->workspace, gb, &e);
     return complete(g.c, e, "gemm_bf16_fp32", 3);
 }
 
@@ -1393,15 +1434,16 @@ hk_status hk_gemm_bf16_fp32_backward(hk_context* h, const hk_tensor* a, const hk
     const size_t dy_bytes = (static_cast<size_t>(numel(dy)) * 2 + 255) & ~size_t(255);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    const size_t ws = dy_bytes + std::max(hk::gemm_workspace_bytes(sdx.batch, sdx.m, sdx.n, sdx.k, dx_ta, dx_tb),
-                                          hk::gemm_workspace_bytes(sdw.batch, sdw.m, sdw.n, sdw.k, dw_ta, dw_tb));
-    if ((st = ensure_workspace(g.c, ws)) != HK_OK) return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, dy_bytes, {gemm_scratch(g.c, sdx, dx_ta, dx_tb, a->data, b->data, da->data),
+                                               gemm_scratch(g.c, sdw, dw_ta, dw_tb, a->data, b->data, db->data)}, &gb);
+    if (st != HK_OK) return st;
     void* dyb_ptr = g.c->workspace;
     void* gws = static_cast<char*>(g.c->workspace) + dy_bytes;
     dyb.data = dyb_ptr;
     hipError_t e = hk::cast_apply(1, dy->data, dyb_ptr, numel(dy), g.c->stream);
-    if (e == hipSuccess) run_gemm(g.c, sdx, dx_a->data, dx_b->data, da->data, dx_ta, dx_tb, gws, &e);
-    if (e == hipSuccess) run_gemm(g.c, sdw, dw_a->data, dw_b->data, db->data, dw_ta, dw_tb, gws, &e);
+    if (e == hipSuccess) run_gemm(g.c, sdx, dx_a->data, dx_b->data, da->data, dx_ta, dx_tb, gws, gb, &e);
+    if (e == hipSuccess) run_gemm(g.c, sdw, dw_a->data, dw_b->data, db->data, dw_ta, dw_tb, gws, gb, &e);
     return complete(g.c, e, "gemm_bf16_fp32_backward", 3);
 }
 
@@ -1446,12 +1488,13 @@ hk_status hk_linear_frozen_bf16_fp32(hk_context* h, const hk_tensor* x, const hk
     const size_t x_bytes = (static_cast<size_t>(numel(x)) * 2 + 255) & ~size_t(255);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, x_bytes + hk::gemm_workspace_bytes(1, s.m, s.n, s.k, HK_NO, HK_YES))) != HK_OK)
-        return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, x_bytes, {gemm_scratch(g.c, s, HK_NO, HK_YES, nullptr, w->data, y->data)}, &gb);
+    if (st != HK_OK) return st;
     void* xb = g.c->workspace;
     hipError_t e = hk::cast_apply(1, x->data, xb, numel(x), g.c->stream);
     if (e == hipSuccess)
-        run_gemm(g.c, s, xb, w->data, y->data, HK_NO, HK_YES, static_cast<char*>(g.c->workspace) + x_bytes, &e);
+        run_gemm(g.c, s, xb, w->data, y->data, HK_NO, HK_YES, static_cast<char*>(g.c->workspace) + x_bytes, gb, &e);
     return complete(g.c, e, "linear_frozen_bf16_fp32", 2);
 }
 
@@ -1473,12 +1516,13 @@ hk_status hk_linear_frozen_bf16_fp32_backward(hk_context* h, const hk_tensor* w,
     const size_t dy_bytes = (static_cast<size_t>(numel(dy)) * 2 + 255) & ~size_t(255);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, dy_bytes + hk::gemm_workspace_bytes(1, s.m, s.n, s.k, HK_NO, HK_NO))) != HK_OK)
-        return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, dy_bytes, {gemm_scratch(g.c, s, HK_NO, HK_NO, nullptr, w->data, dx->data)}, &gb);
+    if (st != HK_OK) return st;
     void* dyb_ptr = g.c->workspace;
     hipError_t e = hk::cast_apply(1, dy->data, dyb_ptr, numel(dy), g.c->stream);
     if (e == hipSuccess)
-        run_gemm(g.c, s, dyb_ptr, w->data, dx->data, HK_NO, HK_NO, static_cast<char*>(g.c->workspace) + dy_bytes, &e);
+        run_gemm(g.c, s, dyb_ptr, w->data, dx->data, HK_NO, HK_NO, static_cast<char*>(g.c->workspace) + dy_bytes, gb, &e);
     return complete(g.c, e, "linear_frozen_bf16_fp32_backward", 2);
 }
 
@@ -1566,15 +1610,17 @@ hk_status hk_gemm_padded_bf16_fp32(hk_context* h, const hk_tensor* a, const hk_t
     const size_t out_bytes = crop ? ws_round(static_cast<size_t>(s.batch * s.m * s.n) * 4) : 0;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, out_bytes + hk::gemm_workspace_bytes(s.batch, s.m, s.n, s.k, ta, tb))) != HK_OK)
-        return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, out_bytes, {gemm_scratch(g.c, s, ta, tb, a_pad->data, b_pad->data,
+                                                             crop ? nullptr : out->data)}, &gb);
+    if (st != HK_OK) return st;
     float* native_out = crop ? static_cast<float*>(g.c->workspace) : static_cast<float*>(out->data);
     void* gws = static_cast<char*>(g.c->workspace) + out_bytes;
     const int64_t ar = p.a_pad.shape[p.rank - 2], ac = p.a_pad.shape[p.rank - 1];
     const int64_t br = p.b_pad.shape[p.rank - 2], bc = p.b_pad.shape[p.rank - 1];
     hipError_t e = hk::pad_bf16(0, a->data, a_pad->data, p.batch, p.a_rows, p.a_cols, ar, ac, g.c->stream);
     if (e == hipSuccess) e = hk::pad_bf16(0, b->data, b_pad->data, p.batch, p.b_rows, p.b_cols, br, bc, g.c->stream);
-    if (e == hipSuccess) run_gemm(g.c, s, a_pad->data, b_pad->data, native_out, ta, tb, gws, &e);
+    if (e == hipSuccess) run_gemm(g.c, s, a_pad->data, b_pad->data, native_out, ta, tb, gws, gb, &e);
     if (e == hipSuccess && crop)
         e = hk::crop_f32(native_out, static_cast<float*>(out->data), p.batch, p.m, p.n, s.m, s.n, g.c->stream);
     return complete(g.c, e, "gemm_padded_bf16_fp32", crop ? 4 : 3);
@@ -1617,9 +1663,12 @@ hk_status hk_gemm_padded_bf16_fp32_backward(hk_context* h, const hk_tensor* a_pa
     const size_t pb_bytes = crop_b ? ws_round(static_cast<size_t>(numel(&p.b_pad)) * 4) : 0;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    const size_t gws_bytes = std::max(hk::gemm_workspace_bytes(sda.batch, sda.m, sda.n, sda.k, da_ta, da_tb),
-                                      hk::gemm_workspace_bytes(sdb.batch, sdb.m, sdb.n, sdb.k, db_ta, db_tb));
-    if ((st = ensure_workspace(g.c, dy_bytes + pa_bytes + pb_bytes + gws_bytes)) != HK_OK) return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, dy_bytes + pa_bytes + pb_bytes,
+                               {gemm_scratch(g.c, sda, da_ta, da_tb, a_pad->data, b_pad->data, crop_a ? nullptr : da->data),
+                                gemm_scratch(g.c, sdb, db_ta, db_tb, a_pad->data, b_pad->data, crop_b ? nullptr : db->data)},
+                               &gb);
+    if (st != HK_OK) return st;
     char* w = static_cast<char*>(g.c->workspace);
     dyp.data = w;
     float* pa = crop_a ? reinterpret_cast<float*>(w + dy_bytes) : static_cast<float*>(da->data);
@@ -1627,8 +1676,8 @@ hk_status hk_gemm_padded_bf16_fp32_backward(hk_context* h, const hk_tensor* a_pa
     void* gws = w + dy_bytes + pa_bytes + pb_bytes;
     int kernels = 3;
     hipError_t e = hk::pad_bf16(0, dy->data, dyp.data, p.batch, p.m, p.n, s.m, s.n, g.c->stream);
-    if (e == hipSuccess) run_gemm(g.c, sda, da_a->data, da_b->data, pa, da_ta, da_tb, gws, &e);
-    if (e == hipSuccess) run_gemm(g.c, sdb, db_a->data, db_b->data, pb, db_ta, db_tb, gws, &e);
+    if (e == hipSuccess) run_gemm(g.c, sda, da_a->data, da_b->data, pa, da_ta, da_tb, gws, gb, &e);
+    if (e == hipSuccess) run_gemm(g.c, sdb, db_a->data, db_b->data, pb, db_ta, db_tb, gws, gb, &e);
     const int64_t ar = p.a_pad.shape[p.rank - 2], ac = p.a_pad.shape[p.rank - 1];
     const int64_t br = p.b_pad.shape[p.rank - 2], bc = p.b_pad.shape[p.rank - 1];
     if (e == hipSuccess && crop_a) {
@@ -1668,8 +1717,11 @@ hk_status hk_linear_frozen_padded_bf16_fp32(hk_context* h, const hk_tensor* x, c
     const size_t ob = crop ? ws_round(static_cast<size_t>(s.m * s.n) * 4) : 0;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, xb + wb + ob + hk::gemm_workspace_bytes(1, s.m, s.n, s.k, HK_NO, HK_YES))) != HK_OK)
-        return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, xb + wb + ob,
+                               {gemm_scratch(g.c, s, HK_NO, HK_YES, nullptr, w_pad ? w_pad->data : w_tail ? nullptr : w->data,
+                                             crop ? nullptr : y->data)}, &gb);
+    if (st != HK_OK) return st;
     char* ws = static_cast<char*>(g.c->workspace);
     void* xpad = ws;
     // aligned weights are used in place (reference: "aligned weights reuse their actual handle")
@@ -1683,7 +1735,7 @@ hk_status hk_linear_frozen_padded_bf16_fp32(hk_context* h, const hk_tensor* x, c
         ++kernels;
     }
     float* native_out = crop ? reinterpret_cast<float*>(ws + xb + wb) : static_cast<float*>(y->data);
-    if (e == hipSuccess) run_gemm(g.c, s, xpad, wuse, native_out, HK_NO, HK_YES, ws + xb + wb + ob, &e);
+    if (e == hipSuccess) run_gemm(g.c, s, xpad, wuse, native_out, HK_NO, HK_YES, ws + xb + wb + ob, gb, &e);
     if (e == hipSuccess && crop) {
         e = hk::crop_f32(native_out, static_cast<float*>(y->data), 1, p.m, p.n, s.m, s.n, g.c->stream);
         ++kernels;
@@ -1718,12 +1770,14 @@ hk_status hk_linear_frozen_padded_bf16_fp32_backward(hk_context* h, const hk_ten
     const size_t ob = crop ? ws_round(static_cast<size_t>(s.m * s.k) * 4) : 0;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, db + ob + hk::gemm_workspace_bytes(1, sdx.m, sdx.n, sdx.k, HK_NO, HK_NO))) != HK_OK)
-        return st;
+    size_t gb;
+    st = ensure_gemm_workspace(g.c, db + ob, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, nullptr, w_pad->data, crop ? nullptr : dx->data)},
+                               &gb);
+    if (st != HK_OK) return st;
     char* ws = static_cast<char*>(g.c->workspace);
     float* native_out = crop ? reinterpret_cast<float*>(ws + db) : static_cast<float*>(dx->data);
     hipError_t e = hk::pad_bf16(0, dy->data, ws, 1, p.m, p.n, s.m, s.n, g.c->stream);
-    if (e == hipSuccess) run_gemm(g.c, sdx, ws, w_pad->data, native_out, HK_NO, HK_NO, ws + db + ob, &e);
+    if (e == hipSuccess) run_gemm(g.c, sdx, ws, w_pad->data, native_out, HK_NO, HK_NO, ws + db + ob, gb, &e);
     if (e == hipSuccess && crop)
         e = hk::crop_f32(native_out, static_cast<float*>(dx->data), 1, p.m, p.k, s.m, s.k, g.c->stream);
     return complete(g.c, e, "linear_frozen_padded_bf16_fp32_backward", crop ? 3 : 2);
@@ -2751,6 +2805,23 @@ struct Carve {
     }
 };
 
+// Workspace for a plan(carve, error, context or null, CUs): what it takes with the scratch its
+// products want, else (no memory, the limit, a capturing stream) with what they need (*lean set).
+hk_status ensure_planned(Ctx* c, const std::function<void(Carve&, hipError_t*, Ctx*, int)>& plan, bool* lean) {
+    hipError_t e = hipSuccess;
+    size_t bytes[2];
+    for (int i = 0; i < 2; ++i) {
+        *lean = i == 1;
+        Carve size{nullptr};
+        plan(size, &e, nullptr, c->num_cus);
+        bytes[i] = size.used;
+    }
+    size_t granted;
+    const hk_status st = ensure_gemm_workspace(c, 0, {{bytes[1], bytes[0]}}, &granted);
+    *lean = granted < bytes[0];
+    return st;
+}
+
 // BF16 operand: `t` itself when BF16, else its RNE rounding into the workspace.
 const void* bf16_operand(const hk_tensor* t, Carve& w, hipError_t* e, hipStream_t s) {
     if (t->dtype == HK_BF16) return t->data;
@@ -2761,22 +2832,31 @@ const void* bf16_operand(const hk_tensor* t, Carve& w, hipError_t* e, hipStream_
 
 // S = bf16(Q) bf16(K)^T * scale (+ mask) and P = softmax(S), both F32 [B*Hkv, rows, N].
 void composed_probs(const ComposedShape& sh, const void* qb, const void* kb, float scale, const hk_tensor* mask,
-                    float* sbuf, float* p, void* gws, int num_cus, hipStream_t s, hipError_t* e) {
+                    float* sbuf, float* p, void* gws, size_t gb, int num_cus, hipStream_t s, hipError_t* e) {
     const int64_t G = sh.groups(), R = sh.rows();
-    if (*e == hipSuccess) *e = hk::gemm_bf16(qb, kb, sbuf, false, G, R, sh.n, sh.d, HK_NO, HK_YES, gws, num_cus, s);
+    if (*e == hipSuccess) *e = hk::gemm_bf16(qb, kb, sbuf, false, G, R, sh.n, sh.d, HK_NO, HK_YES, gws, gb, num_cus, s);
     if (*e == hipSuccess)
         *e = hk::scale_mask(sbuf, mask ? static_cast<const float*>(mask->data) : nullptr, scale, sh.scores(), s);
     if (*e == hipSuccess) *e = hk::softmax_forward(sbuf, p, G * R, sh.n, 0, s);
 }
 
-size_t composed_gemm_ws(const ComposedShape& sh) {
+// GEMM scratch of the composed path's products: what they need (lean) or what they want. `aligned`:
+// every caller tensor they read or write is 16-byte aligned.
+size_t composed_gemm_ws(const ComposedShape& sh, bool aligned, bool lean, int cus) {
     const int64_t G = sh.groups(), R = sh.rows();
-    size_t w = hk::gemm_workspace_bytes(G, R, sh.n, sh.d, HK_NO, HK_YES);
-    w = std::max(w, hk::gemm_workspace_bytes(G, R, sh.dv, sh.n, HK_NO, HK_NO));   // O, dQ (Dv or D wide)
-    w = std::max(w, hk::gemm_workspace_bytes(G, R, sh.d, sh.n, HK_NO, HK_NO));
-    w = std::max(w, hk::gemm_workspace_bytes(G, R, sh.n, sh.dv, HK_NO, HK_YES));  // dP
-    w = std::max(w, hk::gemm_workspace_bytes(G, sh.n, sh.d, R, HK_YES, HK_NO));   // dK
-    w = std::max(w, hk::gemm_workspace_bytes(G, sh.n, sh.dv, R, HK_YES, HK_NO));  // dV
+    size_t w = 0;
+    auto add = [&](int64_t m, int64_t n, int64_t k, int ta, int tb) {
+        for (bool bf16 : {false, true}) {
+            const hk::GemmWorkspace g = hk::gemm_workspace(G, m, n, k, ta, tb, bf16, aligned, cus);
+            w = std::max(w, lean ? g.need : g.want);
+        }
+    };
+    add(R, sh.n, sh.d, HK_NO, HK_YES);   // S
+    add(R, sh.dv, sh.n, HK_NO, HK_NO);   // O
+    add(R, sh.d, sh.n, HK_NO, HK_NO);    // dQ
+    add(R, sh.n, sh.dv, HK_NO, HK_YES);  // dP
+    add(sh.n, sh.d, R, HK_YES, HK_NO);   // dK
+    add(sh.n, sh.dv, R, HK_YES, HK_NO);  // dV
     return w;
 }
 
@@ -2792,29 +2872,30 @@ hk_status hk_attention_masked_forward(hk_context* h, const hk_tensor* q, const h
         return fail(HK_INVALID_ARGUMENT, "O must be F32 (or BF16) shaped like Q with the value width");
     if (mask ? !disjoint({o}, {q, k, v, mask}) : !disjoint({o}, {q, k, v})) return HK_INVALID_ARGUMENT;
     const int64_t G = sh.groups(), R = sh.rows();
-    auto plan = [&](Carve& w, hipError_t* e, Ctx* c) {
+    const bool aligned = aligned16({q->data, k->data, v->data, o->data});
+    bool lean = false;
+    auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
         const void* qb = bf16_operand(q, w, e, c ? c->stream : nullptr);
         const void* kb = bf16_operand(k, w, e, c ? c->stream : nullptr);
         const void* vb = bf16_operand(v, w, e, c ? c->stream : nullptr);
         float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));
         float* p = static_cast<float*>(w.take(sh.scores() * 4));
         void* pb = w.take(sh.scores() * 2);
-        void* gws = w.take(composed_gemm_ws(sh));
+        const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
+        void* gws = w.take(gb);
         if (!c) return;
-        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, c->num_cus, c->stream, e);
+        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, gb, cus, c->stream, e);
         if (*e == hipSuccess) *e = hk::cast_apply(1, p, pb, sh.scores(), c->stream);
         if (*e == hipSuccess)
             *e = hk::gemm_bf16(pb, vb, o->data, o->dtype == HK_BF16, G, R, sh.dv, sh.n, HK_NO, HK_NO, gws,
-                               c->num_cus, c->stream);
+                               gb, cus, c->stream);
     };
-    Carve size{nullptr};
-    hipError_t e = hipSuccess;
-    plan(size, &e, nullptr);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, size.used)) != HK_OK) return st;
+    hipError_t e = hipSuccess;
+    if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
-    plan(w, &e, g.c);
+    plan(w, &e, g.c, g.c->num_cus);
     return complete(g.c, e, "attention_masked_forward", 6);
 }
 
@@ -2849,7 +2930,9 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
             if (overlaps(outs[i], outs[j])) return fail(HK_INVALID_ARGUMENT, "outputs overlap each other");
     }
     const int64_t G = sh.groups(), R = sh.rows();
-    auto plan = [&](Carve& w, hipError_t* e, Ctx* c) {
+    const bool aligned = aligned16({q->data, k->data, v->data, dout->data, dq->data, dk->data, dv->data});
+    bool lean = false;
+    auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
         hipStream_t s = c ? c->stream : nullptr;
         const void* qb = bf16_operand(q, w, e, s);
         const void* kb = bf16_operand(k, w, e, s);
@@ -2859,33 +2942,31 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
         float* p = static_cast<float*>(w.take(sh.scores() * 4));
         float* ds = dmask ? static_cast<float*>(dmask->data) : static_cast<float*>(w.take(sh.scores() * 4));
         void* b16 = w.take(sh.scores() * 2);  // bf16(scale * dS), then bf16(P)
-        void* gws = w.take(composed_gemm_ws(sh));
+        const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
+        void* gws = w.take(gb);
         if (!c) return;
-        const int cus = c->num_cus;
         // recompute P (the reference keeps it in its autodiff graph)
-        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, cus, s, e);
+        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, gb, cus, s, e);
         // dP = bf16(dO) bf16(V)^T; dS = P * (dP - rowsum(P * dP)) (softmax_backward); dMask = dS
-        if (*e == hipSuccess) *e = hk::gemm_bf16(dob, vb, sbuf, false, G, R, sh.n, sh.dv, HK_NO, HK_YES, gws, cus, s);
+        if (*e == hipSuccess) *e = hk::gemm_bf16(dob, vb, sbuf, false, G, R, sh.n, sh.dv, HK_NO, HK_YES, gws, gb, cus, s);
         if (*e == hipSuccess) *e = hk::softmax_backward(p, sbuf, ds, G * R, sh.n, 0, s);
         // dQ = bf16(scale dS) bf16(K); dK = bf16(scale dS)^T bf16(Q) (the group's heads summed in the GEMM)
         if (*e == hipSuccess) *e = hk::scale_to_bf16(ds, scale, b16, sh.scores(), s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, kb, dq->data, dq->dtype == HK_BF16, G, R, sh.d, sh.n, HK_NO, HK_NO, gws, cus, s);
+            *e = hk::gemm_bf16(b16, kb, dq->data, dq->dtype == HK_BF16, G, R, sh.d, sh.n, HK_NO, HK_NO, gws, gb, cus, s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, qb, dk->data, dk->dtype == HK_BF16, G, sh.n, sh.d, R, HK_YES, HK_NO, gws, cus, s);
+            *e = hk::gemm_bf16(b16, qb, dk->data, dk->dtype == HK_BF16, G, sh.n, sh.d, R, HK_YES, HK_NO, gws, gb, cus, s);
         // dV = bf16(P)^T bf16(dO)
         if (*e == hipSuccess) *e = hk::cast_apply(1, p, b16, sh.scores(), s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, dob, dv->data, dv->dtype == HK_BF16, G, sh.n, sh.dv, R, HK_YES, HK_NO, gws, cus, s);
+            *e = hk::gemm_bf16(b16, dob, dv->data, dv->dtype == HK_BF16, G, sh.n, sh.dv, R, HK_YES, HK_NO, gws, gb, cus, s);
     };
-    Carve size{nullptr};
-    hipError_t e = hipSuccess;
-    plan(size, &e, nullptr);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, size.used)) != HK_OK) return st;
+    hipError_t e = hipSuccess;
+    if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
-    plan(w, &e, g.c);
+    plan(w, &e, g.c, g.c->num_cus);
     return complete(g.c, e, "attention_masked_backward", 11);
 }
 

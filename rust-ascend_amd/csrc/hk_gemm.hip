@@ -12,12 +12,13 @@
 //     global->LDS loads; a K-contiguous operand (A [M,K], B [N,K]) is staged in 128-byte k-rows
 //     and read with 16-byte LDS reads, an MN-contiguous one (A stored [K,M] or B stored [K,N]) in
 //     512-byte rows of 256 columns and read with transposing LDS reads.
-//   * Smaller problems: MN-contiguous operands are first transposed into the workspace by an
-//     HBM-bound kernel, then a workgroup of 4 wavefronts (2x2) computes a BMxBN output tile (256, 128 or 64
-//     when a larger grid would not fill the 256 CUs). Each wave owns a (BM/2)x(BN/2) block of
-//     32x32 MFMA tiles, v_mfma_f32_32x32x16_bf16, accumulators in the AGPR half of the
-//     register file.
-//   * K loop in steps of BK = 64: A and B slices are prefetched from HBM into registers one
+//   * Smaller problems -> gemm_mid_kernel (hk_gemm_mid.hpp): tiles from 256x128 down to 32x64 with
+//     the same MFMAs, in-place transposes and global->LDS loads, K split over workgroups where
+//     even those tiles are too few; pick_gemm estimates each shape's time per tile and split.
+//   * Operands past 32-bit byte offsets or off 16-byte alignment -> gemm_nt_kernel: MN-contiguous
+//     operands are first transposed into the workspace, then four wavefronts (2x2) compute a
+//     BMxBN output tile (256, 128 or 64) of v_mfma_f32_32x32x16_bf16.
+//   * gemm_nt_kernel's K loop in steps of BK = 64: A and B slices are prefetched from HBM into registers one
 //     step ahead, written to a double-buffered LDS tile (rows of 64 BF16 = 128 B, 16-byte
 //     chunks XOR-swizzled by row%8 so both the row-contiguous writes and the 32-row
 //     fragment reads are bank-conflict-free), one barrier per step.
@@ -28,6 +29,7 @@
 //     slices run on the same XCD's L2.
 #include "hk_common.hpp"
 #include "hk_gemm_device.hpp"
+#include "hk_gemm_mid.hpp"
 #include "hk_kernels.hpp"
 
 namespace hk {
@@ -175,265 +177,6 @@ gemm_nt_kernel(GemmArgs p) {
     }
 }
 
-// Same GEMM for K % 32 == 0, with the operand slices moved by the global->LDS path
-// (buffer_load ... lds) instead of through registers:
-//   * K steps of 32 rotate through four LDS stages, so the loads of step kt+3 are in flight
-//     while step kt is multiplied (no staging registers, no ds_write instructions);
-//   * the stages are four separately declared arrays and the K loop is unrolled by four, so
-//     every access names its stage statically: the compiler can then tell the loads into one
-//     stage from the fragment reads of another and does not make the reads wait for them;
-//   * a stage row is 32 BF16 = 64 B = 4 chunks of 16 B; the chunk index is XORed with
-//     (row/4)%4. gfx950's LDS serves a 16-byte read for 16 lanes per clock (64 banks), and
-//     a fragment read has 16 consecutive rows at the same chunk in those lanes: four rows share
-//     each 256-byte bank line, and the XOR moves the four to distinct chunks, so the 16 reads
-//     hit 16 distinct bank groups (measured: 2x the throughput of a (row/2)%4 swizzle). Each
-//     wave load instruction fills 1 KB of consecutive LDS (16 rows), so lane l fetches the
-//     global chunk the swizzle places at its position (row l/4, chunk (l%4) ^ ((l/16) % 4));
-//   * each step is two 16-wide k slices ("phases"); a phase issues the next slice's fragment
-//     reads, then the current slice's MFMAs, and the compiler may not reorder across phases.
-constexpr int kSBK = 32;       // K per stage (four stages)
-__device__ __forceinline__ int swz32(int row, int chunk) {  // element offset in a [rows][32] stage
-    return row * kSBK + ((chunk ^ ((row >> 2) & 3)) << 3);
-}
-
-// This wave's MFMA operands for one 16-wide k slice of a stage.
-template <int BM, int BN>
-struct Frags {
-    bf16x8_t a[BM / 64];
-    bf16x8_t b[BN / 64];
-};
-
-template <int BM, int BN>
-__device__ __forceinline__ void read_frags(const uint16_t* stage, int ks, int wm, int wn, int lr, int lk,
-                                           Frags<BM, BN>& f) {
-    const int c = ks * 2 + lk;
-    const uint16_t* lb = stage + BM * kSBK;
-#pragma unroll
-    for (int i = 0; i < BM / 64; ++i)
-        f.a[i] = *reinterpret_cast<const bf16x8_t*>(stage + swz32(wm * (BM / 2) + i * 32 + lr, c));
-#pragma unroll
-    for (int j = 0; j < BN / 64; ++j)
-        f.b[j] = *reinterpret_cast<const bf16x8_t*>(lb + swz32(wn * (BN / 2) + j * 32 + lr, c));
-}
-
-// The empty asm pins the fragments to VGPRs (the accumulators fill the AGPR file; left to
-// itself the register allocator may park fragments there and spill accumulators).
-template <int BM, int BN>
-__device__ __forceinline__ void mma_frags(Frags<BM, BN>& f, f32x16_t (&acc)[BM / 64][BN / 64]) {
-#pragma unroll
-    for (int i = 0; i < BM / 64; ++i) asm volatile("" : "+v"(f.a[i]));
-#pragma unroll
-    for (int j = 0; j < BN / 64; ++j) asm volatile("" : "+v"(f.b[j]));
-#pragma unroll
-    for (int i = 0; i < BM / 64; ++i)
-#pragma unroll
-        for (int j = 0; j < BN / 64; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
-}
-
-// Fragment r of a slice: r < TI is A fragment r, otherwise B fragment r - TI.
-template <int BM, int BN>
-__device__ __forceinline__ void read_frag(const uint16_t* stage, int ks, int r, int wm, int wn, int lr, int lk,
-                                          Frags<BM, BN>& f) {
-    constexpr int TI = BM / 64;
-    const int c = ks * 2 + lk;
-    if (r < TI)
-        f.a[r] = *reinterpret_cast<const bf16x8_t*>(stage + swz32(wm * (BM / 2) + r * 32 + lr, c));
-    else
-        f.b[r - TI] =
-            *reinterpret_cast<const bf16x8_t*>(stage + BM * kSBK + swz32(wn * (BN / 2) + (r - TI) * 32 + lr, c));
-}
-
-// One phase: the MFMAs of the current slice (fragments in cur) with, spread between them
-// in this order, the reads of the next slice's fragments (read(r), r < TI + TJ, one after
-// each of the first MFMAs, so they complete well before the next phase needs them) and P
-// global->LDS loads (load(d)). Spreading matters because issue is in order: a burst of LDS or
-// memory instructions that the memory pipelines accept slowly would hold back the MFMAs
-// behind it. The compiler may not reorder across the fences.
-template <int BM, int BN, int P, class Read, class Load>
-__device__ __forceinline__ void mma_phase(Frags<BM, BN>& cur, f32x16_t (&acc)[BM / 64][BN / 64], Read&& read,
-                                          Load&& load) {
-    constexpr int TI = BM / 64, TJ = BN / 64, NM = TI * TJ, NR = TI + TJ;
-#pragma unroll
-    for (int i = 0; i < TI; ++i) asm volatile("" : "+v"(cur.a[i]));
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) asm volatile("" : "+v"(cur.b[j]));
-    phase_fence();
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi) {
-        const int i = mi / TJ, j = mi % TJ;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[j], cur.a[i], acc[i][j], 0, 0, 0);
-        phase_fence();
-        // reads: r in [mi*NR/NM', ...) over the first NM' = max(NM/2, 1) MFMAs
-        constexpr int NMR = NM / 2 > 0 ? NM / 2 : 1;
-#pragma unroll
-        for (int r = mi * NR / NMR; r < (mi + 1) * NR / NMR && r < NR; ++r) read(r);
-#pragma unroll
-        for (int d = mi * P / NM; d < (mi + 1) * P / NM; ++d) load(d);
-        phase_fence();
-    }
-}
-
-// mma_frags with the P global->LDS instructions of one step spread between the MFMAs, so
-// the wave issues them while the matrix core is busy instead of stalling on a burst of
-// vector memory issue. load(d) issues instruction d.
-template <int BM, int BN, int P, class Load>
-__device__ __forceinline__ void mma_frags_loads(Frags<BM, BN>& f, f32x16_t (&acc)[BM / 64][BN / 64], Load&& load) {
-    constexpr int TI = BM / 64, TJ = BN / 64, NM = TI * TJ;
-#pragma unroll
-    for (int i = 0; i < TI; ++i) asm volatile("" : "+v"(f.a[i]));
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) asm volatile("" : "+v"(f.b[j]));
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi) {
-        const int i = mi / TJ, j = mi % TJ;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
-        // loads [mi*P/NM, (mi+1)*P/NM) follow MFMA mi
-#pragma unroll
-        for (int d = mi * P / NM; d < (mi + 1) * P / NM; ++d) {
-            phase_fence();
-            load(d);
-            phase_fence();
-        }
-    }
-}
-
-
-template <int BM, int BN, bool OUT_BF16>
-__device__ __forceinline__ void store_tile(const GemmArgs& p, const f32x16_t (&acc)[BM / 64][BN / 64], int tm,
-                                           int tn, int64_t g, int wm, int wn, int lr, int lk) {
-#pragma unroll
-    for (int i = 0; i < BM / 64; ++i) {
-        const int m = tm * BM + wm * (BM / 2) + i * 32 + lr;
-        if (m >= p.m) continue;
-#pragma unroll
-        for (int j = 0; j < BN / 64; ++j) {
-#pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                const int n = tn * BN + wn * (BN / 2) + j * 32 + grp * 8 + lk * 4;
-                if (n >= p.n) continue;
-                const int64_t off = (g * p.m + m) * static_cast<int64_t>(p.n) + n;
-                if constexpr (OUT_BF16) {
-                    u32x2_t w = {pack_bf16x2(acc[i][j][grp * 4 + 0], acc[i][j][grp * 4 + 1]),
-                                 pack_bf16x2(acc[i][j][grp * 4 + 2], acc[i][j][grp * 4 + 3])};
-                    *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(p.c) + off) = w;
-                } else {
-                    f32x4_t w = {acc[i][j][grp * 4 + 0], acc[i][j][grp * 4 + 1], acc[i][j][grp * 4 + 2],
-                                 acc[i][j][grp * 4 + 3]};
-                    *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.c) + off) = w;
-                }
-            }
-        }
-    }
-}
-
-// NS LDS stages in a ring: step kt reads stage kt % NS while the loads of steps kt+1 .. kt+NS-1 are
-// in flight. A grid of at most one 64x64 tile per CU (C1's 128 tiles, 1024^3's 256) is bound by
-// that pipeline's depth: each tile walks K in 32-deep steps, each waiting for its loads, so it
-// keeps 8 stages (7 steps in flight, 64 KB of LDS); measured back to back on MI355X that takes
-// 512x1024x1024 from 6.03 to 5.80 us and 1024^3 from 6.44 to 6.15 us. Fuller grids keep 4 (with
-// 8, 512x4096x4096's 512 tiles went from 32.2 to 32.8 us).
-template <int BM, int BN, bool OUT_BF16, int NS>
-__global__ void __launch_bounds__(kThreads, (BM >= 256 ? 1 : 2))
-gemm_nt_dma_kernel(GemmArgs p) {
-    constexpr int TI = BM / 64;
-    constexpr int TJ = BN / 64;
-    constexpr int kStage = (BM + BN) * kSBK;        // elements per stage
-    constexpr int kPerWave = (BM + BN) / 16 / 4;    // 1 KB (16-row) load instructions per wave per step
-    static_assert(NS >= 4, "the barrier's wait count assumes NS - 3 whole steps in flight");
-    __shared__ __attribute__((aligned(1024))) uint16_t stages[NS][kStage];
-
-    const int tiles = p.tiles_m * p.tiles_n;
-    int bid = blockIdx.x;
-    if ((tiles & 7) == 0) bid = (bid & 7) * (tiles >> 3) + (bid >> 3);
-    constexpr int GROUP = 8;
-    const int per_group = GROUP * p.tiles_n;
-    const int first_m = (bid / per_group) * GROUP;
-    const int gsize = min(p.tiles_m - first_m, GROUP);
-    const int tm = first_m + (bid % per_group) % gsize;
-    const int tn = (bid % per_group) / gsize;
-    const int64_t g = blockIdx.z;
-    const uint16_t* A = p.a + g * static_cast<int64_t>(p.m) * p.k;
-    const uint16_t* B = weight_slice(p, tm * BM, g);
-
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31, lk = lane >> 5;
-
-    // Loads go through buffer resources over this batch's A and B. The row offset is part of
-    // the per-lane (VGPR) offset, which the hardware checks against the buffer's size, so rows
-    // past M (N) read as zero instead of reading past the matrix (the scalar offset, which
-    // carries only the K position, is not range-checked); they only feed outputs that are not
-    // stored.
-    const i32x4_t ra = buffer_resource(A, p.m * p.k * 2);
-    const i32x4_t rb = buffer_resource(B, p.n * p.k * 2);
-    // instruction i of this wave fills stage rows 16*(wave + 4*i) .. +15
-    const int r_in = lane >> 2;
-    const int voff = ((16 * wave + r_in) * p.k + ((lane & 3) ^ ((r_in >> 2) & 3)) * 8) * 2;
-    auto fetch_one = [&](uint16_t* stage, int kt, int i) {
-        const uint32_t dst = lds_address(stage + (16 * wave + 64 * i) * kSBK);
-        if (i < BM / 64)
-            load_lds16(ra, dst, voff + (tm * BM + 64 * i) * p.k * 2, kt * kSBK * 2);
-        else
-            load_lds16(rb, dst, voff + (tn * BN + 64 * (i - BM / 64)) * p.k * 2, kt * kSBK * 2);
-    };
-    auto fetch = [&](uint16_t* stage, int kt) {
-#pragma unroll
-        for (int i = 0; i < kPerWave; ++i) fetch_one(stage, kt, i);
-    };
-
-    f32x16_t acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    // Step kt multiplies stage X; its first fragments arrive in fa. Its two phases also issue
-    // the loads of step kt+NS-1 into stage Z, freed by the barrier of step kt-1. Between them the
-    // workgroup waits for step kt+1 to land in stage Y (the loads of steps kt+2 .. kt+NS-2 and the
-    // first half of step kt+NS-1 stay in flight) and meets at the barrier, and Y's first fragments
-    // are read while X's last MFMAs run. Every step issues its loads, so the wait counts are the
-    // same for all steps: past the last step the loads repeat step nk-1 into stages that are no
-    // longer read.
-    const int nk = p.k / kSBK;
-    const int last = nk - 1;
-    Frags<BM, BN> fa, fb;
-    auto step = [&](const uint16_t* X, const uint16_t* Y, uint16_t* Z, int kt) {
-        const int ahead = kt + NS - 1 < nk ? kt + NS - 1 : last;
-        // the loads of step kt+NS-1 are split over both phases (stage Z stays free until that
-        // step reads it); at the barrier the second half is still in flight
-        constexpr int P0 = (kPerWave + 1) / 2, P1 = kPerWave - P0;
-        mma_phase<BM, BN, P0>(
-            fa, acc, [&](int r) { read_frag<BM, BN>(X, 1, r, wm, wn, lr, lk, fb); },
-            [&](int d) { fetch_one(Z, ahead, d); });
-        if (kt + 1 < nk) stage_barrier<(NS - 3) * kPerWave + P0>();
-        // after the last step these reads fetch fragments that are never used
-        mma_phase<BM, BN, P1>(
-            fb, acc, [&](int r) { read_frag<BM, BN>(Y, 0, r, wm, wn, lr, lk, fa); },
-            [&](int d) { fetch_one(Z, ahead, P0 + d); });
-    };
-
-#pragma unroll
-    for (int u = 0; u < NS - 1; ++u) fetch(stages[u], nk > u ? u : last);
-    stage_barrier<(NS - 2) * kPerWave>();
-    read_frags<BM, BN>(stages[0], 0, wm, wn, lr, lk, fa);
-    int kt = 0;
-    do {  // nk >= 1: the accumulators never bypass the MFMAs on their way to the epilogue
-#pragma unroll
-        for (int u = 0; u < NS; ++u)
-            if (u == 0 || kt + u < nk) step(stages[u], stages[(u + 1) % NS], stages[(u + NS - 1) % NS], kt + u);
-        kt += NS;
-    } while (kt < nk);
-    // the trailing loads must land before the workgroup ends and its LDS is handed on
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-
-    store_tile<BM, BN, OUT_BF16>(p, acc, tm, tn, g, wm, wn, lr, lk);
-}
-
 // out[g][c][r] = in[g][r][c] for BF16, 64x64 tiles through LDS (padded rows).
 __global__ void __launch_bounds__(256)
 transpose_bf16(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int64_t rows, int64_t cols) {
@@ -452,16 +195,6 @@ transpose_bf16(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int6
         const int64_t c = c0 + i, r = r0 + tx;
         if (r < rows && c < cols) dst[c * rows + r] = tile[tx][i];
     }
-}
-
-// The 256x256-tile 4-wave kernel (every transpose) applies when there are enough tiles to fill
-// the GPU, K % 8 == 0 (a partial last stage takes the KTAIL variant) and 32-bit byte offsets
-// up to the end of the last (zero-padded) stage.
-bool pp_applies(int64_t batch, int64_t m, int64_t n, int64_t k, int num_cus) {
-    const int64_t tiles = ((m + kPPTile - 1) / kPPTile) * ((n + kPPTile - 1) / kPPTile) * batch;
-    const int64_t k64 = (k + kPK - 1) / kPK * kPK;
-    return tiles >= num_cus && k > 0 && k % 8 == 0 && m * k64 * 2 < (int64_t{1} << 31) &&
-           n * k64 * 2 < (int64_t{1} << 31);
 }
 
 // Output tile width: 256 (NJ = 8) or 192 (NJ = 6) for a grid of `batch` x M/256 x N/(32 NJ) tiles
@@ -490,11 +223,10 @@ void launch_pp_nj(const GemmArgs& p, const dim3& grid, bool a_mn, bool b_mn, hip
     else hipLaunchKernelGGL((gemm_nt_m16_kernel<OUT_BF16, false, false, false, NJ>), grid, dim3(kW4Threads), 0, s, p);
 }
 
+// nj: 8, or 6 for 192-wide tiles (whole K stages only: the KTAIL variants are square).
 template <bool OUT_BF16>
-void launch_pp(const GemmArgs& a, int64_t batch, bool a_mn, bool b_mn, int num_cus, hipStream_t s) {
+void launch_pp(const GemmArgs& a, int64_t batch, bool a_mn, bool b_mn, int nj, hipStream_t s) {
     GemmArgs p = a;
-    // narrower tiles only for whole K stages (the KTAIL variants stay square)
-    const int nj = p.k % kPK == 0 ? pick_tile_nj(batch, p.m, p.n, num_cus) : 8;
     p.tiles_m = (p.m + kPPTile - 1) / kPPTile;
     p.tiles_n = (p.n + 32 * nj - 1) / (32 * nj);
     const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n), 1, static_cast<unsigned>(batch));
@@ -515,30 +247,13 @@ void launch_pp(const GemmArgs& a, int64_t batch, bool a_mn, bool b_mn, int num_c
 }
 
 template <int BM, int BN>
-void launch_nt(const GemmArgs& a, int64_t batch, bool out_bf16, int num_cus, hipStream_t s) {
+void launch_nt(const GemmArgs& a, int64_t batch, bool out_bf16, hipStream_t s) {
     GemmArgs p = a;
     p.tiles_m = (p.m + BM - 1) / BM;
     p.tiles_n = (p.n + BN - 1) / BN;
     const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n), 1, static_cast<unsigned>(batch));
-    // the global->LDS kernel needs whole K steps and 32-bit byte offsets into A and B
-    const bool whole_steps = p.k % kSBK == 0 && p.k > 0 && static_cast<int64_t>(p.m) * p.k * 2 < (int64_t{1} << 31) &&
-                             static_cast<int64_t>(p.n) * p.k * 2 < (int64_t{1} << 31);
-    if (whole_steps && p.k % kPK == 0 && BM == kPPTile && BN == kPPTile) {
-        if (out_bf16) launch_pp<true>(p, batch, false, false, num_cus, s);
-        else launch_pp<false>(p, batch, false, false, num_cus, s);
-    } else if (whole_steps && BM == 64 && grid.x * grid.z <= static_cast<unsigned>(num_cus)) {
-        if constexpr (BM == 64) {
-            if (out_bf16) hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, true, 8>), grid, dim3(kThreads), 0, s, p);
-            else hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, false, 8>), grid, dim3(kThreads), 0, s, p);
-        }
-    } else if (whole_steps && out_bf16)
-        hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, true, 4>), grid, dim3(kThreads), 0, s, p);
-    else if (whole_steps)
-        hipLaunchKernelGGL((gemm_nt_dma_kernel<BM, BN, false, 4>), grid, dim3(kThreads), 0, s, p);
-    else if (out_bf16)
-        hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, true>), grid, dim3(kThreads), 0, s, p);
-    else
-        hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, false>), grid, dim3(kThreads), 0, s, p);
+    if (out_bf16) hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, true>), grid, dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, false>), grid, dim3(kThreads), 0, s, p);
 }
 
 // Output tile of 256, 128 or 64: the largest whose grid still fills the CUs.
@@ -546,60 +261,222 @@ void launch_nt_sized(const GemmArgs& p, int64_t batch, bool out_bf16, int num_cu
     const int64_t m = p.m, n = p.n;
     const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256) * batch;
     const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128) * batch;
-    if (t256 >= num_cus) launch_nt<256, 256>(p, batch, out_bf16, num_cus, s);
-    else if (t128 >= num_cus) launch_nt<128, 128>(p, batch, out_bf16, num_cus, s);
-    else launch_nt<64, 64>(p, batch, out_bf16, num_cus, s);
+    if (t256 >= num_cus) launch_nt<256, 256>(p, batch, out_bf16, s);
+    else if (t128 >= num_cus) launch_nt<128, 128>(p, batch, out_bf16, s);
+    else launch_nt<64, 64>(p, batch, out_bf16, s);
+}
+
+// The tile shapes a product may run on. `per_cu` workgroups share a CU; a stage of 64 k costs `k1` us
+// and a tile's start and end `t1` us with one workgroup on the CU, `k2` and `t2` (per pair) with two;
+// each further round of a single-workgroup shape costs t2 besides its stages. The figures are a
+// least-squares fit on MI355X to measured (shape, tile, split) times over 120 shapes (M 16-5600,
+// N 64-14000, K 64-14000, batches 1-32, every transpose). The choice they lead to is on average
+// 3.3% slower than the best measured one (40% at worst); the rule it replaces (the largest of 256, 128
+// and 64 whose grid fills the CUs, after a transposing pass) was on average 113% slower.
+enum GemmTile { kT256, kT256x192, kT256x128, kT128, kT128Pair, kT64x128, kT128x64, kT64, kT32x64, kTiles };
+struct TileCost {
+    int bm, bn, per_cu, slots;  // slots: K stages in the LDS ring
+    float k1, t1, k2, t2;
+};
+constexpr TileCost kTileCost[kTiles] = {
+    {256, 256, 1, 2, 1.232f, 6.44f, 0.0f, 1.08f},  {256, 192, 1, 2, 0.922f, 5.32f, 0.0f, 8.67f},
+    {256, 128, 1, 3, 0.715f, 3.72f, 0.0f, 3.67f},  {128, 128, 1, 4, 0.447f, 2.96f, 0.0f, 3.72f},
+    {128, 128, 2, 2, 0.658f, 1.88f, 0.915f, 3.42f}, {64, 128, 2, 3, 0.314f, 1.44f, 0.625f, 3.12f},
+    {128, 64, 2, 3, 0.279f, 1.63f, 0.644f, 2.74f},  {64, 64, 2, 4, 0.191f, 1.02f, 0.421f, 2.21f},
+    {32, 64, 2, 6, 0.142f, 0.94f, 0.393f, 1.55f},
+};
+
+struct GemmChoice {
+    int tile = kT64;
+    int splits = 1;
+    float us = 0.0f;
+};
+
+// Estimated time (us) of the product on one tile shape with K cut into `splits`.
+float tile_time(const TileCost& t, int64_t batch, int64_t m, int64_t n, int64_t k, bool out_bf16, int splits,
+                int num_cus) {
+    const int64_t nk = (k + kPK - 1) / kPK, per = (nk + splits - 1) / splits;
+    const int64_t wgs = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * splits;
+    const int64_t rounds = (wgs + num_cus - 1) / num_cus;
+    float us = t.per_cu == 1 ? rounds * per * t.k1 + t.t1 + (rounds - 1) * t.t2
+                             : (rounds / 2) * (per * t.k2 + t.t2) + (rounds % 2) * (per * t.k1 + t.t1);
+    const float out = static_cast<float>(batch) * m * n;
+    const float bytes = static_cast<float>(batch) * (m + n) * k * 2 + out * (splits > 1 ? 4 * splits : out_bf16 ? 2 : 4);
+    us = fmaxf(us, bytes * (bytes > 64e6f ? 1.8e-7f : 2.8e-7f));  // 5.5 TB/s; short streams reach 3.5
+    if (bytes > 64e6f) {
+        // operands past the caches arrive at the rate that the loads in flight allow over a round trip
+        // of 2.5 us (16 x 6336 x 12208: 99 workgroups 55 us, 198 36 us)
+        const int64_t resident = wgs < num_cus * t.per_cu ? wgs : num_cus * t.per_cu;
+        us = fmaxf(us, bytes * 2.5f / (static_cast<float>(resident) * (t.slots - 1) * (t.bm + t.bn) * (2 * kPK)));
+    }
+    if (splits > 1) us += 1.9f + out * 4 * (splits + 0.5f) * 2.4e-7f;  // the reducing launch, the planes
+    return us;
+}
+
+constexpr int64_t kMaxSplitBytes = int64_t{64} << 20;  // F32 partial planes of a K split
+
+// An operand slice (K rounded up to a stage) below 2^31 bytes, and unsigned 32-bit offsets up to the
+// end of its last 256-row tile.
+bool fits_32bit(int64_t rows, int64_t k) {
+    const int64_t k64 = (k + kPK - 1) / kPK * kPK;
+    return rows * k64 * 2 < (int64_t{1} << 31) && (rows + 255) / 256 * 256 * k64 * 2 < (int64_t{1} << 32);
+}
+// The kernels that read every transpose in place (buffer loads of 16 bytes): K % 8 == 0 and 16-byte
+// aligned operands. Callers' M and N are multiples of 16, so MN-major rows are aligned too.
+bool in_place_applies(int64_t m, int64_t n, int64_t k, bool aligned) {
+    return aligned && k > 0 && k % 8 == 0 && fits_32bit(m, k) && fits_32bit(n, k);
+}
+
+// The tile shape and K split of least estimated time whose partial planes fit ws_bytes. An MN-major
+// A needs tiles of at least 64 rows; 192-wide tiles take whole K stages.
+GemmChoice pick_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_mn, bool out_bf16, size_t ws_bytes,
+                     int num_cus) {
+    GemmChoice best;
+    best.us = INFINITY;
+    const int64_t nk = (k + kPK - 1) / kPK;
+    for (int t = 0; t < kTiles; ++t) {
+        const TileCost& c = kTileCost[t];
+        if ((a_mn && c.bm < 64) || (t == kT256x192 && k % kPK != 0)) continue;
+        const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * batch;
+        for (int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            // K is split only where the tiles leave CUs idle, into at least two stages each
+            const int64_t planes = batch * m * n * 4 * splits;
+            if (splits > 1 && (t <= kT256x192 || tiles >= 2 * num_cus || tiles * splits > 4 * num_cus ||
+                               nk < 2 * splits || planes > kMaxSplitBytes || static_cast<size_t>(planes) > ws_bytes))
+                break;
+            const float us = tile_time(c, batch, m, n, k, out_bf16, splits, num_cus);
+            if (us < best.us) best = GemmChoice{t, splits, us};
+        }
+    }
+    return best;
+}
+
+// The choice for a product: full grids of 256x256 tiles (at least one per CU, at most a fifth of
+// them past the output's edges) keep the 256-wide kernels; the rest take pick_gemm's.
+GemmChoice choose_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_mn, bool out_bf16, size_t ws_bytes,
+                       int num_cus) {
+    const int64_t tiles = ((m + kPPTile - 1) / kPPTile) * ((n + kPPTile - 1) / kPPTile) * batch;
+    if (tiles >= num_cus && 5 * batch * m * n >= 4 * tiles * kPPTile * kPPTile) {
+        GemmChoice c;
+        c.tile = k % kPK == 0 && pick_tile_nj(batch, m, n, num_cus) == 6 ? kT256x192 : kT256;
+        return c;
+    }
+    return pick_gemm(batch, m, n, k, a_mn, out_bf16, ws_bytes, num_cus);
+}
+
+template <int WM, int WN, int NI, int NJ, int NS, int PER_CU, bool OUT_BF16>
+void launch_mid_as(MidArgs& p, int64_t batch, bool a_mn, bool b_mn, hipStream_t s) {
+    constexpr int BM = 16 * WM * NI, BN = 16 * WN * NJ;
+    p.tiles_m = (p.m + BM - 1) / BM;
+    p.tiles_n = (p.n + BN - 1) / BN;
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits), 1, static_cast<unsigned>(batch));
+    if constexpr (BM >= 64) {
+        if (a_mn && b_mn) {
+            hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, NI, NJ, NS, true, true, OUT_BF16, kEpiPlain, PER_CU>), grid,
+                               dim3(kThreads), 0, s, p);
+            return;
+        }
+        if (a_mn) {
+            hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, NI, NJ, NS, true, false, OUT_BF16, kEpiPlain, PER_CU>), grid,
+                               dim3(kThreads), 0, s, p);
+            return;
+        }
+    }
+    if (b_mn)
+        hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, NI, NJ, NS, false, true, OUT_BF16, kEpiPlain, PER_CU>), grid,
+                           dim3(kThreads), 0, s, p);
+    else
+        hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, NI, NJ, NS, false, false, OUT_BF16, kEpiPlain, PER_CU>), grid,
+                           dim3(kThreads), 0, s, p);
+}
+
+template <int WM, int WN, int NI, int NJ, int NS, int PER_CU>
+void launch_mid(MidArgs& p, int64_t batch, bool out_bf16, bool a_mn, bool b_mn, hipStream_t s) {
+    if (out_bf16 && p.splits == 1) launch_mid_as<WM, WN, NI, NJ, NS, PER_CU, true>(p, batch, a_mn, b_mn, s);
+    else launch_mid_as<WM, WN, NI, NJ, NS, PER_CU, false>(p, batch, a_mn, b_mn, s);
+}
+
+void set_splits(MidArgs& p, int splits) {
+    const int nk = (p.k + kPK - 1) / kPK;
+    p.stages_per_split = (nk + splits - 1) / splits;
+    p.splits = (nk + p.stages_per_split - 1) / p.stages_per_split;  // every split holds a stage
+}
+
+void launch_choice(const GemmChoice& c, const GemmArgs& a, int64_t batch, bool out_bf16, bool a_mn, bool b_mn,
+                   void* workspace, hipStream_t s) {
+    if (c.tile == kT256 || c.tile == kT256x192) {
+        const int nj = c.tile == kT256 ? 8 : 6;
+        if (out_bf16) launch_pp<true>(a, batch, a_mn, b_mn, nj, s);
+        else launch_pp<false>(a, batch, a_mn, b_mn, nj, s);
+        return;
+    }
+    MidArgs p{};
+    static_cast<GemmArgs&>(p) = a;
+    set_splits(p, c.splits);
+    p.partial = static_cast<float*>(workspace);
+    switch (c.tile) {
+        case kT256x128: launch_mid<2, 2, 8, 4, 3, 1>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        case kT128: launch_mid<2, 2, 4, 4, 4, 1>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        case kT128Pair: launch_mid<2, 2, 4, 4, 2, 2>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        case kT64x128: launch_mid<2, 2, 2, 4, 3, 2>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        case kT128x64: launch_mid<2, 2, 4, 2, 3, 2>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        case kT64: launch_mid<2, 2, 2, 2, 4, 2>(p, batch, out_bf16, a_mn, b_mn, s); break;
+        default: launch_mid<1, 4, 2, 1, 6, 2>(p, batch, out_bf16, a_mn, b_mn, s); break;
+    }
+    if (p.splits == 1) return;
+    const int64_t total = batch * p.m * p.n;
+    const dim3 grid(flat_blocks(total / 4, 256));
+    if (out_bf16) hipLaunchKernelGGL((splitk_reduce<true>), grid, dim3(256), 0, s, p.partial, p.c, p.splits, total);
+    else hipLaunchKernelGGL((splitk_reduce<false>), grid, dim3(256), 0, s, p.partial, p.c, p.splits, total);
 }
 
 size_t round256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // namespace
 
-size_t gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb) {
-    size_t bytes = 0;
-    if (ta) bytes += round256(static_cast<size_t>(batch * m * k) * 2);
-    if (!tb) bytes += round256(static_cast<size_t>(batch * n * k) * 2);
-    return bytes;
+GemmWorkspace gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
+                             int num_cus) {
+    GemmWorkspace w;
+    if (in_place_applies(m, n, k, aligned)) {
+        const GemmChoice c = choose_gemm(batch, m, n, k, ta != 0, out_bf16, SIZE_MAX, num_cus);
+        if (c.splits > 1) w.want = static_cast<size_t>(batch * m * n) * 4 * c.splits;
+        return w;
+    }
+    if (ta) w.need += round256(static_cast<size_t>(batch * m * k) * 2);
+    if (!tb) w.need += round256(static_cast<size_t>(batch * n * k) * 2);
+    w.want = w.need;
+    return w;
 }
 
 hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_t batch, int64_t m, int64_t n,
-                     int64_t k, int ta, int tb, void* workspace, int num_cus, hipStream_t s) {
-    const uint16_t* ak = static_cast<const uint16_t*>(a);
-    const uint16_t* bk = static_cast<const uint16_t*>(b);
-    if (pp_applies(batch, m, n, k, num_cus)) {  // MN-major operands are read in place
-        GemmArgs p{};
-        p.a = ak;
-        p.b = bk;
-        p.c = c;
-        p.m = static_cast<int>(m);
-        p.n = static_cast<int>(n);
-        p.k = static_cast<int>(k);
-        if (out_bf16) launch_pp<true>(p, batch, ta != 0, tb == 0, num_cus, s);
-        else launch_pp<false>(p, batch, ta != 0, tb == 0, num_cus, s);
+                     int64_t k, int ta, int tb, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s) {
+    GemmArgs p{};
+    p.a = static_cast<const uint16_t*>(a);
+    p.b = static_cast<const uint16_t*>(b);
+    p.c = c;
+    p.m = static_cast<int>(m);
+    p.n = static_cast<int>(n);
+    p.k = static_cast<int>(k);
+    if (in_place_applies(m, n, k, aligned16({a, b, c}))) {
+        const GemmChoice ch = choose_gemm(batch, m, n, k, ta != 0, out_bf16 != 0, ws_bytes, num_cus);
+        launch_choice(ch, p, batch, out_bf16 != 0, ta != 0, tb == 0, workspace, s);
         return hipGetLastError();
     }
     char* ws = static_cast<char*>(workspace);
     if (ta) {  // A stored [K,M] -> [M,K]
         uint16_t* t = reinterpret_cast<uint16_t*>(ws);
         hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)((m + 63) / 64), (unsigned)((k + 63) / 64), (unsigned)batch),
-                           dim3(256), 0, s, ak, t, k, m);
-        ak = t;
+                           dim3(256), 0, s, p.a, t, k, m);
+        p.a = t;
         ws += round256(static_cast<size_t>(batch * m * k) * 2);
     }
     if (!tb) {  // B stored [K,N] -> [N,K]
         uint16_t* t = reinterpret_cast<uint16_t*>(ws);
         hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)((n + 63) / 64), (unsigned)((k + 63) / 64), (unsigned)batch),
-                           dim3(256), 0, s, bk, t, k, n);
-        bk = t;
+                           dim3(256), 0, s, p.b, t, k, n);
+        p.b = t;
     }
-    GemmArgs p{};
-    p.a = ak;
-    p.b = bk;
-    p.c = c;
-    p.m = static_cast<int>(m);
-    p.n = static_cast<int>(n);
-    p.k = static_cast<int>(k);
-    launch_nt_sized(p, batch, out_bf16, num_cus, s);
+    launch_nt_sized(p, batch, out_bf16 != 0, num_cus, s);
     return hipGetLastError();
 }
 
@@ -683,12 +560,10 @@ hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_b
     p.n = static_cast<int>(n);
     p.k = static_cast<int>(k);
     p.block_group = block_group;
-    if (pp_applies(1, m, n, k, num_cus)) {
-        if (out_bf16) launch_pp<true>(p, 1, false, false, num_cus, s);
-        else launch_pp<false>(p, 1, false, false, num_cus, s);
-    } else {
-        launch_nt_sized(p, 1, out_bf16, num_cus, s);
-    }
+    if (in_place_applies(m, n, k, aligned16({a, w, c})))
+        launch_choice(choose_gemm(1, m, n, k, false, out_bf16 != 0, 0, num_cus), p, 1, out_bf16 != 0, false, false, nullptr, s);
+    else
+        launch_nt_sized(p, 1, out_bf16 != 0, num_cus, s);
     return hipGetLastError();
 }
 

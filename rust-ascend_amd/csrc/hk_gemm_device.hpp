@@ -19,7 +19,7 @@ struct GemmArgs {
     int m, n, k;
     int tiles_m, tiles_n;
     // M-grouped form (batch 1): block_group[r / 256] is the weight slice of rows r of A and C.
-    // Group ends are multiples of 256, so an output tile (256, 128 or 64 rows) has one group.
+    // Group ends are multiples of 256, so an output tile (at most 256 rows) has one group.
     const int32_t* block_group;
     // 4-wave kernel tile order: 0 = bands of 4 M-tile rows per XCD, else bands of this many
     // N-tile columns.
@@ -125,7 +125,7 @@ __device__ __forceinline__ int swz64(int row, int chunk) {  // element offset in
 constexpr int kW4Threads = 256;
 
 // Byte offset past any operand's buffer range: a buffer load at it reads zero. The range check
-// compares the unsigned 32-bit offset with the resource's byte count, which pp_applies keeps
+// compares the unsigned 32-bit offset with the resource's byte count, which the launchers keep
 // below 2^31 (m * k * 2 <= m * k64 * 2 < 2^31), so 2^31 is out of range for every operand.
 constexpr int kOutOfRange = static_cast<int>(0x80000000u);
 
@@ -153,11 +153,10 @@ struct RopeRowIn {  // the lane's 16 angles of one row: split-half c[j] = angles
     f32x4_t s[4];   // (fragment 2q + 1)
 };
 
-template <class Args>
-__device__ __forceinline__ void store_qkv_rope(const Args& p, f32x4_t (&acc)[8][8], int tm, int tn, int wm, int wn,
-                                               int l16, int lg) {
+// m0: the lane's first row (rows m0 + 16 i); n0: the wave's first column, a head's first.
+template <int NI, class Args>
+__device__ __forceinline__ void store_qkv_rope(const Args& p, f32x4_t (&acc)[NI][8], int m0, int n0, int lg) {
     const QkvRopeOut& o = p.qkv;
-    const int n0 = tn * kPPTile + 128 * wn;
     if (n0 >= p.n) return;
     const int head = n0 >> 7;
     uint16_t* plane;
@@ -170,8 +169,7 @@ __device__ __forceinline__ void store_qkv_rope(const Args& p, f32x4_t (&acc)[8][
         plane = o.v, hx = o.hkv, hh = head - o.hq - o.hkv;
     }
     const bool rotate = head < o.hq + o.hkv;
-    const int m0 = tm * kPPTile + 128 * wm + l16;
-    constexpr int kAhead = 4;
+    constexpr int kAhead = NI < 4 ? NI : 4;
     RopeRowIn in[kAhead];
     auto load_row = [&](RopeRowIn& r, int i) __attribute__((always_inline)) {
         const int s = min(m0 + 16 * i, p.m - 1) % o.seq;  // issued for every row (no load under a branch)
@@ -198,7 +196,7 @@ __device__ __forceinline__ void store_qkv_rope(const Args& p, f32x4_t (&acc)[8][
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) load_row(in[i], i);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NI; ++i) {
         const int m = m0 + 16 * i;
         if (m < p.m) {
             const int b = m / o.seq, s = m - b * o.seq;
@@ -236,7 +234,7 @@ __device__ __forceinline__ void store_qkv_rope(const Args& p, f32x4_t (&acc)[8][
                 }
             }
         }
-        if (i + kAhead < 8) load_row(in[i % kAhead], i + kAhead);
+        if (i + kAhead < NI) load_row(in[i % kAhead], i + kAhead);
     }
 }
 
@@ -520,7 +518,7 @@ __device__ __forceinline__ void gemm_m16_tile(Args p) {
 
     if constexpr (EPI == kEpiQkvRope) {
         static_assert(NJ == 8 && OUT_BF16, "the fused QKV epilogue needs 128-column wave blocks");
-        store_qkv_rope(p, acc, tm, tn, wm, wn, l16, lg);
+        store_qkv_rope<8>(p, acc, tm * kPPTile + 128 * wm + l16, tn * kPPTile + 128 * wn, lg);
         return;
     } else if constexpr (EPI != kEpiPlain) {
         const int m0 = tm * kPPTile + 128 * wm + l16, n0 = tn * kTileN + kWaveN * wn;

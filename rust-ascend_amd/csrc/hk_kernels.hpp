@@ -45,9 +45,15 @@ hipError_t cast_apply(int to_bf16, const void* in, void* out, int64_t n, hipStre
 
 // ---- GEMM (hk_gemm.hip)
 // C[g] = op(A[g]) op(B[g]) for g < batch; A, B BF16; C BF16 or F32. ta/tb as in the
-// reference (0 = row-major [M,K] / [K,N]; 1 = [K,M] / [N,K]). Operands that are not
-// K-contiguous are first transposed into `workspace` (gemm_workspace_bytes).
-size_t gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb);
+// reference (0 = row-major [M,K] / [K,N]; 1 = [K,M] / [N,K]). Scratch of one product: `need` bytes
+// are required (operands off 16-byte alignment or past 32-bit offsets are transposed into them),
+// `want` bytes (>= need) let small grids split K; with less the product runs unsplit. `aligned`: A, B
+// and C all 16-byte aligned.
+struct GemmWorkspace {
+    size_t need = 0, want = 0;
+};
+GemmWorkspace gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
+                             int num_cus);
 
 // Generic floating matmul (hk_matmul.hip). MatmulBatch: the output's batch dims (innermost last,
 // at most 4) and one operand's element stride along each (0 where the operand broadcasts).
@@ -88,7 +94,7 @@ size_t matmul_backward_workspace_bytes(const MatmulSpec& s);
 hipError_t matmul_backward(const MatmulSpec& s, const void* a, const void* b, const void* dy, void* da, void* db,
                            void* workspace, int num_cus, hipStream_t st);
 hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_t batch, int64_t m,
-                     int64_t n, int64_t k, int ta, int tb, void* workspace, int num_cus, hipStream_t s);
+                     int64_t n, int64_t k, int ta, int tb, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s);
 // M-grouped NT GEMM: C[i, :] = A[i, :] W[g(i)]^T with A [m, k], W [groups, n, k], C [m, n];
 // g(i) = block_group[i / 256] (group ends are multiples of 256). No workspace.
 hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_bf16, int64_t m, int64_t n,
