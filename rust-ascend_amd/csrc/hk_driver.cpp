@@ -1999,7 +1999,7 @@ hk_status hk_qkv_projection_rope(hk_context* h, const hk_tensor* x, const hk_ten
     if (g.st != HK_OK) return g.st;
     hipError_t e = hk::gemm_qkv_rope(x->data, w->data, T, H, S, Hq, Hkv, static_cast<const float*>(cos->data),
                                      static_cast<const float*>(sin->data), layout, q->data, k->data, v->data,
-                                     g.c->stream);
+                                     g.c->num_cus, g.c->stream);
     return complete(g.c, e, op, 1);
 }
 
@@ -2025,7 +2025,7 @@ hk_status hk_linear_residual(hk_context* h, const hk_tensor* x, const hk_tensor*
     if (!disjoint({y}, {x, w, residual})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    hipError_t e = hk::gemm_residual(x->data, w->data, residual->data, y->data, M, N, K, g.c->stream);
+    hipError_t e = hk::gemm_residual(x->data, w->data, residual->data, y->data, M, N, K, g.c->num_cus, g.c->stream);
     return complete(g.c, e, op, 1);
 }
 
@@ -2046,7 +2046,7 @@ hk_status hk_swiglu_projection(hk_context* h, const hk_tensor* x, const hk_tenso
     if (!disjoint({gate, up, act}, {x, w_gu})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    hipError_t e = hk::gemm_swiglu(x->data, w_gu->data, gate->data, up->data, act->data, T, F, H, g.c->stream);
+    hipError_t e = hk::gemm_swiglu(x->data, w_gu->data, gate->data, up->data, act->data, T, F, H, g.c->num_cus, g.c->stream);
     return complete(g.c, e, op, 1);
 }
 
@@ -2067,7 +2067,8 @@ hk_status hk_swiglu_projection_backward(hk_context* h, const hk_tensor* dy, cons
     if (!disjoint({dgu}, {dy, wd, gate, up})) return HK_INVALID_ARGUMENT;
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    hipError_t e = hk::gemm_swiglu_backward(dy->data, wd->data, gate->data, up->data, dgu->data, T, F, H, g.c->stream);
+    hipError_t e = hk::gemm_swiglu_backward(dy->data, wd->data, gate->data, up->data, dgu->data, T, F, H, g.c->num_cus,
+                                           g.c->stream);
     return complete(g.c, e, op, 1);
 }
 

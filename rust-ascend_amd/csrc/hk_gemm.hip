@@ -491,10 +491,53 @@ bool qkv_rope_applies(int64_t tokens, int64_t hidden, int64_t width) {
 }
 
 namespace {
+// The tile of a fused-epilogue product (K is never split: the epilogue needs the whole sum): the
+// 256x256 kernel for full grids as choose_gemm has it, else the least estimated time of those built.
+// The products of a 512-token layer of hidden 2048 made 16-88 workgroups of 256x256; with these tiles
+// its two residual projections take 46 us instead of 187, gate/up 49 (66), the SwiGLU backward 28 (66)
+// and the QKV projection 20 (63).
+int pick_epi_tile(int64_t m, int64_t n, int64_t k, std::initializer_list<int> built, int num_cus) {
+    const GemmChoice full = choose_gemm(1, m, n, k, false, true, 0, num_cus);
+    if (full.us == 0.0f) return kT256;  // a full grid (not estimated)
+    int best = kT256;
+    float us = tile_time(kTileCost[kT256], 1, m, n, k, true, 1, num_cus);
+    for (int t : built) {
+        const float e = tile_time(kTileCost[t], 1, m, n, k, true, 1, num_cus);
+        if (e < us) us = e, best = t;
+    }
+    return best;
+}
+
+template <int WM, int WN, int NI, int NJ, int NS, int PER_CU, int EPI, bool B_MN>
+void launch_epi_mid(const GemmEpiArgs& a, hipStream_t s) {
+    MidArgs p{};
+    static_cast<GemmEpiArgs&>(p) = a;
+    set_splits(p, 1);
+    p.tiles_m = (p.m + 16 * WM * NI - 1) / (16 * WM * NI);
+    p.tiles_n = (p.n + 16 * WN * NJ - 1) / (16 * WN * NJ);
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n));
+    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, NI, NJ, NS, false, B_MN, true, EPI, PER_CU>), grid, dim3(kThreads), 0, s, p);
+}
+
 // A fused-epilogue GEMM over p.m x p.n outputs (256x256 tiles, bands of 8 N-tiles per XCD unless
-// the tile grid is square, as launch_pp chooses).
+// the tile grid is square, as launch_pp chooses; smaller tiles below a full grid). The QKV epilogue
+// needs a whole 128-column head per wave, so its smaller tiles stack the four waves along M.
 template <int EPI, bool B_MN>
-hipError_t launch_epi(GemmEpiArgs p, hipStream_t s) {
+hipError_t launch_epi(GemmEpiArgs p, int num_cus, hipStream_t s) {
+    if constexpr (EPI == kEpiQkvRope) {
+        switch (pick_epi_tile(p.m, p.n, p.k, {kT128Pair, kT64x128}, num_cus)) {
+            case kT128Pair: launch_epi_mid<4, 1, 2, 8, 2, 2, EPI, B_MN>(p, s); return hipGetLastError();
+            case kT64x128: launch_epi_mid<4, 1, 1, 8, 3, 2, EPI, B_MN>(p, s); return hipGetLastError();
+            default: break;
+        }
+    } else {
+        switch (pick_epi_tile(p.m, p.n, p.k, {kT128Pair, kT64x128, kT64}, num_cus)) {
+            case kT128Pair: launch_epi_mid<2, 2, 4, 4, 2, 2, EPI, B_MN>(p, s); return hipGetLastError();
+            case kT64x128: launch_epi_mid<2, 2, 2, 4, 3, 2, EPI, B_MN>(p, s); return hipGetLastError();
+            case kT64: launch_epi_mid<2, 2, 2, 2, 4, 2, EPI, B_MN>(p, s); return hipGetLastError();
+            default: break;
+        }
+    }
     p.tiles_m = (p.m + kPPTile - 1) / kPPTile;
     p.tiles_n = (p.n + kPPTile - 1) / kPPTile;
     p.band_n = p.tiles_m == p.tiles_n ? 0 : 8;
@@ -518,36 +561,36 @@ GemmEpiArgs epi_args(const void* a, const void* b, void* c, int64_t m, int64_t n
 
 hipError_t gemm_qkv_rope(const void* x, const void* w, int64_t tokens, int64_t hidden, int64_t seq, int64_t hq,
                          int64_t hkv, const float* cos_t, const float* sin_t, int layout, void* q, void* k, void* v,
-                         hipStream_t s) {
+                         int num_cus, hipStream_t s) {
     GemmEpiArgs p = epi_args(x, w, nullptr, tokens, (hq + 2 * hkv) * 128, hidden);
     p.qkv = QkvRopeOut{static_cast<uint16_t*>(q), static_cast<uint16_t*>(k), static_cast<uint16_t*>(v), cos_t, sin_t,
                        static_cast<int>(seq), static_cast<int>(hq), static_cast<int>(hkv), layout};
-    return launch_epi<kEpiQkvRope, false>(p, s);
+    return launch_epi<kEpiQkvRope, false>(p, num_cus, s);
 }
 
 hipError_t gemm_residual(const void* x, const void* w, const void* res, void* y, int64_t m, int64_t n, int64_t k,
-                         hipStream_t s) {
+                         int num_cus, hipStream_t s) {
     GemmEpiArgs p = epi_args(x, w, y, m, n, k);
     p.res = static_cast<const uint16_t*>(res);
-    return launch_epi<kEpiResidual, false>(p, s);
+    return launch_epi<kEpiResidual, false>(p, num_cus, s);
 }
 
 hipError_t gemm_swiglu(const void* x, const void* w_gu, void* gate, void* up, void* act, int64_t m, int64_t f,
-                       int64_t k, hipStream_t s) {
+                       int64_t k, int num_cus, hipStream_t s) {
     GemmEpiArgs p = epi_args(x, w_gu, nullptr, m, 2 * f, k);
     p.gate = static_cast<uint16_t*>(gate);
     p.up = static_cast<uint16_t*>(up);
     p.act = static_cast<uint16_t*>(act);
-    return launch_epi<kEpiSwiglu, false>(p, s);
+    return launch_epi<kEpiSwiglu, false>(p, num_cus, s);
 }
 
 hipError_t gemm_swiglu_backward(const void* dy, const void* wd, const void* gate, const void* up, void* dgu, int64_t m,
-                                int64_t f, int64_t k, hipStream_t s) {
+                                int64_t f, int64_t k, int num_cus, hipStream_t s) {
     GemmEpiArgs p = epi_args(dy, wd, nullptr, m, f, k);
     p.gate = const_cast<uint16_t*>(static_cast<const uint16_t*>(gate));
     p.up = const_cast<uint16_t*>(static_cast<const uint16_t*>(up));
     p.dgu = static_cast<uint16_t*>(dgu);
-    return launch_epi<kEpiSwigluBwd, true>(p, s);
+    return launch_epi<kEpiSwigluBwd, true>(p, num_cus, s);
 }
 
 hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_bf16, int64_t m, int64_t n, int64_t k,

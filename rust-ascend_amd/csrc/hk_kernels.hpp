@@ -106,21 +106,21 @@ hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_b
 bool qkv_rope_applies(int64_t tokens, int64_t hidden, int64_t width);
 hipError_t gemm_qkv_rope(const void* x, const void* w, int64_t tokens, int64_t hidden, int64_t seq, int64_t hq,
                          int64_t hkv, const float* cos_t, const float* sin_t, int layout, void* q, void* k, void* v,
-                         hipStream_t s);
-// The other fused-epilogue GEMMs of a decoder layer (BF16, 256x256 tiles at any M and N; they apply
+                         int num_cus, hipStream_t s);
+// The other fused-epilogue GEMMs of a decoder layer (BF16, any M and N; they apply
 // when K % 8 == 0 and M K, N K stay below 2^30 elements, K rounded up to 64):
 bool epi_applies(int64_t m, int64_t n, int64_t k);
 // y [m, n] = res + x [m, k] W [n, k]^T (the product rounded to BF16 before the add)
 hipError_t gemm_residual(const void* x, const void* w, const void* res, void* y, int64_t m, int64_t n, int64_t k,
-                         hipStream_t s);
+                         int num_cus, hipStream_t s);
 // gate, up, act [m, f]: x [m, k] W_gu [2f, k]^T with W_gu's rows interleaving gate and up in blocks of
 // 16 (row 32 b + r: gate row 16 b + r for r < 16, else up row 16 b + r - 16); act = SiLU(gate) up
 hipError_t gemm_swiglu(const void* x, const void* w_gu, void* gate, void* up, void* act, int64_t m, int64_t f,
-                       int64_t k, hipStream_t s);
+                       int64_t k, int num_cus, hipStream_t s);
 // dgu [m, 2f] (interleaved as W_gu's rows) = the SwiGLU gradients of gate and up for
 // dM = dY [m, k] Wd [k, f] (Wd stored [k, f])
 hipError_t gemm_swiglu_backward(const void* dy, const void* wd, const void* gate, const void* up, void* dgu, int64_t m,
-                                int64_t f, int64_t k, hipStream_t s);
+                                int64_t f, int64_t k, int num_cus, hipStream_t s);
 
 // ---- NLLLoss (hk_loss.hip)
 // dtype 0 F32, 1 F16, 2 BF16 (input, weight, out, total, grad, dinput); id_bytes 4 or 8;

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from gpu_util import DEV
-from rust_ascend_hip import HipRuntime
+from rust_ascend_hip import HipRuntime, runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +112,59 @@ def test_grouped_small_grid():
     want = torch.cat([a[:256].double() @ w[0].double().t().contiguous(), a[256:].double() @ w[2].double().t().contiguous()])
     assert err(out, want) <= bound(320, torch.float32)
     groups.close()
+
+
+# ------------------------------------------------------------------ fused epilogues below a full grid
+
+def bf(shape, seed, scale=1.0):
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(seed)
+    return (torch.randn(shape, generator=gen, device=DEV) * scale).to(torch.bfloat16)
+
+
+def call(name, *args):
+    runtime._call(name, *(runtime.desc(t) if isinstance(t, torch.Tensor) else t for t in args))
+
+
+def rounded(t):
+    return t.to(torch.bfloat16).double()
+
+
+# a product that lands within its sum's error of a BF16 tie rounds the other way in float64: one BF16
+# step (2^-8) of few values, so the rounded results are compared to 2^-8 of the norm
+@pytest.mark.parametrize("t,h,f", [(130, 264, 96), (512, 2048, 1408), (1000, 1024, 2944), (1, 128, 16)])
+def test_small_fused_ffn(t, h, f):
+    x, wg, wu, wd, res = bf((t, h), 1), bf((f, h), 2, h ** -0.5), bf((f, h), 3, h ** -0.5), bf((h, f), 4, 0.1), bf((t, h), 5)
+    w_gu = torch.stack([wg.view(f // 16, 16, h), wu.view(f // 16, 16, h)], 1).reshape(2 * f, h).contiguous()
+    gate, up, act = (torch.empty((t, f), device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    print(f"fused ffn {t}x{h}x{f}", flush=True)
+    call("hk_swiglu_projection", x, w_gu, gate, up, act)
+    g = rounded(x.double() @ wg.double().t().contiguous())
+    u = rounded(x.double() @ wu.double().t().contiguous())
+    assert err(gate, g) <= 2 ** -8 and err(up, u) <= 2 ** -8
+    assert torch.equal(act, HipRuntime.silu_mul(gate, up))
+    if h % 16 == 0:
+        y = torch.empty((t, h), device=DEV, dtype=torch.bfloat16)
+        call("hk_linear_residual", act, wd, res, y)
+        assert err(y, rounded(act.double() @ wd.double().t().contiguous()) + res.double()) <= 2 ** -8
+    dy, dgu = bf((t, h), 6), torch.empty((t, 2 * f), device=DEV, dtype=torch.bfloat16)
+    call("hk_swiglu_projection_backward", dy, wd, gate, up, dgu)
+    dm = dy.double() @ wd.double()
+    sg = torch.sigmoid(gate.double())
+    d = dgu.view(t, f // 16, 2, 16)
+    assert err(d[:, :, 0].reshape(t, f), dm * up.double() * sg * (1 + gate.double() * (1 - sg))) <= 2 ** -7
+    assert err(d[:, :, 1].reshape(t, f), dm * gate.double() * sg) <= 2 ** -7
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("b,s,h,hq,hkv", [(1, 512, 2048, 16, 4), (2, 72, 264, 2, 1), (1, 1, 128, 1, 1), (3, 100, 1024, 8, 8)])
+def test_small_fused_qkv_rope(b, s, h, hq, hkv, layout):
+    """The rotated head planes of the fused projection against the BF16 product split and rotated."""
+    x, w = bf((b * s, h), 1), bf(((hq + 2 * hkv) * 128, h), 2, h ** -0.5)
+    ang = torch.arange(s, device=DEV)[:, None] * 5e5 ** (-torch.arange(0, 128, 2, device=DEV) / 128)
+    cos, sin = ang.cos().float().contiguous(), ang.sin().float().contiguous()
+    print(f"fused qkv {b}x{s}x{h} {hq}/{hkv} layout {layout}", flush=True)
+    q, k, v = HipRuntime.qkv_projection_rope(x, w, cos, sin, b, hq, hkv, layout)
+    rows = (x.double() @ w.double().t().contiguous()).to(torch.bfloat16).view(b, s, -1)
+    for got, want in zip((q, k, v), HipRuntime.qkv_rope_split(rows, cos, sin, hq, hkv, layout)):
+        assert err(got, want.double()) <= 2 ** -8
