@@ -838,23 +838,313 @@ attn_fwd_pp16(FwdArgs a) {
     }
 }
 
-int64_t clamp_diag(const AttnShape& sh) {
-    // visible iff key_start + j <= query_start + i  <=>  j <= i + (query_start - key_start)
-    if (!sh.causal) return 0;
-    const uint64_t qs = sh.query_start, ks = sh.key_start;
-    if (qs >= ks) {
-        const uint64_t d = qs - ks;
-        return d > static_cast<uint64_t>(sh.n) ? sh.n : static_cast<int64_t>(d);
+// ---------------------------------------------------------------------------- decode
+//
+// A few queries per head against a long K/V (the generation step): the pass is the stream of K and
+// V from HBM, and everything follows from that. One workgroup holds all the query rows that read one
+// KV head (the group's heads x M rows are consecutive in Q, up to 64: NR blocks of 16), so K and V are
+// read once per KV head instead of once per query head, and the keys are split over workgroups until
+// the grid fills the CUs; a second kernel combines the splits' partial (O, m, l).
+//   * four independent waves, each walking every fourth 32-key tile of the split with its own online
+//     softmax and its own ring of NS tiles in LDS (128 KB per workgroup in flight; HBM needs ~80 KB
+//     per CU), waited for by vmcnt alone: no barrier until the waves merge at the end;
+//   * S = K Q^T by 16x16x32 MFMAs, K as the first operand, so a lane holds 8 of a query row's 32
+//     scores (keys 4 g + 0..3 and 16 + 4 g + 0..3 of its 16-lane group g); converted to BF16 they are
+//     directly the second operand of O^T = V^T P^T, whose key order the transposing V reads match.
+// Against the ping-pong kernel, whose workgroup is 256 query rows of one head and walks all keys in
+// turn, one query of B8 Hq32 Hkv8 N4096 D128 takes 31 us (4.3 TB/s, of which ~8 us are start, merge and
+// the second launch) instead of 126.
+template <int D>
+struct DecodeTile {
+    static constexpr int kKeys = 32;
+    static constexpr int kElems = kKeys * D;          // one operand's tile
+    static constexpr int kInstr = kElems * 2 / 1024;  // 1 KB loads per operand per tile
+    static constexpr int kSlots = D == 128 ? 2 : 4;   // ring depth: 32 KB per wave
+    // Rows past n lie past the buffer's range and read as zero (their scores are masked).
+    static __device__ __forceinline__ void issue(const i32x4_t& rk, const i32x4_t& rv, uint16_t* slot, int key0, int lane) {
+        constexpr int kRows = 512 / D;  // rows per load
+#pragma unroll
+        for (int q = 0; q < kInstr; ++q) {
+            const int row = q * kRows + lane / (D / 8), pos = lane % (D / 8);
+            const int off = (key0 + row) * (D * 2) + ((pos ^ tile_swz<D>(row)) << 4);
+            load_lds16(rk, lds_address(slot + 512 * q), off, 0);
+            load_lds16(rv, lds_address(slot + kElems + 512 * q), off, 0);
+        }
     }
-    const uint64_t d = ks - qs;
-    const uint64_t cap = static_cast<uint64_t>(sh.m + sh.n + 1);
-    return -static_cast<int64_t>(d > cap ? cap : d);
+};
+
+struct DecodeArgs : FwdArgs {
+    int splits;       // workgroups per KV head
+    int split_tiles;  // 32-key tiles per split
+    int tiles;        // 32-key tiles that some query sees
+    float* po;        // splits > 1: partial O [splits][rows][D], then m and l [splits][rows]
+    float* pm;
+    float* pl;
+    int64_t rows;     // B Hq M
+};
+
+constexpr int kDecodeMaxRows = 64;
+
+template <int D, int NR>
+__global__ void __launch_bounds__(256, 1)
+attn_decode(DecodeArgs a) {
+    using Tile = DecodeTile<D>;
+    constexpr int KS = D / 32, DB = D / 16, NS = Tile::kSlots, kRows = 16 * NR;
+    constexpr int kPerTile = 2 * Tile::kInstr;
+    static_assert((NS - 1) * kPerTile < 64, "vmcnt range");
+    __shared__ __attribute__((aligned(1024))) uint16_t ring[4][NS][2 * Tile::kElems];
+    __shared__ float wave_m[4][kRows], wave_l[4][kRows];
+    static_assert(sizeof(ring) >= 4 * kRows * D * sizeof(float), "the merge reuses the ring");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const int logical = xcd_logical();
+    const int split = logical % a.splits;
+    const int64_t pair = logical / a.splits;  // b * Hkv + kv head
+    const int queries = static_cast<int>(a.m);
+    const int rows = static_cast<int>(a.heads / a.kv_heads) * queries;
+    const uint16_t* Q = a.q + pair * rows * D;
+    const i32x4_t rk = buffer_resource(a.k + pair * a.n * D, static_cast<int>(a.n * D * 2));
+    const i32x4_t rv = buffer_resource(a.v + pair * a.n * D, static_cast<int>(a.n * D * 2));
+
+    bf16x8_t qf[NR][KS];
+    int key_limit[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        const int row = min(16 * r + l16, rows - 1);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[r][ks] = *reinterpret_cast<const bf16x8_t*>(Q + row * D + 32 * ks + 8 * g);
+        int64_t limit = a.n - 1;
+        if (a.causal) limit = row % queries + a.diag < limit ? row % queries + a.diag : limit;
+        key_limit[r] = static_cast<int>(limit < -1 ? -1 : limit);
+    }
+    f32x4_t o[NR][DB];
+    float m_run[NR], l_run[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        m_run[r] = -INFINITY, l_run[r] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DB; ++d) o[r][d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    const int first = split * a.split_tiles + wave, end = min(a.tiles, (split + 1) * a.split_tiles);
+    const int nt = first < end ? (end - first + 3) / 4 : 0;  // this wave's tiles: first + 4 j
+    if (nt > 0) {
+        auto issue = [&](int j) __attribute__((always_inline)) {  // past the end: the last tile again (never read)
+            Tile::issue(rk, rv, ring[wave][j % NS], (first + 4 * min(j, nt - 1)) * Tile::kKeys, lane);
+        };
+#pragma unroll
+        for (int j = 0; j < NS; ++j) issue(j);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) settle(qf[r]);  // one wait, after the first tiles' loads are on their way
+        for (int j = 0; j < nt; ++j) {
+            const uint16_t* kt = ring[wave][j % NS];
+            const uint16_t* vt = kt + Tile::kElems;
+            asm volatile("" ::: "memory");
+            constexpr int kLeft = (NS - 1) * kPerTile;
+            __builtin_amdgcn_s_waitcnt((kLeft & 15) | ((kLeft >> 4) << 14) | (7 << 4) | (15 << 8));
+            asm volatile("" ::: "memory");
+            f32x4_t s[NR][2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const bf16x8_t kf = tile_read16<D>(kt, 16 * h + l16, 4 * ks + g);
+#pragma unroll
+                    for (int r = 0; r < NR; ++r)
+                        s[r][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            kf, qf[r][ks], ks == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : s[r][h], 0, 0, 0);
+                }
+            const int key0 = (first + 4 * j) * Tile::kKeys + 4 * g;
+            bf16x8_t pb[NR];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                float x[8], mt = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    x[e] = key0 + 16 * (e >> 2) + (e & 3) <= key_limit[r] ? s[r][e >> 2][e & 3] * a.scale_log2 : -INFINITY;
+                    mt = fmaxf(mt, x[e]);
+                }
+                mt = quad_max(mt);  // over the row's four 16-lane groups
+                const float m_new = fmaxf(m_run[r], mt);
+                const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_run[r] - m_new);
+                const float neg_m = m_new == -INFINITY ? 0.0f : -m_new;
+                m_run[r] = m_new;
+                float ls = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    x[e] = fast_exp2(x[e] + neg_m);
+                    ls += x[e];
+                }
+                l_run[r] = l_run[r] * alpha + ls;
+#pragma unroll
+                for (int d = 0; d < DB; ++d)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[r][d][e] *= alpha;
+                const u32x4_t w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]),
+                                   pack_bf16x2(x[6], x[7])};
+                pb[r] = __builtin_bit_cast(bf16x8_t, w);
+            }
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                const int col = 16 * d + 4 * (l16 & 3), kr = 4 * g + (l16 >> 2);
+                const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(vt + tile_off<D>(kr, col)));
+                const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(vt + tile_off<D>(kr + 16, col)));
+                typedef short v8i16_t __attribute__((ext_vector_type(8)));
+                const v8i16_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+                for (int r = 0; r < NR; ++r)
+                    o[r][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), pb[r], o[r][d], 0, 0, 0);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of the slot done
+            issue(j + NS);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+
+    // Merge the four waves through LDS (in wave order).
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(ring);  // [4][kRows][D]
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        const float l = quad_sum(l_run[r]);
+        const int row = 16 * r + l16;
+        if (g == 0) wave_m[wave][row] = m_run[r], wave_l[wave][row] = l;
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+            *reinterpret_cast<f32x4_t*>(red + (wave * kRows + row) * D + 16 * d + 4 * g) = o[r][d];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRows * (D / 4); i += 256) {
+        const int row = i / (D / 4), col = (i % (D / 4)) * 4;
+        if (row >= rows) continue;
+        float m = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) m = fmaxf(m, wave_m[w][row]);
+        float l = 0.0f;
+        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = m == -INFINITY ? 1.0f : fast_exp2(wave_m[w][row] - m);
+            l += wave_l[w][row] * f;
+            const f32x4_t x = *reinterpret_cast<const f32x4_t*>(red + (w * kRows + row) * D + col);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += x[e] * f;
+        }
+        const int64_t out_row = pair * rows + row;
+        if (a.splits == 1) {
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            store_o4(a, out_row * D + col, sum[0] * inv, sum[1] * inv, sum[2] * inv, sum[3] * inv);
+            if (col == 0) a.lse[out_row] = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
+        } else {
+            const int64_t part = split * a.rows + out_row;
+            *reinterpret_cast<f32x4_t*>(a.po + part * D + col) = sum;
+            if (col == 0) a.pm[part] = m, a.pl[part] = l;
+        }
+    }
+}
+
+// O and lse of a row from its splits' partials: one wave per row. Lane s reads split s's m and l (at most
+// 64 splits), so the weights need one round trip; then each group of D / 4 lanes adds every
+// (256 / D)-th split's O, and the groups' sums are added pairwise (a fixed order).
+template <int D>
+__global__ void __launch_bounds__(256)
+attn_decode_combine(DecodeArgs a) {
+    constexpr int kLanes = D / 4, kGroups = 64 / kLanes;
+    const int lane = threadIdx.x & 63;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (row >= a.rows) return;
+    const int64_t mine = lane * a.rows + row;
+    const float ms = lane < a.splits ? a.pm[mine] : -INFINITY;
+    const float ls = lane < a.splits ? a.pl[mine] : 0.0f;
+    const float m = wave_max(ms);
+    const float w = m == -INFINITY ? 1.0f : fast_exp2(ms - m);
+    const float l = wave_sum(lane < a.splits ? ls * w : 0.0f);
+    const int col = (lane % kLanes) * 4, grp = lane / kLanes;
+    f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < a.splits; s0 += 8 * kGroups) {
+        f32x4_t x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int s = s0 + u * kGroups + grp;
+            x[u] = s < a.splits ? *reinterpret_cast<const f32x4_t*>(a.po + (s * a.rows + row) * D + col) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int s = s0 + u * kGroups + grp;
+            const float f = __shfl(w, s & 63);  // past the splits the O read above is zero
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += s < a.splits ? x[u][e] * f : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int step = kLanes; step < 64; step *= 2)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += __shfl_xor(sum[e], step);
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if (grp == 0) store_o4(a, row * D + col, sum[0] * inv, sum[1] * inv, sum[2] * inv, sum[3] * inv);
+    if (lane == 0) a.lse[row] = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
+}
+
+// The decode kernel takes the shapes whose query rows per KV head fit its 64 (and D = 64 or 128).
+bool decode_applies(const AttnShape& sh) {
+    return (sh.d == 64 || sh.d == 128) && sh.heads / sh.kv_heads * sh.m <= kDecodeMaxRows;
+}
+
+// 32-key tiles up to the last key that some query sees.
+int decode_tiles(const AttnShape& sh) {
+    int64_t keys = sh.n;
+    if (sh.causal) {
+        const int64_t seen = sh.m + attention_diag(sh);  // the last query sees keys 0 .. m - 1 + diag
+        keys = seen < 0 ? 0 : (seen < keys ? seen : keys);
+    }
+    return static_cast<int>((keys + 31) / 32);
+}
+
+size_t decode_split_bytes(const AttnShape& sh, int splits) {
+    return splits > 1 ? static_cast<size_t>(splits) * sh.batch * sh.heads * sh.m * (sh.d + 2) * sizeof(float) : 0;
+}
+
+// Splits of the keys: least estimated time of rounds of one workgroup per CU, each reading one tile per
+// wave and step at up to 44 GB/s per CU and 5.8 TB/s in all, 5 us of start, merge and launch, and 3.5 us
+// for the combining launch. Measured (us, forced splits) at B8 Hq32 Hkv8 N4096 D128: 1 47, 2 35, 3 31,
+// 4 31, 8 35; at B1 8 splits 11.9, 16 11.2, 32 11.2; at B32 92 unsplit and 101 with 2.
+int decode_splits(const AttnShape& sh, size_t ws_bytes, int num_cus) {
+    const int64_t pairs = sh.batch * sh.kv_heads;
+    const int tiles = decode_tiles(sh);
+    int best = 1;
+    double best_us = 0.0;
+    for (int splits = 1; splits <= 64; ++splits) {
+        if (splits > 1 && (tiles < 4 * splits || decode_split_bytes(sh, splits) > ws_bytes)) break;
+        const int64_t wgs = pairs * splits, rounds = (wgs + num_cus - 1) / num_cus;
+        const double resident = static_cast<double>(wgs < num_cus ? wgs : num_cus);
+        const double bytes = 4.0 * 32 * sh.d * 4;  // one tile of K and V per wave
+        const double step = bytes * fmax(resident / 5.8e6, 1 / 0.044e6);
+        const int per_wave = ((tiles + splits - 1) / splits + 3) / 4;
+        const double us = rounds * (per_wave * step + 5.0) + (splits > 1 ? 3.5 : 0.0);
+        if (splits == 1 || us < best_us) best = splits, best_us = us;
+    }
+    return best;
+}
+
+template <int D>
+hipError_t launch_decode(DecodeArgs a, const AttnShape& sh, hipStream_t s) {
+    const int row_blocks = static_cast<int>((sh.heads / sh.kv_heads * sh.m + 15) / 16);
+    const dim3 grid(static_cast<unsigned>(sh.batch * sh.kv_heads * a.splits));
+    if (row_blocks == 1) hipLaunchKernelGGL((attn_decode<D, 1>), grid, dim3(256), 0, s, a);
+    else if (row_blocks == 2) hipLaunchKernelGGL((attn_decode<D, 2>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_decode<D, 4>), grid, dim3(256), 0, s, a);
+    if (a.splits > 1) {
+        hipLaunchKernelGGL((attn_decode_combine<D>), dim3(static_cast<unsigned>((a.rows + 3) / 4)), dim3(256), 0, s, a);
+    }
+    return hipGetLastError();
 }
 
 template <int D>
 hipError_t launch_fwd(const AttnShape& sh, const void* q, const void* k, const void* v, void* o, float* lse,
-                      hipStream_t s) {
-    FwdArgs a;
+                      void* workspace, size_t ws_bytes, int num_cus, hipStream_t s) {
+    DecodeArgs a{};
     a.q = static_cast<const uint16_t*>(q);
     a.k = static_cast<const uint16_t*>(k);
     a.v = static_cast<const uint16_t*>(v);
@@ -865,17 +1155,27 @@ hipError_t launch_fwd(const AttnShape& sh, const void* q, const void* k, const v
     a.kv_heads = sh.kv_heads;
     a.m = sh.m;
     a.n = sh.n;
-    a.diag = clamp_diag(sh);
+    a.diag = attention_diag(sh);
     a.scale_log2 = sh.scale * kLog2e;
     a.causal = sh.causal;
     if constexpr (D >= 64) {
+        if (decode_applies(sh)) {
+            a.tiles = decode_tiles(sh);
+            a.splits = decode_splits(sh, ws_bytes, num_cus);
+            a.split_tiles = (a.tiles + a.splits - 1) / a.splits;
+            a.rows = sh.batch * sh.heads * sh.m;
+            a.po = static_cast<float*>(workspace);
+            a.pm = a.po + a.splits * a.rows * D;
+            a.pl = a.pm + a.splits * a.rows;
+            return launch_decode<D>(a, sh, s);
+        }
         a.mblocks = static_cast<int>((sh.m + kPPBlockM - 1) / kPPBlockM);
         const dim3 grid(static_cast<unsigned>(sh.batch * sh.heads * a.mblocks));
-        hipLaunchKernelGGL((attn_fwd_pp16<D>), grid, dim3(kPPThreads), 0, s, a);
+        hipLaunchKernelGGL((attn_fwd_pp16<D>), grid, dim3(kPPThreads), 0, s, static_cast<const FwdArgs&>(a));
     } else {
         a.mblocks = static_cast<int>((sh.m + kBlockM - 1) / kBlockM);
         const dim3 grid(static_cast<unsigned>(sh.batch * sh.heads * a.mblocks));
-        hipLaunchKernelGGL((attn_fwd<D>), grid, dim3(kThreads), 0, s, a);
+        hipLaunchKernelGGL((attn_fwd<D>), grid, dim3(kThreads), 0, s, static_cast<const FwdArgs&>(a));
     }
     return hipGetLastError();
 }
@@ -1814,7 +2114,7 @@ int dkv_splits_for(const AttnShape& sh, int num_cus) {
         if (v == 1 || v == 2 || v == 4) return v;
     }
     const int64_t blocks = (sh.n + kKBlock - 1) / kKBlock, qsteps = (sh.m + kQStep - 1) / kQStep;
-    const int64_t group = sh.heads / sh.kv_heads, diag = clamp_diag(sh);
+    const int64_t group = sh.heads / sh.kv_heads, diag = attention_diag(sh);
     int64_t heaviest = 0, work = 0;
     for (int64_t nb = 0; nb < blocks; ++nb) {
         const int64_t qfirst = sh.causal ? std::max<int64_t>(nb * kKBlock - diag, 0) : 0;
@@ -1859,7 +2159,7 @@ hipError_t launch_bwd(const AttnShape& sh, const void* q, const void* k, const v
     a.kv_heads = sh.kv_heads;
     a.m = sh.m;
     a.n = sh.n;
-    a.diag = clamp_diag(sh);
+    a.diag = attention_diag(sh);
     a.scale = sh.scale;
     a.scale_log2 = sh.scale * kLog2e;
     a.causal = sh.causal;
@@ -1916,13 +2216,17 @@ size_t attention_bwd_workspace_bytes(const AttnShape& sh) {
     return stat_bytes(sh) + ((ds_bytes(sh) + 255) & ~size_t(255)) + partial_bytes(sh);
 }
 
+size_t attention_fwd_workspace_bytes(const AttnShape& sh, int num_cus) {
+    return decode_applies(sh) ? decode_split_bytes(sh, decode_splits(sh, SIZE_MAX, num_cus)) : 0;
+}
+
 hipError_t attention_forward(const AttnShape& sh, const void* q, const void* k, const void* v, void* o, float* lse,
-                             hipStream_t s) {
+                             void* workspace, size_t ws_bytes, int num_cus, hipStream_t s) {
     switch (sh.d) {
-        case 16: return launch_fwd<16>(sh, q, k, v, o, lse, s);
-        case 32: return launch_fwd<32>(sh, q, k, v, o, lse, s);
-        case 64: return launch_fwd<64>(sh, q, k, v, o, lse, s);
-        case 128: return launch_fwd<128>(sh, q, k, v, o, lse, s);
+        case 16: return launch_fwd<16>(sh, q, k, v, o, lse, workspace, ws_bytes, num_cus, s);
+        case 32: return launch_fwd<32>(sh, q, k, v, o, lse, workspace, ws_bytes, num_cus, s);
+        case 64: return launch_fwd<64>(sh, q, k, v, o, lse, workspace, ws_bytes, num_cus, s);
+        case 128: return launch_fwd<128>(sh, q, k, v, o, lse, workspace, ws_bytes, num_cus, s);
         default: return hipErrorInvalidValue;
     }
 }

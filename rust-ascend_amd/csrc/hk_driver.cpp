@@ -267,13 +267,13 @@ hk_status ensure_workspace(Ctx* c, size_t bytes) {
     return HK_OK;
 }
 
-// Workspace of an op that takes `fixed` bytes and then GEMM scratch: grows to the scratch the products
-// want, or, where that cannot be had (the workspace limit, device memory, a capturing stream, on
-// which nothing may be allocated), to what they need. *gemm_bytes: the scratch they may use.
-hk_status ensure_gemm_workspace(Ctx* c, size_t fixed, std::initializer_list<hk::GemmWorkspace> products,
-                                size_t* gemm_bytes) {
+// Workspace of an op that takes `fixed` bytes and then scratch shared by its products: grows to what
+// they want, or, where that cannot be had (the workspace limit, device memory, a capturing stream,
+// on which nothing may be allocated), to what they need. *scratch_bytes: the scratch they may use.
+hk_status ensure_scratch(Ctx* c, size_t fixed, std::initializer_list<hk::Scratch> products,
+                         size_t* scratch_bytes) {
     size_t need = 0, want = 0;
-    for (const hk::GemmWorkspace& w : products) {
+    for (const hk::Scratch& w : products) {
         need = std::max(need, w.need);
         want = std::max(want, w.want);
     }
@@ -287,7 +287,7 @@ hk_status ensure_gemm_workspace(Ctx* c, size_t fixed, std::initializer_list<hk::
         st = grow ? ensure_workspace(c, fixed + want) : HK_HIP_ERROR;
         if (st == HK_HIP_ERROR && want > need) st = ensure_workspace(c, fixed + need);
     }
-    *gemm_bytes = st == HK_OK ? c->ws_bytes - fixed : 0;
+    *scratch_bytes = st == HK_OK ? c->ws_bytes - fixed : 0;
     return st;
 }
 
@@ -465,7 +465,7 @@ bool aligned16(std::initializer_list<const void*> ptrs) {
 }
 
 // Scratch of run_gemm with these operands (pieces of the workspace are 256-byte aligned: null here).
-hk::GemmWorkspace gemm_scratch(const Ctx* c, const GemmSpec& s, int ta, int tb, const void* a, const void* b,
+hk::Scratch gemm_scratch(const Ctx* c, const GemmSpec& s, int ta, int tb, const void* a, const void* b,
                                const void* out) {
     return hk::gemm_workspace(s.batch, s.m, s.n, s.k, ta, tb, s.out_dtype == HK_BF16, aligned16({a, b, out}), c->num_cus);
 }
@@ -722,7 +722,7 @@ hk_status hk_gemm_into(hk_context* h, const hk_tensor* a, const hk_tensor* b, in
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a->data, b->data, out->data)}, &gb);
+    st = ensure_scratch(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a->data, b->data, out->data)}, &gb);
     if (st != HK_OK) return st;
     hipError_t e;
     run_gemm(g.c, s, a->data, b->data, out->data, ta, tb, g.c->workspace, gb, &e);
@@ -1374,7 +1374,7 @@ hk_status hk_linear_nt_backward(hk_context* h, const hk_tensor* x, const hk_tens
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, dy->data, w->data, dx->data),
+    st = ensure_scratch(g.c, 0, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, dy->data, w->data, dx->data),
                                         gemm_scratch(g.c, sdw, HK_YES, HK_NO, dy->data, x->data, dw->data)}, &gb);
     if (st != HK_OK) return st;
     hipError_t e;
@@ -1397,7 +1397,7 @@ hk_status hk_gemm_bf16_fp32(hk_context* h, const hk_tensor* a, const hk_tensor* 
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a_bf16->data, b_bf16->data, out->data)}, &gb);
+    st = ensure_scratch(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a_bf16->data, b_bf16->data, out->data)}, &gb);
     if (st != HK_OK) return st;
     hipError_t e = hk::cast_apply(1, a->data, a_bf16->data, numel(a), g.c->stream);
     if (e == hipSuccess) e = hk::cast_apply(1, b->data, b_bf16->data, numel(b), g.c->stream);
@@ -1435,7 +1435,7 @@ hk_status hk_gemm_bf16_fp32_backward(hk_context* h, const hk_tensor* a, const hk
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, dy_bytes, {gemm_scratch(g.c, sdx, dx_ta, dx_tb, a->data, b->data, da->data),
+    st = ensure_scratch(g.c, dy_bytes, {gemm_scratch(g.c, sdx, dx_ta, dx_tb, a->data, b->data, da->data),
                                                gemm_scratch(g.c, sdw, dw_ta, dw_tb, a->data, b->data, db->data)}, &gb);
     if (st != HK_OK) return st;
     void* dyb_ptr = g.c->workspace;
@@ -1489,7 +1489,7 @@ hk_status hk_linear_frozen_bf16_fp32(hk_context* h, const hk_tensor* x, const hk
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, x_bytes, {gemm_scratch(g.c, s, HK_NO, HK_YES, nullptr, w->data, y->data)}, &gb);
+    st = ensure_scratch(g.c, x_bytes, {gemm_scratch(g.c, s, HK_NO, HK_YES, nullptr, w->data, y->data)}, &gb);
     if (st != HK_OK) return st;
     void* xb = g.c->workspace;
     hipError_t e = hk::cast_apply(1, x->data, xb, numel(x), g.c->stream);
@@ -1517,7 +1517,7 @@ hk_status hk_linear_frozen_bf16_fp32_backward(hk_context* h, const hk_tensor* w,
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, dy_bytes, {gemm_scratch(g.c, s, HK_NO, HK_NO, nullptr, w->data, dx->data)}, &gb);
+    st = ensure_scratch(g.c, dy_bytes, {gemm_scratch(g.c, s, HK_NO, HK_NO, nullptr, w->data, dx->data)}, &gb);
     if (st != HK_OK) return st;
     void* dyb_ptr = g.c->workspace;
     hipError_t e = hk::cast_apply(1, dy->data, dyb_ptr, numel(dy), g.c->stream);
@@ -1611,7 +1611,7 @@ hk_status hk_gemm_padded_bf16_fp32(hk_context* h, const hk_tensor* a, const hk_t
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, out_bytes, {gemm_scratch(g.c, s, ta, tb, a_pad->data, b_pad->data,
+    st = ensure_scratch(g.c, out_bytes, {gemm_scratch(g.c, s, ta, tb, a_pad->data, b_pad->data,
                                                              crop ? nullptr : out->data)}, &gb);
     if (st != HK_OK) return st;
     float* native_out = crop ? static_cast<float*>(g.c->workspace) : static_cast<float*>(out->data);
@@ -1664,7 +1664,7 @@ hk_status hk_gemm_padded_bf16_fp32_backward(hk_context* h, const hk_tensor* a_pa
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, dy_bytes + pa_bytes + pb_bytes,
+    st = ensure_scratch(g.c, dy_bytes + pa_bytes + pb_bytes,
                                {gemm_scratch(g.c, sda, da_ta, da_tb, a_pad->data, b_pad->data, crop_a ? nullptr : da->data),
                                 gemm_scratch(g.c, sdb, db_ta, db_tb, a_pad->data, b_pad->data, crop_b ? nullptr : db->data)},
                                &gb);
@@ -1718,7 +1718,7 @@ hk_status hk_linear_frozen_padded_bf16_fp32(hk_context* h, const hk_tensor* x, c
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, xb + wb + ob,
+    st = ensure_scratch(g.c, xb + wb + ob,
                                {gemm_scratch(g.c, s, HK_NO, HK_YES, nullptr, w_pad ? w_pad->data : w_tail ? nullptr : w->data,
                                              crop ? nullptr : y->data)}, &gb);
     if (st != HK_OK) return st;
@@ -1771,7 +1771,7 @@ hk_status hk_linear_frozen_padded_bf16_fp32_backward(hk_context* h, const hk_ten
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     size_t gb;
-    st = ensure_gemm_workspace(g.c, db + ob, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, nullptr, w_pad->data, crop ? nullptr : dx->data)},
+    st = ensure_scratch(g.c, db + ob, {gemm_scratch(g.c, sdx, HK_NO, HK_NO, nullptr, w_pad->data, crop ? nullptr : dx->data)},
                                &gb);
     if (st != HK_OK) return st;
     char* ws = static_cast<char*>(g.c->workspace);
@@ -2621,13 +2621,17 @@ hk_status hk_attention_forward(hk_context* h, const hk_tensor* q, const hk_tenso
     Staged sq = staged(q), sk = staged(k), sv = staged(v);
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
-    if ((st = ensure_workspace(g.c, sq.bytes + sk.bytes + sv.bytes)) != HK_OK) return st;
+    const size_t staging = sq.bytes + sk.bytes + sv.bytes;
+    size_t split_bytes;
+    st = ensure_scratch(g.c, staging, {{0, hk::attention_fwd_workspace_bytes(sh, g.c->num_cus)}}, &split_bytes);
+    if (st != HK_OK) return st;
     char* cursor = static_cast<char*>(g.c->workspace);
     hipError_t e = stage(q, sq, cursor, g.c->stream);
     if (e == hipSuccess) e = stage(k, sk, cursor, g.c->stream);
     if (e == hipSuccess) e = stage(v, sv, cursor, g.c->stream);
     if (e == hipSuccess)
-        e = hk::attention_forward(sh, sq.p, sk.p, sv.p, o->data, static_cast<float*>(lse->data), g.c->stream);
+        e = hk::attention_forward(sh, sq.p, sk.p, sv.p, o->data, static_cast<float*>(lse->data),
+                                  static_cast<char*>(g.c->workspace) + staging, split_bytes, g.c->num_cus, g.c->stream);
     return complete(g.c, e, "attention_forward", 1 + (sq.bytes ? 3 : 0));
 }
 
@@ -2818,7 +2822,7 @@ hk_status ensure_planned(Ctx* c, const std::function<void(Carve&, hipError_t*, C
         bytes[i] = size.used;
     }
     size_t granted;
-    const hk_status st = ensure_gemm_workspace(c, 0, {{bytes[1], bytes[0]}}, &granted);
+    const hk_status st = ensure_scratch(c, 0, {{bytes[1], bytes[0]}}, &granted);
     *lean = granted < bytes[0];
     return st;
 }
@@ -2848,7 +2852,7 @@ size_t composed_gemm_ws(const ComposedShape& sh, bool aligned, bool lean, int cu
     size_t w = 0;
     auto add = [&](int64_t m, int64_t n, int64_t k, int ta, int tb) {
         for (bool bf16 : {false, true}) {
-            const hk::GemmWorkspace g = hk::gemm_workspace(G, m, n, k, ta, tb, bf16, aligned, cus);
+            const hk::Scratch g = hk::gemm_workspace(G, m, n, k, ta, tb, bf16, aligned, cus);
             w = std::max(w, lean ? g.need : g.want);
         }
     };

@@ -434,9 +434,9 @@ size_t round256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // namespace
 
-GemmWorkspace gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
+Scratch gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
                              int num_cus) {
-    GemmWorkspace w;
+    Scratch w;
     if (in_place_applies(m, n, k, aligned)) {
         const GemmChoice c = choose_gemm(batch, m, n, k, ta != 0, out_bf16, SIZE_MAX, num_cus);
         if (c.splits > 1) w.want = static_cast<size_t>(batch * m * n) * 4 * c.splits;

@@ -49,10 +49,10 @@ hipError_t cast_apply(int to_bf16, const void* in, void* out, int64_t n, hipStre
 // are required (operands off 16-byte alignment or past 32-bit offsets are transposed into them),
 // `want` bytes (>= need) let small grids split K; with less the product runs unsplit. `aligned`: A, B
 // and C all 16-byte aligned.
-struct GemmWorkspace {
+struct Scratch {
     size_t need = 0, want = 0;
 };
-GemmWorkspace gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
+Scratch gemm_workspace(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, int tb, bool out_bf16, bool aligned,
                              int num_cus);
 
 // Generic floating matmul (hk_matmul.hip). MatmulBatch: the output's batch dims (innermost last,
@@ -214,8 +214,24 @@ size_t attention_bwd_workspace_bytes(const AttnShape& sh);
 // Whether the fused kernels can take the shape: one head of Q/K/V (M*D and N*D BF16 elements)
 // within 32-bit buffer offsets, and every launch's work items within a dispatch's 32-bit count.
 bool attention_shape_fits(const AttnShape& sh);
+// Visible keys: key j is seen by query i iff j <= i + attention_diag (causal: key_start + j <=
+// query_start + i), clamped to where every larger or smaller value sees the same.
+inline int64_t attention_diag(const AttnShape& sh) {
+    if (!sh.causal) return 0;
+    const uint64_t qs = sh.query_start, ks = sh.key_start;
+    if (qs >= ks) {
+        const uint64_t d = qs - ks;
+        return d > static_cast<uint64_t>(sh.n) ? sh.n : static_cast<int64_t>(d);
+    }
+    const uint64_t d = ks - qs;
+    const uint64_t cap = static_cast<uint64_t>(sh.m + sh.n + 1);
+    return -static_cast<int64_t>(d > cap ? cap : d);
+}
+// Scratch that a forward of a few queries wants for splitting its keys over workgroups (0: none); with
+// less it runs with fewer splits.
+size_t attention_fwd_workspace_bytes(const AttnShape& sh, int num_cus);
 hipError_t attention_forward(const AttnShape& sh, const void* q, const void* k, const void* v, void* o,
-                             float* lse, hipStream_t s);
+                             float* lse, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s);
 // The backward's rows output (D = 64 or 128, M = N = S): dQ, dK, dV written as BF16 token rows
 // [B, S, row_w] of a fused QKV projection's gradient, dQ and dK rotated back by RoPE (tables
 // [S, D/2]); dq/dk/dv are then not written.
