@@ -2835,14 +2835,17 @@ const void* bf16_operand(const hk_tensor* t, Carve& w, hipError_t* e, hipStream_
     return p;
 }
 
-// S = bf16(Q) bf16(K)^T * scale (+ mask) and P = softmax(S), both F32 [B*Hkv, rows, N].
-void composed_probs(const ComposedShape& sh, const void* qb, const void* kb, float scale, const hk_tensor* mask,
-                    float* sbuf, float* p, void* gws, size_t gb, int num_cus, hipStream_t s, hipError_t* e) {
-    const int64_t G = sh.groups(), R = sh.rows();
-    if (*e == hipSuccess) *e = hk::gemm_bf16(qb, kb, sbuf, false, G, R, sh.n, sh.d, HK_NO, HK_YES, gws, gb, num_cus, s);
+// The scores bf16(Q) bf16(K)^T, F32 [B*Hkv, rows, N].
+void composed_scores(const ComposedShape& sh, const void* qb, const void* kb, float* sbuf, void* gws, size_t gb, int cus,
+                     hipStream_t s, hipError_t* e) {
     if (*e == hipSuccess)
-        *e = hk::scale_mask(sbuf, mask ? static_cast<const float*>(mask->data) : nullptr, scale, sh.scores(), s);
-    if (*e == hipSuccess) *e = hk::softmax_forward(sbuf, p, G * R, sh.n, 0, s);
+        *e = hk::gemm_bf16(qb, kb, sbuf, false, sh.groups(), sh.rows(), sh.n, sh.d, HK_NO, HK_YES, gws, gb, cus, s);
+}
+// P = softmax(S * scale (+ mask)) in F32, S scaled and masked in place.
+void composed_probs(const ComposedShape& sh, float scale, const float* mask, float* sbuf, float* p, hipStream_t s,
+                    hipError_t* e) {
+    if (*e == hipSuccess) *e = hk::scale_mask(sbuf, mask, scale, sh.scores(), s);
+    if (*e == hipSuccess) *e = hk::softmax_forward(sbuf, p, sh.groups() * sh.rows(), sh.n, 0, s);
 }
 
 // GEMM scratch of the composed path's products: what they need (lean) or what they want. `aligned`:
@@ -2878,19 +2881,26 @@ hk_status hk_attention_masked_forward(hk_context* h, const hk_tensor* q, const h
     if (mask ? !disjoint({o}, {q, k, v, mask}) : !disjoint({o}, {q, k, v})) return HK_INVALID_ARGUMENT;
     const int64_t G = sh.groups(), R = sh.rows();
     const bool aligned = aligned16({q->data, k->data, v->data, o->data});
+    const float* mask_data = mask ? static_cast<const float*>(mask->data) : nullptr;
+    const bool fused = hk::masked_softmax_applies(sh.n, mask_data, nullptr);
     bool lean = false;
     auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
         const void* qb = bf16_operand(q, w, e, c ? c->stream : nullptr);
         const void* kb = bf16_operand(k, w, e, c ? c->stream : nullptr);
         const void* vb = bf16_operand(v, w, e, c ? c->stream : nullptr);
         float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));
-        float* p = static_cast<float*>(w.take(sh.scores() * 4));
+        float* p = fused ? nullptr : static_cast<float*>(w.take(sh.scores() * 4));
         void* pb = w.take(sh.scores() * 2);
         const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
         void* gws = w.take(gb);
         if (!c) return;
-        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, gb, cus, c->stream, e);
-        if (*e == hipSuccess) *e = hk::cast_apply(1, p, pb, sh.scores(), c->stream);
+        composed_scores(sh, qb, kb, sbuf, gws, gb, cus, c->stream, e);
+        if (fused) {
+            if (*e == hipSuccess) *e = hk::masked_softmax(sbuf, mask_data, scale, pb, G * R, sh.n, c->stream);
+        } else {
+            composed_probs(sh, scale, mask_data, sbuf, p, c->stream, e);
+            if (*e == hipSuccess) *e = hk::cast_apply(1, p, pb, sh.scores(), c->stream);
+        }
         if (*e == hipSuccess)
             *e = hk::gemm_bf16(pb, vb, o->data, o->dtype == HK_BF16, G, R, sh.dv, sh.n, HK_NO, HK_NO, gws,
                                gb, cus, c->stream);
@@ -2901,7 +2911,7 @@ hk_status hk_attention_masked_forward(hk_context* h, const hk_tensor* q, const h
     if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
     plan(w, &e, g.c, g.c->num_cus);
-    return complete(g.c, e, "attention_masked_forward", 6);
+    return complete(g.c, e, "attention_masked_forward", fused ? 4 : 6);
 }
 
 hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const hk_tensor* k, const hk_tensor* v,
@@ -2936,6 +2946,9 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
     }
     const int64_t G = sh.groups(), R = sh.rows();
     const bool aligned = aligned16({q->data, k->data, v->data, dout->data, dq->data, dk->data, dv->data});
+    const float* mask_data = mask ? static_cast<const float*>(mask->data) : nullptr;
+    float* dmask_data = dmask ? static_cast<float*>(dmask->data) : nullptr;
+    const bool fused = hk::masked_softmax_applies(sh.n, mask_data, dmask_data);
     bool lean = false;
     auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
         hipStream_t s = c ? c->stream : nullptr;
@@ -2943,28 +2956,38 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
         const void* kb = bf16_operand(k, w, e, s);
         const void* vb = bf16_operand(v, w, e, s);
         const void* dob = bf16_operand(dout, w, e, s);
-        float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));  // scores, then dP
-        float* p = static_cast<float*>(w.take(sh.scores() * 4));
-        float* ds = dmask ? static_cast<float*>(dmask->data) : static_cast<float*>(w.take(sh.scores() * 4));
-        void* b16 = w.take(sh.scores() * 2);  // bf16(scale * dS), then bf16(P)
+        float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));  // scores (not fused: then dP)
+        // fused: dP, in dMask's buffer when there is one; otherwise P
+        float* f32 = fused && dmask_data ? dmask_data : static_cast<float*>(w.take(sh.scores() * 4));
+        float* ds = dmask_data;
+        if (!fused && !ds) ds = static_cast<float*>(w.take(sh.scores() * 4));
+        void* dsb = w.take(sh.scores() * 2);                        // bf16(scale * dS) (not fused: then bf16(P))
+        void* pb = fused ? w.take(sh.scores() * 2) : dsb;           // bf16(P)
         const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
         void* gws = w.take(gb);
         if (!c) return;
-        // recompute P (the reference keeps it in its autodiff graph)
-        composed_probs(sh, qb, kb, scale, mask, sbuf, p, gws, gb, cus, s, e);
-        // dP = bf16(dO) bf16(V)^T; dS = P * (dP - rowsum(P * dP)) (softmax_backward); dMask = dS
-        if (*e == hipSuccess) *e = hk::gemm_bf16(dob, vb, sbuf, false, G, R, sh.n, sh.dv, HK_NO, HK_YES, gws, gb, cus, s);
-        if (*e == hipSuccess) *e = hk::softmax_backward(p, sbuf, ds, G * R, sh.n, 0, s);
+        // P is recomputed (the reference keeps it in its autodiff graph); dP = bf16(dO) bf16(V)^T;
+        // dS = P * (dP - rowsum(P * dP)) (softmax_backward); dMask = dS
+        composed_scores(sh, qb, kb, sbuf, gws, gb, cus, s, e);
+        if (!fused) composed_probs(sh, scale, mask_data, sbuf, f32, s, e);
+        float* dp = fused ? f32 : sbuf;
+        if (*e == hipSuccess) *e = hk::gemm_bf16(dob, vb, dp, false, G, R, sh.n, sh.dv, HK_NO, HK_YES, gws, gb, cus, s);
+        if (fused) {
+            if (*e == hipSuccess)
+                *e = hk::masked_softmax_backward(sbuf, mask_data, dp, scale, pb, dsb, ds, G * R, sh.n, s);
+        } else {
+            if (*e == hipSuccess) *e = hk::softmax_backward(f32, dp, ds, G * R, sh.n, 0, s);
+            if (*e == hipSuccess) *e = hk::scale_to_bf16(ds, scale, dsb, sh.scores(), s);
+        }
         // dQ = bf16(scale dS) bf16(K); dK = bf16(scale dS)^T bf16(Q) (the group's heads summed in the GEMM)
-        if (*e == hipSuccess) *e = hk::scale_to_bf16(ds, scale, b16, sh.scores(), s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, kb, dq->data, dq->dtype == HK_BF16, G, R, sh.d, sh.n, HK_NO, HK_NO, gws, gb, cus, s);
+            *e = hk::gemm_bf16(dsb, kb, dq->data, dq->dtype == HK_BF16, G, R, sh.d, sh.n, HK_NO, HK_NO, gws, gb, cus, s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, qb, dk->data, dk->dtype == HK_BF16, G, sh.n, sh.d, R, HK_YES, HK_NO, gws, gb, cus, s);
+            *e = hk::gemm_bf16(dsb, qb, dk->data, dk->dtype == HK_BF16, G, sh.n, sh.d, R, HK_YES, HK_NO, gws, gb, cus, s);
         // dV = bf16(P)^T bf16(dO)
-        if (*e == hipSuccess) *e = hk::cast_apply(1, p, b16, sh.scores(), s);
+        if (!fused && *e == hipSuccess) *e = hk::cast_apply(1, f32, pb, sh.scores(), s);
         if (*e == hipSuccess)
-            *e = hk::gemm_bf16(b16, dob, dv->data, dv->dtype == HK_BF16, G, sh.n, sh.dv, R, HK_YES, HK_NO, gws, gb, cus, s);
+            *e = hk::gemm_bf16(pb, dob, dv->data, dv->dtype == HK_BF16, G, sh.n, sh.dv, R, HK_YES, HK_NO, gws, gb, cus, s);
     };
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
@@ -2972,7 +2995,7 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
     if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
     plan(w, &e, g.c, g.c->num_cus);
-    return complete(g.c, e, "attention_masked_backward", 11);
+    return complete(g.c, e, "attention_masked_backward", fused ? 8 : 11);
 }
 
 }  // extern "C"

@@ -179,6 +179,16 @@ hipError_t softmax_forward(const float* x, float* y, int64_t rows, int64_t width
 hipError_t softmax_backward(const float* y, const float* dy, float* dx, int64_t rows, int64_t width, int logarithmic,
                             hipStream_t s);
 
+// Composed attention's row passes (hk_softmax.hip) over F32 scores [rows, width] from the score GEMM:
+// p = bf16(softmax(scores * scale + mask)) (mask F32 like the scores, or null), and, from dP [rows,
+// width], p again, dsb = bf16(scale * ds) and, when ds is given, ds = P (dP - rowsum(P dP)) in F32
+// (it may be dP's buffer). They apply up to widths of 4096 with 16-byte aligned caller tensors.
+bool masked_softmax_applies(int64_t width, const float* mask, const float* ds);
+hipError_t masked_softmax(const float* scores, const float* mask, float scale, void* p, int64_t rows, int64_t width,
+                          hipStream_t s);
+hipError_t masked_softmax_backward(const float* scores, const float* mask, const float* dp, float scale, void* p, void* dsb,
+                                   float* ds, int64_t rows, int64_t width, hipStream_t s);
+
 // Composed-attention compatibility kernels (hk_heads.hip); F32, contiguous.
 hipError_t causal_mask(float* out, int64_t batch, int64_t queries, int64_t keys, uint64_t query_start,
                        uint64_t key_start, hipStream_t s);

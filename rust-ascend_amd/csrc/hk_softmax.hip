@@ -24,6 +24,7 @@
 #include "hk_kernels.hpp"
 
 #include <initializer_list>
+#include <type_traits>
 
 namespace hk {
 
@@ -127,6 +128,105 @@ softmax_bwd_fast(const float* __restrict__ y, const float* __restrict__ dy, floa
                 for (int e = 0; e < 4; ++e)
                     o[e] = LOG ? gv[j][e] - expf(yv[j][e]) * dot : yv[j][e] * (gv[j][e] - dot);
                 *reinterpret_cast<f32x4_t*>(dr + 4 * c) = o;
+            }
+        }
+    }
+}
+
+// ---- composed attention: the row passes between its GEMMs
+//
+// The chain scale, + mask, softmax, cast (and in the backward softmax's gradient, scale, cast) ran as
+// one kernel per step over [rows, N] F32 scores; these take a score row from the GEMM to the BF16
+// operand of the next one in registers, with the same operations in the same order. HBM-bound: the
+// forward moves 4 (scores) + 4 (mask) + 2 bytes per score instead of 26, the backward 4 + 4 + 4 + 4
+// instead of 44. At 33280 rows of 1056 scores: forward 193 -> 57 us (6.2 TB/s), backward 330 -> 110
+// us (5.1 TB/s; the second operand row in registers leaves half the waves in flight).
+//
+// The probabilities of a lane's chunks of a row, as scale_mask and softmax_fwd_fast compute them.
+template <int MAXJ>
+__device__ __forceinline__ void masked_probs(const float* srow, const float* mrow, float scale, int lane, int chunks,
+                                             f32x4_t (&v)[MAXJ]) {
+    load_row4<MAXJ>(srow, lane, chunks, v);
+    f32x4_t k[MAXJ];
+    if (mrow) load_row4<MAXJ>(mrow, lane, chunks, k);
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < MAXJ; ++j)
+        if (lane + 64 * j < chunks)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[j][e] = mrow ? v[j][e] * scale + k[j][e] : v[j][e] * scale;
+                m = fmaxf(m, v[j][e]);
+            }
+    m = wave_max(m);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < MAXJ; ++j)
+        if (lane + 64 * j < chunks)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[j][e] = expf(v[j][e] - m);
+                s += v[j][e];
+            }
+    const float inv = 1.0f / wave_sum(s);
+#pragma unroll
+    for (int j = 0; j < MAXJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] *= inv;
+}
+
+__device__ __forceinline__ void store_bf16x4(uint16_t* p, const f32x4_t& v) {
+    *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+// p = bf16(softmax(s * scale + mask))
+template <int MAXJ>
+__global__ void __launch_bounds__(kFastThreads)
+masked_softmax_rows(const float* __restrict__ s, const float* __restrict__ mask, float scale, uint16_t* __restrict__ p,
+                    int64_t rows, int width) {
+    const int lane = threadIdx.x & 63, chunks = width >> 2;
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * (kFastThreads / 64) + (threadIdx.x >> 6); row < rows;
+         row += static_cast<int64_t>(gridDim.x) * (kFastThreads / 64)) {
+        f32x4_t v[MAXJ];
+        masked_probs<MAXJ>(s + row * width, mask ? mask + row * width : nullptr, scale, lane, chunks, v);
+#pragma unroll
+        for (int j = 0; j < MAXJ; ++j)
+            if (lane + 64 * j < chunks) store_bf16x4(p + row * width + 4 * (lane + 64 * j), v[j]);
+    }
+}
+
+// P recomputed as above; ds = P (dP - sum(P dP)); p = bf16(P), dsb = bf16(ds * scale), and, when ds is
+// given, ds in F32 (it may be dP's own buffer: a lane stores only what it has read).
+template <int MAXJ>
+__global__ void __launch_bounds__(kFastThreads)
+masked_softmax_bwd_rows(const float* __restrict__ s, const float* __restrict__ mask, const float* dp, float scale,
+                        uint16_t* __restrict__ p, uint16_t* __restrict__ dsb, float* ds, int64_t rows, int width) {
+    const int lane = threadIdx.x & 63, chunks = width >> 2;
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * (kFastThreads / 64) + (threadIdx.x >> 6); row < rows;
+         row += static_cast<int64_t>(gridDim.x) * (kFastThreads / 64)) {
+        f32x4_t v[MAXJ], g[MAXJ];
+        load_row4<MAXJ>(dp + row * width, lane, chunks, g);
+        masked_probs<MAXJ>(s + row * width, mask ? mask + row * width : nullptr, scale, lane, chunks, v);
+        float dot = 0.0f;
+#pragma unroll
+        for (int j = 0; j < MAXJ; ++j)
+            if (lane + 64 * j < chunks)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dot += v[j][e] * g[j][e];
+        dot = wave_sum(dot);
+#pragma unroll
+        for (int j = 0; j < MAXJ; ++j) {
+            const int c = lane + 64 * j;
+            if (c < chunks) {
+                const int64_t at = row * width + 4 * c;
+                store_bf16x4(p + at, v[j]);
+                f32x4_t d;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[e] = v[j][e] * (g[j][e] - dot);
+                if (ds) *reinterpret_cast<f32x4_t*>(ds + at) = d;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[e] *= scale;
+                store_bf16x4(dsb + at, d);
             }
         }
     }
@@ -339,7 +439,42 @@ void launch_bwd(const float* y, const float* dy, float* dx, int64_t rows, int64_
     }
 }
 
+// f(integral_constant<MAXJ>) for the float4 chunks per lane of a row of at most 4096 values
+template <class F>
+void by_chunks(int64_t width, F&& f) {
+    const int per_lane = static_cast<int>((width / 4 + 63) / 64);
+    if (per_lane <= 1) f(std::integral_constant<int, 1>{});
+    else if (per_lane <= 2) f(std::integral_constant<int, 2>{});
+    else if (per_lane <= 4) f(std::integral_constant<int, 4>{});
+    else if (per_lane <= 6) f(std::integral_constant<int, 6>{});
+    else if (per_lane <= 8) f(std::integral_constant<int, 8>{});
+    else f(std::integral_constant<int, 16>{});
+}
+
 }  // namespace
+
+bool masked_softmax_applies(int64_t width, const float* mask, const float* ds) { return fast_softmax(width, {mask, ds}); }
+
+hipError_t masked_softmax(const float* scores, const float* mask, float scale, void* p, int64_t rows, int64_t width,
+                          hipStream_t s) {
+    if (rows == 0) return hipSuccess;
+    by_chunks(width, [&](auto j) {
+        hipLaunchKernelGGL((masked_softmax_rows<decltype(j)::value>), dim3(flat_blocks(rows, 4)), dim3(kFastThreads), 0, s,
+                           scores, mask, scale, static_cast<uint16_t*>(p), rows, static_cast<int>(width));
+    });
+    return hipGetLastError();
+}
+
+hipError_t masked_softmax_backward(const float* scores, const float* mask, const float* dp, float scale, void* p, void* dsb,
+                                   float* ds, int64_t rows, int64_t width, hipStream_t s) {
+    if (rows == 0) return hipSuccess;
+    by_chunks(width, [&](auto j) {
+        hipLaunchKernelGGL((masked_softmax_bwd_rows<decltype(j)::value>), dim3(flat_blocks(rows, 4)), dim3(kFastThreads), 0,
+                           s, scores, mask, dp, scale, static_cast<uint16_t*>(p), static_cast<uint16_t*>(dsb), ds, rows,
+                           static_cast<int>(width));
+    });
+    return hipGetLastError();
+}
 
 hipError_t softmax_forward(const float* x, float* y, int64_t rows, int64_t width, int logarithmic, hipStream_t s) {
     if (rows == 0) return hipSuccess;
