@@ -509,6 +509,20 @@ hk_status hk_nll_loss_backward(hk_context* ctx, const hk_tensor* grad, const hk_
                                const hk_tensor* total_weight, int32_t reduction,
                                int64_t ignore_index, hk_tensor* dinput);
 
+/* Cross entropy of F32 logits [N,C] in one pass over them: log_probs [N,C] = log_softmax(logits) (saved
+ * for the backward), then hk_nll_loss of it (same labels, weights, reductions, checks and sums).
+ * weight may be NULL: class weights of one. Reference: nn::weighted_cross_entropy and nn::cross_entropy
+ * (src/nn/loss.rs:42-64), the composition of log_softmax and nll_loss. */
+hk_status hk_cross_entropy(hk_context* ctx, const hk_tensor* logits, const hk_tensor* target,
+                           const hk_tensor* weight, int32_t reduction, int64_t ignore_index,
+                           hk_tensor* log_probs, hk_tensor* out, hk_tensor* total_weight);
+/* dlogits = the gradient of the above: hk_nll_loss_backward's dense gradient through
+ * hk_softmax_backward (logarithmic), evaluated per value without materializing the former. */
+hk_status hk_cross_entropy_backward(hk_context* ctx, const hk_tensor* grad, const hk_tensor* log_probs,
+                                    const hk_tensor* target, const hk_tensor* weight,
+                                    const hk_tensor* total_weight, int32_t reduction, int64_t ignore_index,
+                                    hk_tensor* dlogits);
+
 /* ---------------------------------------------------------------- composed-attention shims */
 
 /* The fused attention entry points apply the mask and the KV-head mapping themselves; these

@@ -2127,6 +2127,30 @@ hk_status nll_layouts(const hk_tensor* input, const hk_tensor* target, const hk_
 bool nll_out_ok(const hk_tensor* t, int64_t len, int32_t dtype) {
     return t && t->dtype == dtype && t->rank == 1 && t->shape[0] == len && (len == 0 || t->data);
 }
+
+// After a synchronous call: the label check its reduction left in the workspace's first word.
+hk_status labels_in_range(Ctx* c, hk_status st, int64_t classes, int64_t ignore_index) {
+    if (st != HK_OK || c->async) return st;
+    int flag = 0;
+    if (hipMemcpy(&flag, c->workspace, sizeof(flag), hipMemcpyDeviceToHost) != hipSuccess) {
+        c->poisoned = true;
+        return fail(HK_COMPLETION_ERROR, "nll_loss: reading the label check failed");
+    }
+    if (flag)
+        return fail(HK_INVALID_ARGUMENT, "NLLLoss target outside [0, %lld) that is not the ignore index %lld",
+                    static_cast<long long>(classes), static_cast<long long>(ignore_index));
+    return HK_OK;
+}
+
+// hk_cross_entropy's tensors: F32 logits-shaped [N, C], labels [N], F32 weights [C] or null.
+hk_status cross_entropy_layouts(const hk_tensor* x, const hk_tensor* target, const hk_tensor* weight, int32_t reduction) {
+    hk_tensor ones = make_view(reinterpret_cast<void*>(uintptr_t{256}), HK_F32, {x && x->rank == 2 ? x->shape[1] : 0});
+    const hk_status st = nll_layouts(x, target, weight ? weight : &ones, reduction);
+    if (st != HK_OK) return st;
+    if (x->dtype != HK_F32)
+        return fail(HK_INVALID_ARGUMENT, "cross entropy requires same-device FP32 logits[N,C], integer labels[N] and FP32 weights[C]");
+    return HK_OK;
+}
 }  // namespace
 
 hk_status hk_nll_loss(hk_context* h, const hk_tensor* input, const hk_tensor* target, const hk_tensor* weight,
@@ -2144,17 +2168,65 @@ hk_status hk_nll_loss(hk_context* h, const hk_tensor* input, const hk_tensor* ta
     hipError_t e = hk::nll_loss(float_code(input->dtype), target->dtype == HK_I64 ? 8 : 4, input->data, target->data,
                                 weight->data, out->data, total_weight->data, rows, classes, reduction, ignore_index,
                                 g.c->workspace, g.c->stream);
-    st = complete(g.c, e, "nll_loss", 1);
-    if (st != HK_OK || g.c->async) return st;
-    int flag = 0;
-    if (hipMemcpy(&flag, g.c->workspace, sizeof(flag), hipMemcpyDeviceToHost) != hipSuccess) {
-        g.c->poisoned = true;
-        return fail(HK_COMPLETION_ERROR, "nll_loss: reading the label check failed");
+    return labels_in_range(g.c, complete(g.c, e, "nll_loss", 1), classes, ignore_index);
+}
+
+hk_status hk_cross_entropy(hk_context* h, const hk_tensor* logits, const hk_tensor* target, const hk_tensor* weight,
+                           int32_t reduction, int64_t ignore_index, hk_tensor* log_probs, hk_tensor* out,
+                           hk_tensor* total_weight) {
+    hk_status st = cross_entropy_layouts(logits, target, weight, reduction);
+    if (st != HK_OK) return st;
+    const int64_t rows = logits->shape[0], classes = logits->shape[1];
+    if (!nll_out_ok(out, reduction == HK_LOSS_NONE ? rows : 1, HK_F32) || !nll_out_ok(total_weight, 1, HK_F32))
+        return fail(HK_INVALID_ARGUMENT, "cross entropy output must be [N] (None) or [1], total weight [1], in F32");
+    if (!tensor_ok(log_probs, "log probabilities") || log_probs->dtype != HK_F32 || !same_shape(log_probs, logits))
+        return fail(HK_INVALID_ARGUMENT, "cross entropy log probabilities must be F32 shaped like the logits");
+    const hk_tensor none{};
+    if (!disjoint({log_probs, out, total_weight}, {logits, target, weight ? weight : &none})) return HK_INVALID_ARGUMENT;
+    OpGuard g(h);
+    if (g.st != HK_OK) return g.st;
+    if ((st = ensure_workspace(g.c, hk::nll_loss_workspace_bytes(rows))) != HK_OK) return st;
+    const int id_bytes = target->dtype == HK_I64 ? 8 : 4;
+    const float* x = static_cast<const float*>(logits->data);
+    const float* w = weight ? static_cast<const float*>(weight->data) : nullptr;
+    float* y = static_cast<float*>(log_probs->data);
+    hipError_t e;
+    if (hk::log_softmax_nll_applies(classes, x, y)) {
+        float* terms = hk::nll_row_terms(g.c->workspace);
+        e = hk::log_softmax_nll(x, y, rows, classes, target->data, id_bytes, w, ignore_index, terms, terms + rows,
+                                reduction == HK_LOSS_NONE ? static_cast<float*>(out->data) : nullptr, g.c->stream);
+        if (e == hipSuccess)
+            e = hk::nll_loss_reduce(id_bytes, target->data, out->data, total_weight->data, rows, classes, reduction,
+                                    ignore_index, g.c->workspace, g.c->stream);
+    } else {
+        e = hk::softmax_forward(x, y, rows, classes, 1, g.c->stream);
+        if (e == hipSuccess)
+            e = hk::nll_loss(0, id_bytes, y, target->data, w, out->data, total_weight->data, rows, classes, reduction,
+                             ignore_index, g.c->workspace, g.c->stream);
     }
-    if (flag)
-        return fail(HK_INVALID_ARGUMENT, "NLLLoss target outside [0, %lld) that is not the ignore index %lld",
-                    static_cast<long long>(classes), static_cast<long long>(ignore_index));
-    return HK_OK;
+    return labels_in_range(g.c, complete(g.c, e, "cross_entropy", 2), classes, ignore_index);
+}
+
+hk_status hk_cross_entropy_backward(hk_context* h, const hk_tensor* grad, const hk_tensor* log_probs,
+                                    const hk_tensor* target, const hk_tensor* weight, const hk_tensor* total_weight,
+                                    int32_t reduction, int64_t ignore_index, hk_tensor* dlogits) {
+    hk_status st = cross_entropy_layouts(log_probs, target, weight, reduction);
+    if (st != HK_OK) return st;
+    const int64_t rows = log_probs->shape[0], classes = log_probs->shape[1];
+    if (!nll_out_ok(grad, reduction == HK_LOSS_NONE ? rows : 1, HK_F32) || !nll_out_ok(total_weight, 1, HK_F32))
+        return fail(HK_INVALID_ARGUMENT, "cross entropy upstream gradient or saved total weight does not match forward reduction/dtype");
+    if (!tensor_ok(dlogits, "dlogits") || dlogits->dtype != HK_F32 || !same_shape(dlogits, log_probs))
+        return fail(HK_INVALID_ARGUMENT, "cross entropy gradient must be F32 shaped like the logits");
+    const hk_tensor none{};
+    if (!disjoint({dlogits}, {grad, log_probs, target, weight ? weight : &none, total_weight})) return HK_INVALID_ARGUMENT;
+    OpGuard g(h);
+    if (g.st != HK_OK) return g.st;
+    hipError_t e = hk::cross_entropy_backward(
+        static_cast<const float*>(grad->data), static_cast<const float*>(log_probs->data), target->data,
+        target->dtype == HK_I64 ? 8 : 4, weight ? static_cast<const float*>(weight->data) : nullptr,
+        static_cast<const float*>(total_weight->data), static_cast<float*>(dlogits->data), rows, classes, reduction,
+        ignore_index, g.c->stream);
+    return complete(g.c, e, "cross_entropy_backward", 1);
 }
 
 hk_status hk_nll_loss_backward(hk_context* h, const hk_tensor* grad, const hk_tensor* input, const hk_tensor* target,

@@ -127,6 +127,10 @@ hipError_t gemm_swiglu_backward(const void* dy, const void* wd, const void* gate
 // reduction 0 None, 1 Mean, 2 Sum. The forward writes *bad = 1 if a label outside [0, classes)
 // that is not `ignore` occurs.
 size_t nll_loss_workspace_bytes(int64_t rows);  // the label flag and the per-row terms
+// Where the workspace keeps the per-row terms, and their reduction (F32 out and total) alone.
+float* nll_row_terms(void* workspace);
+hipError_t nll_loss_reduce(int id_bytes, const void* target, void* out, void* total, int64_t rows, int64_t classes,
+                           int reduction, int64_t ignore, void* workspace, hipStream_t s);
 hipError_t nll_loss(int dtype, int id_bytes, const void* input, const void* target, const void* weight, void* out,
                     void* total, int64_t rows, int64_t classes, int reduction, int64_t ignore, void* workspace, hipStream_t s);
 hipError_t nll_loss_backward(int dtype, int id_bytes, const void* grad, const void* target, const void* weight,
@@ -178,6 +182,17 @@ int embedding_backward_launches(int64_t tokens, int64_t vocab, int64_t width);
 hipError_t softmax_forward(const float* x, float* y, int64_t rows, int64_t width, int logarithmic, hipStream_t s);
 hipError_t softmax_backward(const float* y, const float* dy, float* dx, int64_t rows, int64_t width, int logarithmic,
                             hipStream_t s);
+
+// Cross entropy's passes over the logits (hk_softmax.hip). y = log_softmax(x) with each row's NLL term
+// -weight[t] y[t] and counted weight (weight null: 1), and the gradient of the summed terms through
+// the log-softmax from its output. The forward applies to 16-byte aligned x and y of widths up to
+// 65536; out (null, or [rows]) receives the terms themselves.
+bool log_softmax_nll_applies(int64_t width, const float* x, const float* y);
+hipError_t log_softmax_nll(const float* x, float* y, int64_t rows, int64_t width, const void* target, int id_bytes,
+                           const float* weight, int64_t ignore, float* row_v, float* row_w, float* out, hipStream_t s);
+hipError_t cross_entropy_backward(const float* grad, const float* y, const void* target, int id_bytes, const float* weight,
+                                  const float* total, float* dx, int64_t rows, int64_t classes, int reduction,
+                                  int64_t ignore, hipStream_t s);
 
 // Composed attention's row passes (hk_softmax.hip) over F32 scores [rows, width] from the score GEMM:
 // p = bf16(softmax(scores * scale + mask)) (mask F32 like the scores, or null), and, from dP [rows,

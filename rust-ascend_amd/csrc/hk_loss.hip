@@ -3,7 +3,7 @@
 // Semantics (reference: CannSession::nll_loss / nll_loss_backward, rust-ascend-driver/src/tensor/
 // loss.rs:31-70, over the closed aclnnNLLLoss / aclnnNLLLossBackward; the expectations of
 // examples/cross_entropy_tensor.rs:38-52): input [N, C] log-probabilities, target [N] class
-// labels, weight [C]. A row whose label equals ignore_index (-1 when the caller sets none,
+// labels, weight [C] (the fused cross entropy also passes none: weights of one). A row whose label equals ignore_index (-1 when the caller sets none,
 // NllLossOptions::ignore, loss.rs:10-12) contributes nothing.
 //   row loss  l_n = -weight[t_n] * input[n, t_n]         (0 for an ignored row)
 //   None -> out[n] = l_n;  Sum -> out[0] = sum_n l_n;  Mean -> out[0] = sum_n l_n / W
@@ -41,7 +41,7 @@ nll_rows_kernel(const T* __restrict__ input, const I* __restrict__ target, const
         const int64_t t = static_cast<int64_t>(target[r]);
         float v = 0.0f, wc = 0.0f;
         if (t != ignore && t >= 0 && t < classes) {
-            const float wt = Elem<T>::load(weight, t);
+            const float wt = weight ? Elem<T>::load(weight, t) : 1.0f;
             v = -(wt * Elem<T>::load(input, r * classes + t));
             wc = wt;
         }
@@ -162,6 +162,21 @@ hipError_t nll_loss(int dtype, int id_bytes, const void* input, const void* targ
                    : nll_forward_t<_Float16, int32_t>(dtype, input, target, weight, out, total, rows, classes, reduction, ignore, ws, s);
     return i64 ? nll_forward_t<uint16_t, int64_t>(dtype, input, target, weight, out, total, rows, classes, reduction, ignore, ws, s)
                : nll_forward_t<uint16_t, int32_t>(dtype, input, target, weight, out, total, rows, classes, reduction, ignore, ws, s);
+}
+
+float* nll_row_terms(void* workspace) { return reinterpret_cast<float*>(static_cast<char*>(workspace) + 256); }
+
+hipError_t nll_loss_reduce(int id_bytes, const void* target, void* out, void* total, int64_t rows, int64_t classes,
+                           int reduction, int64_t ignore, void* ws, hipStream_t s) {
+    const float* row_v = nll_row_terms(ws);
+    int* bad = static_cast<int*>(ws);
+    if (id_bytes == 8)
+        hipLaunchKernelGGL((nll_reduce_kernel<int64_t>), dim3(1), dim3(kNllThreads), 0, s, static_cast<const int64_t*>(target),
+                           row_v, row_v + rows, out, total, 0, rows, classes, reduction, ignore, bad);
+    else
+        hipLaunchKernelGGL((nll_reduce_kernel<int32_t>), dim3(1), dim3(kNllThreads), 0, s, static_cast<const int32_t*>(target),
+                           row_v, row_v + rows, out, total, 0, rows, classes, reduction, ignore, bad);
+    return hipGetLastError();
 }
 
 hipError_t nll_loss_backward(int dtype, int id_bytes, const void* grad, const void* target, const void* weight,

@@ -522,19 +522,43 @@ def nll_loss(input, target, weight, reduction=LossReduction.Mean, ignore_index=N
     return _NllLoss.apply(input, target, weight, LossReduction(reduction), ignore_index)
 
 
+class _CrossEntropy(torch.autograd.Function):
+    """log_softmax and nll_loss as one node: one pass over the logits forward, one over the saved
+    log-probabilities backward. Saves what the two nodes saved: the log-probabilities, label and
+    weight snapshots and the total weight."""
+
+    @staticmethod
+    def forward(ctx, logits, target, weight, reduction, ignore_index):
+        t = target.contiguous().clone()
+        w = None if weight is None else weight.contiguous().clone()
+        out, y, total = HipRuntime.cross_entropy(logits.contiguous(), t, w, reduction, ignore_index)
+        ctx.save_for_backward(y, t, w, total)
+        ctx.reduction, ctx.ignore_index = reduction, ignore_index
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        y, t, w, total = ctx.saved_tensors
+        dx = HipRuntime.cross_entropy_backward(grad.contiguous().to(torch.float32), y, t, w, total, ctx.reduction,
+                                               ctx.ignore_index)
+        return dx, None, None, None, None
+
+
+def _cross_entropy(logits, target, weight, reduction, ignore_index):
+    if logits.dim() != 2 or logits.dtype != torch.float32 or target.dtype not in (torch.int32, torch.int64) or \
+            tuple(target.shape) != (logits.shape[0],) or \
+            (weight is not None and (weight.dtype != torch.float32 or tuple(weight.shape) != (logits.shape[1],))):
+        raise HkError(_lib.INVALID_ARGUMENT, "cross entropy requires same-device FP32 logits[N,C], integer labels[N] "
+                                             "and FP32 weights[C]")
+    return _CrossEntropy.apply(logits, target, weight, LossReduction(reduction), ignore_index)
+
+
 def weighted_cross_entropy(logits, target, weight, reduction=LossReduction.Mean, ignore_index=None):
     """nll_loss(log_softmax(logits)) with fixed class weights: F32 logits [N, C], integer labels [N],
     F32 weights [C]. Reference: nn::weighted_cross_entropy (src/nn/loss.rs:52-64)."""
-    if logits.dim() != 2 or logits.dtype != torch.float32 or weight.dtype != torch.float32 or \
-            target.dtype not in (torch.int32, torch.int64) or tuple(target.shape) != (logits.shape[0],) or \
-            tuple(weight.shape) != (logits.shape[1],):
-        from ._lib import INVALID_ARGUMENT, HkError
-        raise HkError(INVALID_ARGUMENT, "cross entropy requires same-device FP32 logits[N,C], integer labels[N] "
-                                        "and FP32 weights[C]")
-    return nll_loss(log_softmax(logits), target, weight, reduction, ignore_index)
+    return _cross_entropy(logits, target, weight, reduction, ignore_index)
 
 
 def cross_entropy(logits, target, reduction=LossReduction.Mean, ignore_index=None):
     """Unweighted cross entropy (class weights of one). Reference: nn::cross_entropy (src/nn/loss.rs:42-50)."""
-    weight = torch.ones((logits.shape[1],), dtype=torch.float32, device=logits.device)
-    return weighted_cross_entropy(logits, target, weight, reduction, ignore_index)
+    return _cross_entropy(logits, target, None, reduction, ignore_index)

@@ -564,6 +564,29 @@ class HipRuntime:
         return dx
 
     @staticmethod
+    def cross_entropy(logits, target, weight=None, reduction=LossReduction.Mean, ignore_index=None):
+        """[loss, log-probabilities, total weight] of F32 logits [N, C] (weight None: class weights of one)
+        in one pass over the logits: nn::weighted_cross_entropy (src/nn/loss.rs:52-64)."""
+        red = LossReduction(reduction)
+        rows = logits.shape[0] if logits.dim() == 2 else 0
+        y = _empty(logits.shape, torch.float32, logits)
+        out = _empty((rows if red == LossReduction.None_ else 1,), torch.float32, logits)
+        total = _empty((1,), torch.float32, logits)
+        _call("hk_cross_entropy", desc(logits), desc(target), None if weight is None else desc(weight), int(red),
+              _ignore(ignore_index), desc(y), desc(out), desc(total))
+        return out, y, total
+
+    @staticmethod
+    def cross_entropy_backward(grad, log_probs, target, weight, total_weight, reduction=LossReduction.Mean,
+                               ignore_index=None):
+        """The logits' gradient from the saved log-probabilities."""
+        dx = _empty(log_probs.shape, torch.float32, log_probs)
+        _call("hk_cross_entropy_backward", desc(grad), desc(log_probs), desc(target),
+              None if weight is None else desc(weight), desc(total_weight), int(LossReduction(reduction)),
+              _ignore(ignore_index), desc(dx))
+        return dx
+
+    @staticmethod
     def embedding(weight, ids):
         """weight[ids] -> [ids..., H]. Reference: AscendRuntime::embedding (mod.rs:237-241)."""
         out = _empty(tuple(ids.shape) + (weight.shape[1],), weight.dtype, weight)
