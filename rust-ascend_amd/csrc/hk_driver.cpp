@@ -1211,8 +1211,9 @@ hk_status hk_tensor_matmul(hk_context* h, const hk_tensor* a, const hk_tensor* b
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     if (numel(out) == 0) return HK_OK;
-    if ((st = ensure_workspace(g.c, hk::matmul_workspace_bytes(s))) != HK_OK) return st;
-    hipError_t e = hk::matmul(s, a->data, b->data, out->data, g.c->workspace, g.c->num_cus, g.c->stream);
+    size_t wb;
+    if ((st = ensure_scratch(g.c, 0, {hk::matmul_workspace(s, g.c->num_cus)}, &wb)) != HK_OK) return st;
+    hipError_t e = hk::matmul(s, a->data, b->data, out->data, g.c->workspace, wb, g.c->num_cus, g.c->stream);
     return complete(g.c, e, "tensor_matmul", 5);
 }
 
@@ -1234,8 +1235,9 @@ hk_status hk_tensor_matmul_backward(hk_context* h, const hk_tensor* a, const hk_
     OpGuard g(h);
     if (g.st != HK_OK) return g.st;
     if (numel(da) == 0 && numel(db) == 0) return HK_OK;
-    if ((st = ensure_workspace(g.c, hk::matmul_backward_workspace_bytes(s))) != HK_OK) return st;
-    hipError_t e = hk::matmul_backward(s, a->data, b->data, dy->data, da->data, db->data, g.c->workspace,
+    size_t wb;
+    if ((st = ensure_scratch(g.c, 0, {hk::matmul_backward_workspace(s, g.c->num_cus)}, &wb)) != HK_OK) return st;
+    hipError_t e = hk::matmul_backward(s, a->data, b->data, dy->data, da->data, db->data, g.c->workspace, wb,
                                        g.c->num_cus, g.c->stream);
     return complete(g.c, e, "tensor_matmul_backward", 8);
 }

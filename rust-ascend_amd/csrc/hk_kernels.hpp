@@ -68,9 +68,9 @@ struct MatmulSpec {
     int64_t m = 0, n = 0, k = 0;
     MatmulBatch batch, a_batch, b_batch;  // output batch shape; A's and B's strides over it
 };
-size_t matmul_workspace_bytes(const MatmulSpec& s);
-hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, int num_cus,
-                  hipStream_t st);
+Scratch matmul_workspace(const MatmulSpec& s, int num_cus);
+hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, size_t ws_bytes,
+                  int num_cus, hipStream_t st);
 // Module attention's score transform (hk_attention_module.hip) over F32 scores [B, H, Sq, Sk]:
 // masked ? -inf : softcap(s * scale) + bias; masked = (causal and key > query) or mask != 0.
 struct AttnScoreSpec {
@@ -89,10 +89,10 @@ hipError_t attention_scores_backward(const AttnScoreSpec& sp, const float* s, co
                                      const uint8_t* mask, float* dbias, const int64_t* bias_shape, float* workspace,
                                      hipStream_t st);
 hipError_t swap_last_dims(int elem_bytes, const void* x, void* y, int64_t G, int64_t R, int64_t C, hipStream_t st);
-size_t matmul_backward_workspace_bytes(const MatmulSpec& s);
+Scratch matmul_backward_workspace(const MatmulSpec& s, int num_cus);
 // dA = dY B^T summed over A's broadcast batches, dB = A^T dY summed over B's, each in the dtype.
 hipError_t matmul_backward(const MatmulSpec& s, const void* a, const void* b, const void* dy, void* da, void* db,
-                           void* workspace, int num_cus, hipStream_t st);
+                           void* workspace, size_t ws_bytes, int num_cus, hipStream_t st);
 hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_t batch, int64_t m,
                      int64_t n, int64_t k, int ta, int tb, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s);
 // M-grouped NT GEMM: C[i, :] = A[i, :] W[g(i)]^T with A [m, k], W [groups, n, k], C [m, n];

@@ -7,17 +7,20 @@
 // B[b_b..., k, j], A [..., M, K] and B [..., K, N] row-major, batch dims broadcast numpy-style
 // (layout.rs:106-142), FP32 products and sums, the output rounded to the inputs' dtype (RNE).
 //
-// Design: the operands are first gathered into packed, zero-padded NT operands in the workspace,
-// A' [G, Mp, Kp] and B' [G, Np, Kp] (B transposed on the way), one slice per output batch with the
-// broadcast applied by the gather's batch strides (0 along a broadcast dim). Padding with zeros
-// adds nothing to the sums. The product runs on MFMA tiles without any bounds logic: BF16 on the
-// library's BF16 GEMM (hk_gemm.hip), F32 and F16 on the 64x64-tile kernels below, into C'
-// [G, Mp, Np], from which the [G, M, N] output is cropped. This path serves the generic backend
-// op (float_matmul); the transformer's own GEMMs use hk_gemm.hip directly.
+// Design: F32 operands are read in place by matmul_f32_tile, whatever their extents, batch strides and
+// alignment. F16 and BF16 operands (and F32 past 32-bit offsets) are first gathered into packed, zero-padded NT operands in the
+// workspace, A' [G, Mp, Kp] and B' [G, Np, Kp] (B transposed on the way), one slice per output batch
+// with the broadcast applied by the gather's batch strides (0 along a broadcast dim). Padding with
+// zeros adds nothing to the sums. The product then runs on MFMA tiles without any bounds logic: BF16
+// on the library's BF16 GEMM (hk_gemm.hip), F16 and F32 on 64x64-tile kernels, into C' [G, Mp, Np],
+// from which the [G, M, N] output is cropped. This path serves the generic backend op (float_matmul);
+// the transformer's own GEMMs use hk_gemm.hip directly.
 #include "hk_common.hpp"
 #include "hk_kernels.hpp"
 
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 namespace hk {
 
@@ -199,6 +202,214 @@ matmul_f16_nt(const _Float16* __restrict__ A, const _Float16* __restrict__ B, TO
     store_tile64(C + g * Mp * Np, Np, tm * kMT + wm * 32, tn * kMT + wn * 32, lane, acc);
 }
 
+// F32 product of one batch slice, read in place: no gather, no padding, no crop.
+//
+//   C[g][m][n] = sum_k A'[g][m][k] B'[g][n][k], A' stored [M, K] (row stride lda) or, A_MN, [K, M]; B'
+//   stored [N, K] or, B_MN, [K, N]; any extents, 4-byte alignment.
+//
+// What bounds it is the F32 matrix rate (256 flop per clock and CU, 157 TFLOP/s): a 128x128 tile takes
+// 2048 matrix clocks per 16 k against 16 KB of operands, so the loads only have to stay ahead.
+// Tiles travel by global->LDS loads, whose range check zero-fills past the matrix, into a ring of NS
+// stages of 16 k: 16-byte loads where an operand's rows are aligned, else 4-byte ones, of which the 64
+// per 128x128 stage take the memory pipeline longer (~40 clocks each) than the MFMAs take. A K-major operand is staged as 64-byte rows of 16 k (16-byte chunks XOR (row /
+// 4) % 4, so that 16 rows at one chunk lie in distinct banks), an MN-major one as rows of the tile's
+// columns (column XOR 16 (k / 4), so that the four 16-lane groups of a read lie in distinct banks). An
+// MFMA (16x16x4: half the accumulator traffic per flop of 32x32x2) takes one k per 16-lane group: group
+// g contributes k = 4 g + u to MFMA u for A and B alike.
+// Measured: 4096^3 1007 us (136 TFLOP/s); [4000, 1024] x [1024, 1000] with its two gradients 228 us, 378 with
+// gathered operands and a 64x64 kernel; F32 error against float64 5.7e-7 -> 2.9e-7.
+struct F32Args {
+    const float* a;
+    const float* b;
+    float* c;  // [G][M][N], or with splits [splits][G][M][N]
+    MatmulBatch ab, bb;
+    int m, n, k;
+    int lda, ldb;
+    int tiles_m, tiles_n;
+    int splits, steps_per_split;  // K in steps of 16
+};
+
+constexpr int kFK = 16;
+
+__device__ __forceinline__ int64_t batch_offset(const MatmulBatch& mb, int64_t g) {
+    int64_t off = 0;
+    for (int d = mb.dims - 1; d >= 0; --d) {
+        off += g % mb.shape[d] * mb.stride[d];
+        g /= mb.shape[d];
+    }
+    return off;
+}
+
+// T: 128x128 (2) or 64x64 (1) tiles, four waves of 32 T x 32 T as 2T x 2T blocks of 16x16.
+// VA, VB: 16-byte loads of A, B (16-byte aligned base, row stride a multiple of 4 floats).
+template <int T, int NS, bool A_MN, bool B_MN, bool VA, bool VB>
+__global__ void __launch_bounds__(kThreads, 2)
+matmul_f32_tile(F32Args p) {
+    constexpr int W = 64 * T;             // tile edge
+    constexpr int kOp = W * kFK;          // floats of one operand's stage
+    constexpr int kLoadsA = VA ? T : 4 * T, kLoads = kLoadsA + (VB ? T : 4 * T);  // per wave and stage
+    static_assert((NS - 1) * kLoads < 64, "vmcnt range");
+    __shared__ __attribute__((aligned(1024))) float ring[NS][2 * kOp];
+
+    const int tiles = p.tiles_m * p.tiles_n, all = tiles * p.splits;
+    int bid = blockIdx.x;
+    if ((all & 7) == 0) bid = (bid & 7) * (all >> 3) + (bid >> 3);  // XCD-contiguous
+    const int split = bid / tiles;
+    bid -= split * tiles;
+    constexpr int GROUP = 8;
+    const int per_group = GROUP * p.tiles_n, first_m = bid / per_group * GROUP;
+    const int gsize = min(p.tiles_m - first_m, GROUP);
+    const int tm = first_m + bid % per_group % gsize, tn = bid % per_group / gsize;
+    const int64_t g = blockIdx.z;
+    const i32x4_t ra = buffer_resource(p.a + batch_offset(p.ab, g), (A_MN ? p.k : p.m) * p.lda * 4);
+    const i32x4_t rb = buffer_resource(p.b + batch_offset(p.bb, g), (B_MN ? p.k : p.n) * p.ldb * 4);
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, g4 = lane >> 4;
+    const int first = split * p.steps_per_split;
+    const int nk = min((p.k + kFK - 1) / kFK - first, p.steps_per_split);
+
+    // K-major 4-byte load q = wave + 4 d: rows 4 q .. 4 q + 3, whose XOR term is q % 4 = wave
+    const int kk = (((lane & 15) >> 2) ^ wave) << 2 | (lane & 3);
+    auto load = [&](const i32x4_t& r, float* dst, bool mn, bool vec, int row0, int ld, int step, int d) __attribute__((always_inline)) {
+        const int q = wave + 4 * d;
+        int off;
+        if (mn) {  // k-rows of W columns
+            const int per = vec ? 256 : 64, at = per * q + (vec ? 4 * lane : lane);
+            const int k = at / W, pos = at % W;
+            off = ((step * kFK + k) * ld + row0 + (pos ^ ((k >> 2) << 4))) * 4;
+        } else if (vec) {  // 16 rows of four chunks
+            const int k = step * kFK + (((lane & 3) ^ (lane >> 4)) << 2);
+            off = k < p.k ? ((row0 + 16 * q + (lane >> 2)) * ld + k) * 4 : static_cast<int>(0x80000000u);
+        } else {
+            const int k = step * kFK + kk;
+            off = k < p.k ? ((row0 + 4 * q + (lane >> 4)) * ld + k) * 4 : static_cast<int>(0x80000000u);
+        }
+        if (vec) load_lds16(r, lds_address(reinterpret_cast<const uint16_t*>(dst + 256 * q)), off, 0);
+        else load_lds4(r, lds_address(reinterpret_cast<const uint16_t*>(dst + 64 * q)), off, 0);
+    };
+    auto fetch_one = [&](int slot, int step, int d) __attribute__((always_inline)) {
+        if (d < kLoadsA) load(ra, ring[slot], A_MN, VA, tm * W, p.lda, step, d);
+        else load(rb, ring[slot] + kOp, B_MN, VB, tn * W, p.ldb, step, d - kLoadsA);
+    };
+    auto fetch = [&](int slot, int step) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < kLoads; ++d) fetch_one(slot, step, d);
+    };
+    // k = 4 g4 .. 4 g4 + 3 of row (column) `row` of a stage
+    auto frag = [&](const float* t, bool mn, int row) __attribute__((always_inline)) {
+        if (!mn) return *reinterpret_cast<const f32x4_t*>(t + row * kFK + ((g4 ^ ((row >> 2) & 3)) << 2));
+        f32x4_t v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = t[(4 * g4 + u) * W + (row ^ (g4 << 4))];
+        return v;
+    };
+
+    // Two levels of accumulators: `acc` sums 256 k, then joins `sum`, so the error of a long contraction
+    // grows with its number of blocks, not of products.
+    constexpr int B = 2 * T;  // 16x16 blocks per wave and direction
+    f32x4_t acc[B][B], sum[B][B];
+    auto clear = [&](f32x4_t (&x)[B][B]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+#pragma unroll
+            for (int j = 0; j < B; ++j) x[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    auto join = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+#pragma unroll
+            for (int j = 0; j < B; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[i][j][e] += acc[i][j][e];
+    };
+    clear(acc);
+    clear(sum);
+
+    // The MFMAs of a step run while the next step's operands are read. The barrier before them (step s + 1
+    // landed, every read of step s done) frees the slot of step s for step s + NS. Past the last step
+    // the loads repeat it.
+    const int last = first + nk - 1;
+    f32x4_t fa[2][B], fb[2][B];
+    auto read_one = [&](int slot, auto buf, int f) __attribute__((always_inline)) {
+        constexpr int N = decltype(buf)::value;
+        if (f < B) fa[N][f] = frag(ring[slot], A_MN, 16 * (B * wm + f) + l16);
+        else fb[N][f - B] = frag(ring[slot] + kOp, B_MN, 16 * (B * wn + f - B) + l16);
+    };
+    auto landed = [&](auto left) __attribute__((always_inline)) {
+        constexpr int kLeft = decltype(left)::value;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt((kLeft & 15) | ((kLeft >> 4) << 14) | (7 << 4) | (0 << 8));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto step = [&](int s, auto buf) __attribute__((always_inline)) {
+        constexpr int N = decltype(buf)::value;
+        landed(std::integral_constant<int, (NS - 2) * kLoads>{});
+        // the next step's operand reads and the loads spread between the MFMAs (issue is in order)
+        const int slot = s % NS, next = (s + 1) % NS, ahead = min(first + s + NS, last);
+        constexpr int kMfma = 4 * B * B, kMem = 2 * B + kLoads;
+#pragma unroll
+        for (int e = 0; e < kMfma; ++e) {
+            const int u = e / (B * B), i = e / B % B, j = e % B;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[N][j][u], fa[N][i][u], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int f = e * kMem / kMfma; f < (e + 1) * kMem / kMfma; ++f) {
+                if (f < 2 * B) read_one(next, std::integral_constant<int, N ^ 1>{}, f);
+                else fetch_one(slot, ahead, f - 2 * B);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if ((s & 15) == 15) {
+            join();
+            clear(acc);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < NS; ++u) fetch(u, min(first + u, last));
+    landed(std::integral_constant<int, (NS - 1) * kLoads>{});
+#pragma unroll
+    for (int f = 0; f < 2 * B; ++f) read_one(0, std::integral_constant<int, 0>{}, f);
+    for (int s = 0; s < nk; s += 2) {
+        step(s, std::integral_constant<int, 0>{});
+        if (s + 1 < nk) step(s + 1, std::integral_constant<int, 1>{});
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS at exit
+    join();
+
+    float* c = p.c + (static_cast<int64_t>(split) * gridDim.z + g) * p.m * p.n;
+    const bool vec = (p.n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+        const int m = tm * W + 16 * (B * wm + i) + l16;
+        if (m >= p.m) continue;
+        float* row = c + static_cast<int64_t>(m) * p.n;
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const int n = tn * W + 16 * (B * wn + j) + 4 * g4;
+            if (vec && n < p.n) {
+                *reinterpret_cast<f32x4_t*>(row + n) = sum[i][j];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < p.n) row[n + e] = sum[i][j][e];
+            }
+        }
+    }
+}
+
+// out = the sum over the splits, in order, of the partial planes [splits][total].
+__global__ void __launch_bounds__(256)
+sum_planes(const float* __restrict__ partial, float* __restrict__ out, int splits, int64_t total) {
+    for (int64_t i = flat_begin(256); i < total; i += flat_stride(256)) {
+        float sum = partial[i];
+        for (int s = 1; s < splits; ++s) sum += partial[s * total + i];
+        out[i] = sum;
+    }
+}
+
 template <typename T> __device__ __forceinline__ T to_elem(float x);
 template <> __device__ __forceinline__ float to_elem<float>(float x) { return x; }
 template <> __device__ __forceinline__ _Float16 to_elem<_Float16>(float x) { return static_cast<_Float16>(x); }
@@ -362,23 +573,181 @@ void reduce_any(int dtype, const float* c, void* out, const MatmulBatch& ob, con
     else reduce<uint16_t>(c, out, ob, op, rows, cols, R, C, st);
 }
 
-}  // namespace
-
-size_t matmul_workspace_bytes(const MatmulSpec& s) {
+size_t matmul_gathered_bytes(const MatmulSpec& s) {
     return product_bytes(s.dtype, s.batch.count, padded(s.dtype, s.m, s.n, s.k), false);
 }
-
-size_t matmul_backward_workspace_bytes(const MatmulSpec& s) {
+size_t matmul_gathered_backward_bytes(const MatmulSpec& s) {
     const Padded pa = padded(s.dtype, s.m, s.k, s.n), pb = padded(s.dtype, s.k, s.n, s.m);
     return std::max(product_bytes(s.dtype, s.batch.count, pa, true), product_bytes(s.dtype, s.batch.count, pb, true));
 }
 
-hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, int num_cus,
-                  hipStream_t st) {
+// ---- F32 products read in place (matmul_f32_tile)
+
+// One F32 product: the operands' storage and batch strides, C [G][m][n] packed.
+struct F32Product {
+    const float* a;
+    const float* b;
+    MatmulBatch ab, bb;
+    int64_t m, n, k, lda, ldb;
+    bool a_mn, b_mn;
+    bool folded = false;  // the batch has joined M or K: C is the whole result
+};
+
+// Each operand slice and its padded tile edge within 32-bit byte offsets.
+bool f32_fits(const F32Product& x) {
+    auto fits = [](int64_t rows, int64_t ld) { return (rows + 128) * ld * 4 < (int64_t{1} << 31); };
+    return fits(x.a_mn ? x.k : x.m, x.lda) && fits(x.b_mn ? x.k : x.n, x.ldb) && x.ab.count <= 65535 &&
+           x.m <= INT32_MAX - 128 && x.n <= INT32_MAX - 128;
+}
+
+struct F32Choice {
+    bool big;  // 128x128 tiles
+    int splits;
+};
+// The tile and K split (at least 8 steps of 16 k each, partial planes of at most 64 MB) of least
+// estimated time: a 128x128 workgroup takes ~0.95 us a step; 64x64 ones 0.26 us each, but at least 0.42
+// when alone on their CU; a split adds a launch and its planes' traffic.
+F32Choice f32_choose(const F32Product& x, int num_cus, size_t ws_bytes) {
+    const int64_t steps = (x.k + kFK - 1) / kFK, plane = x.ab.count * x.m * x.n * 4;
+    F32Choice best{false, 1};
+    float best_us = INFINITY;
+    for (bool big : {true, false}) {
+        const int64_t w = big ? 128 : 64, tiles = ((x.m + w - 1) / w) * ((x.n + w - 1) / w) * x.ab.count;
+        for (int splits = 1; splits <= 16; ++splits) {
+            if (splits > 1 && (tiles * splits > 4 * num_cus || steps < 8 * splits || plane * splits > (int64_t{64} << 20) ||
+                               static_cast<size_t>(plane * splits) > ws_bytes))
+                break;
+            const int64_t rounds = (tiles * splits + num_cus - 1) / num_cus, per = (steps + splits - 1) / splits;
+            float us = big ? rounds * per * 0.95f : per * fmaxf(rounds * 0.26f, 0.42f);
+            if (splits > 1) us += 4.0f + plane * (splits + 1) * 2.5e-7f;
+            if (us < best_us) best_us = us, best = F32Choice{big, splits};
+        }
+    }
+    return best;
+}
+size_t f32_bytes(const F32Product& x, int num_cus) {
+    const F32Choice c = f32_choose(x, num_cus, SIZE_MAX);
+    return c.splits > 1 ? round256(static_cast<size_t>(x.ab.count * x.m * x.n) * 4 * c.splits) : 0;
+}
+
+template <int T, bool A_MN, bool B_MN>
+void f32_launch_mn(const F32Args& p, bool va, bool vb, const dim3& grid, hipStream_t st) {
+    if (va && vb) hipLaunchKernelGGL((matmul_f32_tile<T, 4, A_MN, B_MN, true, true>), grid, dim3(kThreads), 0, st, p);
+    else if (va) hipLaunchKernelGGL((matmul_f32_tile<T, 4, A_MN, B_MN, true, false>), grid, dim3(kThreads), 0, st, p);
+    else if (vb) hipLaunchKernelGGL((matmul_f32_tile<T, 4, A_MN, B_MN, false, true>), grid, dim3(kThreads), 0, st, p);
+    else hipLaunchKernelGGL((matmul_f32_tile<T, 4, A_MN, B_MN, false, false>), grid, dim3(kThreads), 0, st, p);
+}
+template <int T>
+void f32_launch(const F32Args& p, bool a_mn, bool b_mn, bool va, bool vb, const dim3& grid, hipStream_t st) {
+    if (a_mn && b_mn) f32_launch_mn<T, true, true>(p, va, vb, grid, st);
+    else if (b_mn) f32_launch_mn<T, false, true>(p, va, vb, grid, st);
+    else f32_launch_mn<T, false, false>(p, va, vb, grid, st);  // no product reads only A MN-major
+}
+
+// 16-byte loads: every row of every batch slice 16-byte aligned.
+bool f32_vec(const float* x, const MatmulBatch& b, int64_t ld) {
+    if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || ld % 4 != 0) return false;
+    for (int d = 0; d < b.dims; ++d)
+        if (b.stride[d] % 4 != 0) return false;
+    return true;
+}
+
+void f32_product(const F32Product& x, float* out, void* workspace, size_t ws_bytes, int num_cus, hipStream_t st) {
+    const F32Choice c = f32_choose(x, num_cus, ws_bytes);
+    F32Args p{};
+    p.a = x.a, p.b = x.b, p.ab = x.ab, p.bb = x.bb;
+    p.m = static_cast<int>(x.m), p.n = static_cast<int>(x.n), p.k = static_cast<int>(x.k);
+    p.lda = static_cast<int>(x.lda), p.ldb = static_cast<int>(x.ldb);
+    const int w = c.big ? 128 : 64, steps = (p.k + kFK - 1) / kFK;
+    p.tiles_m = (p.m + w - 1) / w, p.tiles_n = (p.n + w - 1) / w;
+    p.steps_per_split = (steps + c.splits - 1) / c.splits;
+    p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
+    p.c = p.splits > 1 ? static_cast<float*>(workspace) : out;
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits), 1, static_cast<unsigned>(x.ab.count));
+    const bool va = f32_vec(x.a, x.ab, x.lda), vb = f32_vec(x.b, x.bb, x.ldb);
+    if (c.big) f32_launch<2>(p, x.a_mn, x.b_mn, va, vb, grid, st);
+    else f32_launch<1>(p, x.a_mn, x.b_mn, va, vb, grid, st);
+    if (p.splits > 1) {
+        const int64_t total = x.ab.count * x.m * x.n;
+        hipLaunchKernelGGL(sum_planes, dim3(flat_blocks(total, 256)), dim3(256), 0, st, p.c, out, p.splits, total);
+    }
+}
+
+bool is_shared(const MatmulBatch& b) {  // every batch reads the same matrix
+    for (int d = 0; d < b.dims; ++d)
+        if (b.shape[d] > 1 && b.stride[d] != 0) return false;
+    return true;
+}
+bool is_packed(const MatmulBatch& b, int64_t plane) {  // a contiguous [G, plane] operand
+    int64_t st = plane;
+    for (int d = b.dims - 1; d >= 0; --d) {
+        if (b.shape[d] > 1 && b.stride[d] != st) return false;
+        st *= b.shape[d];
+    }
+    return true;
+}
+
+// The three F32 products of a spec: out = A B, dA = dY B^T, dB = A^T dY. With one B for a packed batch
+// of A the batch joins M (dB: the contraction), so B is read once and dB needs no sum over batches.
+F32Product f32_forward(const MatmulSpec& s, const float* a, const float* b) {
+    F32Product x{a, b, s.a_batch, s.b_batch, s.m, s.n, s.k, s.k, s.n, false, true};
+    if (is_shared(s.b_batch) && is_packed(s.a_batch, s.m * s.k)) x.m *= s.batch.count, x.ab = x.bb = MatmulBatch{}, x.folded = true;
+    return x;
+}
+F32Product f32_grad_a(const MatmulSpec& s, const float* dy, const float* b) {
+    F32Product x{dy, b, packed_batch(s.batch, s.m * s.n), s.b_batch, s.m, s.k, s.n, s.n, s.n, false, false};
+    if (is_shared(s.b_batch) && is_packed(s.a_batch, s.m * s.k)) x.m *= s.batch.count, x.ab = x.bb = MatmulBatch{}, x.folded = true;
+    return x;
+}
+F32Product f32_grad_b(const MatmulSpec& s, const float* a, const float* dy) {
+    F32Product x{a, dy, s.a_batch, packed_batch(s.batch, s.m * s.n), s.k, s.n, s.m, s.k, s.n, true, true};
+    if (is_shared(s.b_batch) && is_packed(s.a_batch, s.m * s.k)) x.k *= s.batch.count, x.ab = x.bb = MatmulBatch{}, x.folded = true;
+    return x;
+}
+
+// Bytes of an operand gradient's batch slices, which are summed over the batches the operand broadcasts
+// along (0: the product is the gradient).
+size_t f32_slice_bytes(const F32Product& x, const MatmulBatch& op) {
+    return x.folded || x.ab.count == op.count ? 0 : round256(static_cast<size_t>(x.ab.count * x.m * x.n) * 4);
+}
+
+}  // namespace
+
+Scratch matmul_workspace(const MatmulSpec& s, int num_cus) {
+    if (s.dtype == 0) {
+        const F32Product x = f32_forward(s, nullptr, nullptr);
+        if (f32_fits(x)) return {0, f32_bytes(x, num_cus)};
+    }
+    const size_t bytes = matmul_gathered_bytes(s);
+    return {bytes, bytes};
+}
+
+Scratch matmul_backward_workspace(const MatmulSpec& s, int num_cus) {
+    if (s.dtype == 0) {
+        const F32Product xa = f32_grad_a(s, nullptr, nullptr), xb = f32_grad_b(s, nullptr, nullptr);
+        if (f32_fits(xa) && f32_fits(xb)) {
+            const MatmulBatch oa = operand_shape(s.batch, s.a_batch), ob = operand_shape(s.batch, s.b_batch);
+            const size_t na = f32_slice_bytes(xa, oa), nb = f32_slice_bytes(xb, ob);
+            return {std::max(na, nb), std::max(na + f32_bytes(xa, num_cus), nb + f32_bytes(xb, num_cus))};
+        }
+    }
+    const size_t bytes = matmul_gathered_backward_bytes(s);
+    return {bytes, bytes};
+}
+
+hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, size_t ws_bytes,
+                  int num_cus, hipStream_t st) {
     const int64_t G = s.batch.count;
     const size_t es = s.dtype == 0 ? 4 : 2;
     if (G * s.m * s.n == 0) return hipSuccess;
     if (s.k == 0) return zero_fill(out, G * s.m * s.n * static_cast<int64_t>(es), st);  // an empty contraction
+    if (s.dtype == 0) {
+        const F32Product f = f32_forward(s, static_cast<const float*>(a), static_cast<const float*>(b));
+        if (f32_fits(f)) {
+            f32_product(f, static_cast<float*>(out), workspace, ws_bytes, num_cus, st);
+            return hipGetLastError();
+        }
+    }
     const Padded p = padded(s.dtype, s.m, s.n, s.k);
     const Gather x{a, s.a_batch, s.m, s.k, s.k, 0}, y{b, s.b_batch, s.n, s.k, s.n, 1};
     void* c = nullptr;
@@ -394,7 +763,7 @@ hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, 
 }
 
 hipError_t matmul_backward(const MatmulSpec& s, const void* a, const void* b, const void* dy, void* da, void* db,
-                           void* workspace, int num_cus, hipStream_t st) {
+                           void* workspace, size_t ws_bytes, int num_cus, hipStream_t st) {
     const int64_t G = s.batch.count;
     const size_t es = s.dtype == 0 ? 4 : 2;
     const MatmulBatch oa = operand_shape(s.batch, s.a_batch), obb = operand_shape(s.batch, s.b_batch);
@@ -405,6 +774,25 @@ hipError_t matmul_backward(const MatmulSpec& s, const void* a, const void* b, co
         return zero_fill(db, obb.count * s.k * s.n * static_cast<int64_t>(es), st);
     }
     if (s.k == 0) return hipSuccess;  // dA [.., M, 0] and dB [.., 0, N] hold nothing
+    if (s.dtype == 0) {
+        const F32Product xa = f32_grad_a(s, static_cast<const float*>(dy), static_cast<const float*>(b));
+        const F32Product xb = f32_grad_b(s, static_cast<const float*>(a), static_cast<const float*>(dy));
+        if (f32_fits(xa) && f32_fits(xb)) {
+            auto grad = [&](const F32Product& x, const MatmulBatch& op, void* out) {
+                const size_t bytes = f32_slice_bytes(x, op);
+                if (bytes == 0) {
+                    f32_product(x, static_cast<float*>(out), workspace, ws_bytes, num_cus, st);
+                    return;
+                }
+                float* slices = static_cast<float*>(workspace);  // summed over the broadcast batches
+                f32_product(x, slices, static_cast<char*>(workspace) + bytes, ws_bytes - bytes, num_cus, st);
+                reduce<float>(slices, out, s.batch, op, x.m, x.n, x.m, x.n, st);
+            };
+            grad(xa, oa, da);
+            grad(xb, obb, db);
+            return hipGetLastError();
+        }
+    }
     void* c = nullptr;
     // dA[g] = dY[g] B[g]^T: X = dY [M, N], Y = B as [K, N]; then summed over A's broadcast batches
     {
