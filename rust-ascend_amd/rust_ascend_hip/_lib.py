@@ -39,9 +39,12 @@ class HkError(RuntimeError):
         self.message = message
 
 
+ShapeArray = ctypes.c_int64 * MAX_RANK
+
+
 class HkTensor(ctypes.Structure):
     _fields_ = [("data", ctypes.c_void_p), ("dtype", ctypes.c_int32), ("rank", ctypes.c_int32),
-                ("shape", ctypes.c_int64 * MAX_RANK)]
+                ("shape", ShapeArray)]
 
 
 class HkStats(ctypes.Structure):
@@ -166,6 +169,8 @@ def load(path: str = None):
     """Load libhk.so (the module's LIB_PATH as it stands at the first call, or `path`) and bind
     every entry point; raises HkError(LOAD_ERROR) if absent."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

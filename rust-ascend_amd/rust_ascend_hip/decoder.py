@@ -235,9 +235,11 @@ class DecoderLayer:
 
     def _run(self, calls):
         ctx = runtime._context()
-        check(self._lib.hk_set_stream(ctx, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        check(self._lib.hk_set_stream(ctx, runtime._stream()))
         for fn, args in calls:
-            check(fn(ctx, *args))
+            status = fn(ctx, *args)
+            if status:
+                check(status)
 
     # ------------------------------------------------------------------ public steps
 
