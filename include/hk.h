@@ -400,6 +400,21 @@ hk_status hk_silu_mul(hk_context* ctx, const hk_tensor* gate, const hk_tensor* u
 hk_status hk_silu_mul_backward(hk_context* ctx, const hk_tensor* gate, const hk_tensor* up, const hk_tensor* dy,
                                hk_tensor* dgate, hk_tensor* dup);
 
+/* y = (SiLU(x gate^T) * (x up^T)) down^T with F32 storage and BF16 products: the reference's
+ * nn::swiglu_bf16_fp32 (src/nn/feed_forward.rs:24-42) as one call, with the same roundings (each linear's
+ * operands to BF16, FP32 sums, the gate in F32). x [M,K], gate/up [H,K], down [N,H] F32, every dimension a
+ * positive multiple of 16, 16-byte aligned; what the backward reads is written to x_bf16 [M,K],
+ * gu_bf16 [2H,K] (gate rows, then up rows), down_bf16 [N,H], gu [M,2H] F32 (gate | up) and act_bf16
+ * [M,H]. Operands below 2^30 elements; past that use the separate calls. */
+hk_status hk_swiglu_bf16_fp32(hk_context* ctx, const hk_tensor* x, const hk_tensor* gate, const hk_tensor* up,
+                              const hk_tensor* down, hk_tensor* y, hk_tensor* x_bf16, hk_tensor* gu_bf16,
+                              hk_tensor* down_bf16, hk_tensor* gu, hk_tensor* act_bf16);
+/* F32 gradients of the above from F32 dY [M,N]. dy_bf16 [M,N], dm [M,H] F32 and dgu [M,2H] BF16 are scratch. */
+hk_status hk_swiglu_bf16_fp32_backward(hk_context* ctx, const hk_tensor* dy, const hk_tensor* x_bf16,
+                                       const hk_tensor* gu_bf16, const hk_tensor* down_bf16, const hk_tensor* gu,
+                                       const hk_tensor* act_bf16, hk_tensor* dy_bf16, hk_tensor* dm, hk_tensor* dgu,
+                                       hk_tensor* dx, hk_tensor* dgate, hk_tensor* dup, hk_tensor* ddown);
+
 /* ---------------------------------------------------------------- bias and residual add */
 
 /* y = (x + residual) + bias[c] over the last axis c, in that F32 order; residual may be NULL

@@ -24,6 +24,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/hk.h"
@@ -1401,10 +1402,11 @@ hk_status hk_gemm_bf16_fp32(hk_context* h, const hk_tensor* a, const hk_tensor* 
     size_t gb;
     st = ensure_scratch(g.c, 0, {gemm_scratch(g.c, s, ta, tb, a_bf16->data, b_bf16->data, out->data)}, &gb);
     if (st != HK_OK) return st;
-    hipError_t e = hk::cast_apply(1, a->data, a_bf16->data, numel(a), g.c->stream);
-    if (e == hipSuccess) e = hk::cast_apply(1, b->data, b_bf16->data, numel(b), g.c->stream);
+    const hk::CastJob casts[2] = {{static_cast<const float*>(a->data), a_bf16->data, numel(a)},
+                                  {static_cast<const float*>(b->data), b_bf16->data, numel(b)}};
+    hipError_t e = hk::cast_many(casts, 2, g.c->stream);
     if (e == hipSuccess) run_gemm(g.c, s, a_bf16->data, b_bf16->data, out->data, ta, tb, g.c->workspace, gb, &e);
-    return complete(g.c, e, "gemm_bf16_fp32", 3);
+    return complete(g.c, e, "gemm_bf16_fp32", 2);
 }
 
 hk_status hk_gemm_bf16_fp32_backward(hk_context* h, const hk_tensor* a, const hk_tensor* b, const hk_tensor* dy,
@@ -1826,6 +1828,104 @@ hk_status hk_silu_mul(hk_context* h, const hk_tensor* gate, const hk_tensor* up,
     const int64_t n = numel(gate);
     hipError_t e = hk::silu_mul(gate->dtype == HK_BF16, gate->data, up->data, y->data, n, g.c->stream);
     return complete(g.c, e, "silu_mul", n ? 1 : 0);
+}
+
+namespace {
+// The FP32 SwiGLU block's tensors: X [M,K], gate/up [H,K], down [N,H] (F32 in the forward, their BF16
+// snapshots in the backward), every dimension a positive multiple of 16, products read in place.
+hk_status swiglu_fp32_dims(int64_t m, int64_t k, int64_t hid, int64_t n) {
+    for (int64_t x : {m, k, hid, n})
+        if (x <= 0 || x % 16 != 0 || x > INT32_MAX)
+            return fail(HK_INVALID_ARGUMENT, "SwiGLU requires aligned X[M,K], gate/up[H,K] and down[N,H]");
+    // the six products: (M, 2H, K), (M, N, H), (M, H, N), (N, H, M), (M, K, 2H), (2H, K, M)
+    if (!hk::gemm_reads_in_place(m, 2 * hid, k) || !hk::gemm_reads_in_place(m, n, hid) || !hk::gemm_reads_in_place(m, hid, n) ||
+        !hk::gemm_reads_in_place(n, hid, m) || !hk::gemm_reads_in_place(m, k, 2 * hid) || !hk::gemm_reads_in_place(2 * hid, k, m))
+        return fail(HK_INVALID_ARGUMENT, "fused SwiGLU operands must stay below 2^30 elements (use the composition)");
+    return HK_OK;
+}
+bool matrix_of(const hk_tensor* t, int32_t dtype, int64_t rows, int64_t cols) {
+    return t && t->dtype == dtype && t->rank == 2 && t->shape[0] == rows && t->shape[1] == cols && aligned16({t->data}) && t->data;
+}
+}  // namespace
+
+hk_status hk_swiglu_bf16_fp32(hk_context* h, const hk_tensor* x, const hk_tensor* gate, const hk_tensor* up,
+                              const hk_tensor* down, hk_tensor* y, hk_tensor* x_bf16, hk_tensor* gu_bf16,
+                              hk_tensor* down_bf16, hk_tensor* gu, hk_tensor* act_bf16) {
+    for (const hk_tensor* t : {x, gate, up, down})
+        if (!tensor_ok(t, "SwiGLU input") || t->rank != 2 || t->dtype != HK_F32)
+            return fail(HK_INVALID_ARGUMENT, "SwiGLU requires rank-2 FP32 input and weights");
+    const int64_t M = x->shape[0], K = x->shape[1], H = gate->shape[0], N = down->shape[0];
+    hk_status st = swiglu_fp32_dims(M, K, H, N);
+    if (st != HK_OK) return st;
+    if (!matrix_of(x, HK_F32, M, K) || !matrix_of(gate, HK_F32, H, K) || !matrix_of(up, HK_F32, H, K) ||
+        !matrix_of(down, HK_F32, N, H) || !matrix_of(y, HK_F32, M, N) || !matrix_of(x_bf16, HK_BF16, M, K) ||
+        !matrix_of(gu_bf16, HK_BF16, 2 * H, K) || !matrix_of(down_bf16, HK_BF16, N, H) || !matrix_of(gu, HK_F32, M, 2 * H) ||
+        !matrix_of(act_bf16, HK_BF16, M, H))
+        return fail(HK_INVALID_ARGUMENT, "SwiGLU requires 16-byte aligned X[M,K], gate/up[H,K], down[N,H], Y[M,N] F32 and the "
+                                         "snapshots X, [2H,K], [N,H], act[M,H] BF16, gate|up [M,2H] F32");
+    if (!disjoint({y, x_bf16, gu_bf16, down_bf16, gu, act_bf16}, {x, gate, up, down})) return HK_INVALID_ARGUMENT;
+    OpGuard g(h);
+    if (g.st != HK_OK) return g.st;
+    const int cus = g.c->num_cus;
+    size_t gb;
+    st = ensure_scratch(g.c, 0, {hk::gemm_workspace(1, M, 2 * H, K, HK_NO, HK_YES, false, true, cus),
+                                 hk::gemm_workspace(1, M, N, H, HK_NO, HK_YES, false, true, cus)}, &gb);
+    if (st != HK_OK) return st;
+    uint16_t* w = static_cast<uint16_t*>(gu_bf16->data);
+    const hk::CastJob casts[4] = {{static_cast<const float*>(x->data), x_bf16->data, M * K},
+                                  {static_cast<const float*>(gate->data), w, H * K},
+                                  {static_cast<const float*>(up->data), w + H * K, H * K},
+                                  {static_cast<const float*>(down->data), down_bf16->data, N * H}};
+    hipError_t e = hk::cast_many(casts, 4, g.c->stream);
+    if (e == hipSuccess)
+        e = hk::gemm_bf16(x_bf16->data, w, gu->data, 0, 1, M, 2 * H, K, HK_NO, HK_YES, g.c->workspace, gb, cus, g.c->stream);
+    if (e == hipSuccess) e = hk::silu_mul_rows(static_cast<const float*>(gu->data), act_bf16->data, M, H, g.c->stream);
+    if (e == hipSuccess)
+        e = hk::gemm_bf16(act_bf16->data, down_bf16->data, y->data, 0, 1, M, N, H, HK_NO, HK_YES, g.c->workspace, gb, cus,
+                          g.c->stream);
+    return complete(g.c, e, "swiglu_bf16_fp32", 4);
+}
+
+hk_status hk_swiglu_bf16_fp32_backward(hk_context* h, const hk_tensor* dy, const hk_tensor* x_bf16, const hk_tensor* gu_bf16,
+                                       const hk_tensor* down_bf16, const hk_tensor* gu, const hk_tensor* act_bf16,
+                                       hk_tensor* dy_bf16, hk_tensor* dm, hk_tensor* dgu, hk_tensor* dx, hk_tensor* dgate,
+                                       hk_tensor* dup, hk_tensor* ddown) {
+    for (const hk_tensor* t : {dy, x_bf16, gu_bf16, down_bf16})
+        if (!tensor_ok(t, "SwiGLU input") || t->rank != 2) return fail(HK_INVALID_ARGUMENT, "SwiGLU backward requires rank-2 tensors");
+    const int64_t M = x_bf16->shape[0], K = x_bf16->shape[1], H = gu_bf16->shape[0] / 2, N = down_bf16->shape[0];
+    hk_status st = swiglu_fp32_dims(M, K, H, N);
+    if (st != HK_OK) return st;
+    if (!matrix_of(dy, HK_F32, M, N) || !matrix_of(x_bf16, HK_BF16, M, K) || !matrix_of(gu_bf16, HK_BF16, 2 * H, K) ||
+        !matrix_of(down_bf16, HK_BF16, N, H) || !matrix_of(gu, HK_F32, M, 2 * H) || !matrix_of(act_bf16, HK_BF16, M, H) ||
+        !matrix_of(dy_bf16, HK_BF16, M, N) || !matrix_of(dm, HK_F32, M, H) || !matrix_of(dgu, HK_BF16, M, 2 * H) ||
+        !matrix_of(dx, HK_F32, M, K) || !matrix_of(dgate, HK_F32, H, K) || !matrix_of(dup, HK_F32, H, K) ||
+        !matrix_of(ddown, HK_F32, N, H))
+        return fail(HK_INVALID_ARGUMENT, "SwiGLU backward requires the forward's snapshots, F32 dY[M,N], scratch dY[M,N] BF16, "
+                                         "dM[M,H] F32, dgate|dup[M,2H] BF16 and F32 gradients of X, gate, up and down");
+    if (!disjoint({dy_bf16, dm, dgu, dx, dgate, dup, ddown}, {dy, x_bf16, gu_bf16, down_bf16, gu, act_bf16}))
+        return HK_INVALID_ARGUMENT;
+    OpGuard g(h);
+    if (g.st != HK_OK) return g.st;
+    const int cus = g.c->num_cus;
+    size_t gb;
+    st = ensure_scratch(g.c, 0, {hk::gemm_workspace(1, M, H, N, HK_NO, HK_NO, false, true, cus),
+                                 hk::gemm_workspace(1, N, H, M, HK_YES, HK_NO, false, true, cus),
+                                 hk::gemm_workspace(1, M, K, 2 * H, HK_NO, HK_NO, false, true, cus)}, &gb);
+    if (st != HK_OK) return st;
+    void* ws = g.c->workspace;
+    hipStream_t s = g.c->stream;
+    const hk::CastJob cast = {static_cast<const float*>(dy->data), dy_bf16->data, M * N};
+    hipError_t e = hk::cast_many(&cast, 1, s);
+    // dM = dY down, then (dgate | dup) in BF16, the operand of the two products over gate|up
+    if (e == hipSuccess) e = hk::gemm_bf16(dy_bf16->data, down_bf16->data, dm->data, 0, 1, M, H, N, HK_NO, HK_NO, ws, gb, cus, s);
+    if (e == hipSuccess) e = hk::gemm_bf16(dy_bf16->data, act_bf16->data, ddown->data, 0, 1, N, H, M, HK_YES, HK_NO, ws, gb, cus, s);
+    if (e == hipSuccess)
+        e = hk::silu_mul_rows_backward(static_cast<const float*>(gu->data), static_cast<const float*>(dm->data), dgu->data, M, H, s);
+    if (e == hipSuccess) e = hk::gemm_bf16(dgu->data, gu_bf16->data, dx->data, 0, 1, M, K, 2 * H, HK_NO, HK_NO, ws, gb, cus, s);
+    if (e == hipSuccess)
+        e = hk::gemm_bf16_two_outputs(dgu->data, x_bf16->data, static_cast<float*>(dgate->data), static_cast<float*>(dup->data), H,
+                                      2 * H, K, M, HK_YES, HK_NO, cus, s);
+    return complete(g.c, e, "swiglu_bf16_fp32_backward", 6);
 }
 
 hk_status hk_silu_mul_backward(hk_context* h, const hk_tensor* gate, const hk_tensor* up, const hk_tensor* dy,
@@ -2671,11 +2771,17 @@ struct Staged {
 Staged staged(const hk_tensor* t) {
     return {t->data, t->dtype == HK_F32 ? ws_round(static_cast<size_t>(numel(t)) * 2) : 0};
 }
-hipError_t stage(const hk_tensor* t, Staged& st, char*& cursor, hipStream_t s) {
-    if (!st.bytes) return hipSuccess;
-    st.p = cursor;
-    cursor += st.bytes;
-    return hk::cast_apply(1, t->data, const_cast<void*>(st.p), numel(t), s);
+// Rounds the tensors that need it into the workspace at cursor, in one launch.
+hipError_t stage(std::initializer_list<std::pair<const hk_tensor*, Staged*>> tensors, char*& cursor, hipStream_t s) {
+    hk::CastJob jobs[4];
+    int count = 0;
+    for (const auto& t : tensors) {
+        if (!t.second->bytes) continue;
+        t.second->p = cursor;
+        jobs[count++] = {static_cast<const float*>(t.first->data), cursor, numel(t.first)};
+        cursor += t.second->bytes;
+    }
+    return hk::cast_many(jobs, count, s);
 }
 }  // namespace
 
@@ -2700,13 +2806,11 @@ hk_status hk_attention_forward(hk_context* h, const hk_tensor* q, const hk_tenso
     st = ensure_scratch(g.c, staging, {{0, hk::attention_fwd_workspace_bytes(sh, g.c->num_cus)}}, &split_bytes);
     if (st != HK_OK) return st;
     char* cursor = static_cast<char*>(g.c->workspace);
-    hipError_t e = stage(q, sq, cursor, g.c->stream);
-    if (e == hipSuccess) e = stage(k, sk, cursor, g.c->stream);
-    if (e == hipSuccess) e = stage(v, sv, cursor, g.c->stream);
+    hipError_t e = stage({{q, &sq}, {k, &sk}, {v, &sv}}, cursor, g.c->stream);
     if (e == hipSuccess)
         e = hk::attention_forward(sh, sq.p, sk.p, sv.p, o->data, static_cast<float*>(lse->data),
                                   static_cast<char*>(g.c->workspace) + staging, split_bytes, g.c->num_cus, g.c->stream);
-    return complete(g.c, e, "attention_forward", 1 + (sq.bytes ? 3 : 0));
+    return complete(g.c, e, "attention_forward", 1 + (sq.bytes ? 1 : 0));
 }
 
 namespace {
@@ -2772,10 +2876,7 @@ hk_status attention_backward_common(hk_context* h, const hk_tensor* q, const hk_
     }
     if (st != HK_OK) return st;
     char* cursor = static_cast<char*>(g.c->workspace) + stat_bytes;
-    hipError_t e = stage(q, sq, cursor, g.c->stream);
-    if (e == hipSuccess) e = stage(k, sk, cursor, g.c->stream);
-    if (e == hipSuccess) e = stage(v, sv, cursor, g.c->stream);
-    if (e == hipSuccess) e = stage(dout, sd, cursor, g.c->stream);
+    hipError_t e = stage({{q, &sq}, {k, &sk}, {v, &sv}, {dout, &sd}}, cursor, g.c->stream);
     if (e == hipSuccess)
         e = hk::attention_backward(sh, sq.p, sk.p, sv.p, o->data, static_cast<const float*>(lse->data), sd.p,
                                    rows ? nullptr : dq->data, rows ? 1 : dq->dtype == HK_BF16,
@@ -2783,7 +2884,7 @@ hk_status attention_backward_common(hk_context* h, const hk_tensor* q, const hk_
                                    rows ? 1 : dk->dtype == HK_BF16, rows ? &rows_out : nullptr, g.c->workspace,
                                    g.c->stream);
     return complete(g.c, e, rows ? "attention_backward_qkv_rows" : "attention_backward",
-                    3 + (sq.bytes ? 3 : 0) + (sd.bytes ? 1 : 0));
+                    3 + (sq.bytes || sd.bytes ? 1 : 0));
 }
 }  // namespace
 

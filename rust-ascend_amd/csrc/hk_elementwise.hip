@@ -165,6 +165,56 @@ scale_to_bf16_kernel(const float* __restrict__ x, float scale, uint16_t* __restr
 
 }  // namespace
 
+// The FP32 SwiGLU block: gate and up come from one GEMM as rows (gate | up), and the products on either side
+// take BF16, so the element-wise passes write BF16 directly: 10 bytes per value forward instead of 18
+// (silu_mul, then a cast), 16 backward instead of 32.
+namespace {
+__global__ void __launch_bounds__(kEwThreads)
+silu_mul_rows_kernel(const float* __restrict__ gu, uint16_t* __restrict__ act, int64_t chunks, int width) {
+    const int per = width / 8;
+    for (int64_t i = flat_begin(kEwThreads); i < chunks; i += flat_stride(kEwThreads)) {
+        const int64_t row = i / per;
+        const int c = static_cast<int>(i - row * per) * 8;
+        float g[8], u[8], y[8];
+        load8(gu + row * 2 * width + c, g);
+        load8(gu + row * 2 * width + width + c, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = silu_mul1(g[e], u[e]);
+        store8(act + row * width + c, y);
+    }
+}
+__global__ void __launch_bounds__(kEwThreads)
+silu_mul_rows_bwd_kernel(const float* __restrict__ gu, const float* __restrict__ dm, uint16_t* __restrict__ dgu, int64_t chunks, int width) {
+    const int per = width / 8;
+    for (int64_t i = flat_begin(kEwThreads); i < chunks; i += flat_stride(kEwThreads)) {
+        const int64_t row = i / per;
+        const int c = static_cast<int>(i - row * per) * 8;
+        float g[8], u[8], d[8], dg[8], du[8];
+        load8(gu + row * 2 * width + c, g);
+        load8(gu + row * 2 * width + width + c, u);
+        load8(dm + row * width + c, d);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) silu_mul_bwd1(g[e], u[e], d[e], dg[e], du[e]);
+        store8(dgu + row * 2 * width + c, dg);
+        store8(dgu + row * 2 * width + width + c, du);
+    }
+}
+}  // namespace
+
+hipError_t silu_mul_rows(const float* gu, void* act, int64_t rows, int64_t width, hipStream_t s) {
+    const int64_t chunks = rows * (width / 8);
+    hipLaunchKernelGGL(silu_mul_rows_kernel, dim3(flat_blocks(chunks, kEwThreads)), dim3(kEwThreads), 0, s, gu,
+                       static_cast<uint16_t*>(act), chunks, static_cast<int>(width));
+    return hipGetLastError();
+}
+
+hipError_t silu_mul_rows_backward(const float* gu, const float* dm, void* dgu, int64_t rows, int64_t width, hipStream_t s) {
+    const int64_t chunks = rows * (width / 8);
+    hipLaunchKernelGGL(silu_mul_rows_bwd_kernel, dim3(flat_blocks(chunks, kEwThreads)), dim3(kEwThreads), 0, s, gu, dm,
+                       static_cast<uint16_t*>(dgu), chunks, static_cast<int>(width));
+    return hipGetLastError();
+}
+
 hipError_t scale_mask(float* scores, const float* mask, float scale, int64_t n, hipStream_t s) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(scale_mask_kernel, dim3(blocks_for(n)), dim3(kEwThreads), 0, s, scores, mask, scale, n);

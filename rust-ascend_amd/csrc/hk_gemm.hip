@@ -480,6 +480,24 @@ hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_
     return hipGetLastError();
 }
 
+hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* c2, int64_t m_split, int64_t m, int64_t n,
+                                 int64_t k, int ta, int tb, int num_cus, hipStream_t s) {
+    if (!in_place_applies(m, n, k, aligned16({a, b, c, c2})) || m_split % 16 != 0) return hipErrorInvalidValue;
+    GemmArgs p{};
+    p.a = static_cast<const uint16_t*>(a);
+    p.b = static_cast<const uint16_t*>(b);
+    p.c = c;
+    p.c2 = reinterpret_cast<void*>(reinterpret_cast<uintptr_t>(c2) - static_cast<uintptr_t>(m_split * n) * sizeof(float));
+    p.m_split = static_cast<int>(m_split);
+    p.m = static_cast<int>(m);
+    p.n = static_cast<int>(n);
+    p.k = static_cast<int>(k);
+    launch_choice(choose_gemm(1, m, n, k, ta != 0, false, 0, num_cus), p, 1, false, ta != 0, tb == 0, nullptr, s);
+    return hipGetLastError();
+}
+
+bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k) { return in_place_applies(m, n, k, true); }
+
 bool epi_applies(int64_t m, int64_t n, int64_t k) {
     const int64_t k64 = (k + kPK - 1) / kPK * kPK;
     return m > 0 && n > 0 && k > 0 && k % 8 == 0 && m * k64 * 2 < (int64_t{1} << 31) &&

@@ -21,6 +21,9 @@ struct GemmArgs {
     // M-grouped form (batch 1): block_group[r / 256] is the weight slice of rows r of A and C.
     // Group ends are multiples of 256, so an output tile (at most 256 rows) has one group.
     const int32_t* block_group;
+    // F32 outputs: rows from m_split on go to c2 (c2 + m n is row m's place), null: all rows to c.
+    void* c2;
+    int m_split;
     // 4-wave kernel tile order: 0 = bands of 4 M-tile rows per XCD, else bands of this many
     // N-tile columns.
     int band_n;
@@ -65,6 +68,11 @@ __device__ __forceinline__ const uint16_t* weight_slice(const GemmArgs& p, int r
     return p.b + slice * static_cast<int64_t>(p.n) * p.k;
 }
 
+
+// Base of row m of an F32 output.
+__device__ __forceinline__ float* out_f32(const GemmArgs& p, int m) {
+    return static_cast<float*>(p.c2 != nullptr && m >= p.m_split ? p.c2 : p.c);
+}
 
 // The compiler may not move instructions across this point.
 __device__ __forceinline__ void phase_fence() { __builtin_amdgcn_sched_barrier(0); }
@@ -550,7 +558,7 @@ __device__ __forceinline__ void gemm_m16_tile(Args p) {
                 u32x2_t w = {pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
                 *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(p.c) + off) = w;
             } else {
-                *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.c) + off) = acc[i][j];
+                *reinterpret_cast<f32x4_t*>(out_f32(p, m) + off) = acc[i][j];
             }
         }
     }

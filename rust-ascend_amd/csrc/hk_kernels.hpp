@@ -42,6 +42,13 @@ hipError_t rope_apply(int dtype_bf16, const void* x, const float* cos_t, const f
                       int64_t rows, int64_t width, int64_t p, int layout, int backward,
                       const RopeMap& map, hipStream_t s);
 hipError_t cast_apply(int to_bf16, const void* in, void* out, int64_t n, hipStream_t s);
+// F32 -> BF16 of up to 4 tensors in one launch.
+struct CastJob {
+    const float* in;
+    void* out;
+    int64_t n;
+};
+hipError_t cast_many(const CastJob* jobs, int count, hipStream_t s);
 
 // ---- GEMM (hk_gemm.hip)
 // C[g] = op(A[g]) op(B[g]) for g < batch; A, B BF16; C BF16 or F32. ta/tb as in the
@@ -95,6 +102,11 @@ hipError_t matmul_backward(const MatmulSpec& s, const void* a, const void* b, co
                            void* workspace, size_t ws_bytes, int num_cus, hipStream_t st);
 hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_t batch, int64_t m,
                      int64_t n, int64_t k, int ta, int tb, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s);
+// One product whose F32 rows [0, m_split) go to c and [m_split, m) to c2 (each packed, m_split % 16 == 0).
+// 16-byte aligned tensors, M, N, K that gemm_reads_in_place takes. No workspace.
+hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* c2, int64_t m_split, int64_t m, int64_t n,
+                                 int64_t k, int ta, int tb, int num_cus, hipStream_t s);
+bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k);
 // M-grouped NT GEMM: C[i, :] = A[i, :] W[g(i)]^T with A [m, k], W [groups, n, k], C [m, n];
 // g(i) = block_group[i / 256] (group ends are multiples of 256). No workspace.
 hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_bf16, int64_t m, int64_t n,
@@ -149,6 +161,11 @@ hipError_t crop_f32(const float* src, float* dst, int64_t batch, int64_t rows, i
 // ---- element-wise (hk_elementwise.hip)
 // SwiGLU gate, element-wise over n values of F32 or BF16 storage.
 hipError_t silu_mul(int dtype_bf16, const void* gate, const void* up, void* y, int64_t n, hipStream_t s);
+// The FP32 SwiGLU block's element-wise passes over gu [rows, 2 width] F32 (gate | up): act [rows, width] BF16 =
+// bf16(SiLU(gate) * up); dgu [rows, 2 width] BF16 = (dgate | dup) from dm [rows, width] F32. width % 8 == 0,
+// 16-byte aligned.
+hipError_t silu_mul_rows(const float* gu, void* act, int64_t rows, int64_t width, hipStream_t s);
+hipError_t silu_mul_rows_backward(const float* gu, const float* dm, void* dgu, int64_t rows, int64_t width, hipStream_t s);
 // Composed attention helpers: scores = scores * scale (+ mask), in place; out = bf16(scale * x).
 hipError_t scale_mask(float* scores, const float* mask, float scale, int64_t n, hipStream_t s);
 hipError_t scale_to_bf16(const float* x, float scale, void* out, int64_t n, hipStream_t s);

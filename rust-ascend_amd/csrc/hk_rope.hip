@@ -241,6 +241,32 @@ cast_f32_to_bf16(const float* __restrict__ in, uint16_t* __restrict__ out, int64
     }
 }
 
+// cast_f32_to_bf16 of up to four tensors: job j takes blocks [first[j], first[j + 1]) of 2048 values each.
+// One launch instead of one per operand (each a few us for the sizes of a projection).
+struct CastJobs {
+    const float* in[4];
+    uint16_t* out[4];
+    int64_t n[4];
+    int64_t first[5];
+    int vec[4];
+};
+__global__ void __launch_bounds__(256)
+cast_many_kernel(CastJobs c) {
+    for (int64_t block = blockIdx.x; block < c.first[4]; block += gridDim.x) {
+        const int j = block >= c.first[2] ? (block >= c.first[3] ? 3 : 2) : (block >= c.first[1] ? 1 : 0);
+        const int64_t i = (block - c.first[j]) * 2048 + threadIdx.x * 8, n = c.n[j];
+        const float* in = c.in[j];
+        uint16_t* out = c.out[j];
+        if (c.vec[j] && i + 8 <= n) {
+            float v[8];
+            load8(in + i, v);
+            store8(out + i, v);
+        } else {
+            for (int64_t e = i; e < n && e < i + 8; ++e) out[e] = f32_to_bf16(in[e]);
+        }
+    }
+}
+
 __global__ void __launch_bounds__(256)
 cast_bf16_to_f32(const uint16_t* __restrict__ in, float* __restrict__ out, int64_t n, int vec) {
     for (int64_t i = flat_begin(256) * 8; i < n; i += flat_stride(256) * 8) {
@@ -261,6 +287,24 @@ hipError_t rope_apply(int dtype_bf16, const void* x, const float* cos_t, const f
                       const RopeMap& map, hipStream_t s) {
     return dtype_bf16 ? rope_t<uint16_t>(x, cos_t, sin_t, y, rows, width, p, layout, backward != 0, map, s)
                       : rope_t<float>(x, cos_t, sin_t, y, rows, width, p, layout, backward != 0, map, s);
+}
+
+hipError_t cast_many(const CastJob* jobs, int count, hipStream_t s) {
+    CastJobs c{};
+    int64_t blocks = 0;
+    for (int j = 0; j < 4; ++j) {
+        c.first[j] = blocks;
+        if (j >= count) continue;
+        c.in[j] = jobs[j].in;
+        c.out[j] = static_cast<uint16_t*>(jobs[j].out);
+        c.n[j] = jobs[j].n;
+        c.vec[j] = aligned16({jobs[j].in, jobs[j].out});
+        blocks += (jobs[j].n + 2047) / 2048;
+    }
+    c.first[4] = blocks;
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(cast_many_kernel, dim3(flat_blocks(blocks, 1)), dim3(256), 0, s, c);
+    return hipGetLastError();
 }
 
 hipError_t cast_apply(int to_bf16, const void* in, void* out, int64_t n, hipStream_t s) {

@@ -124,6 +124,8 @@ SIGNATURES = {
     "hk_cast_into": [_CTX, _T, _T],
     "hk_silu_mul": [_CTX, _T, _T, _T],
     "hk_silu_mul_backward": [_CTX, _T, _T, _T, _T, _T],
+    "hk_swiglu_bf16_fp32": [_CTX] + [_T] * 10,
+    "hk_swiglu_bf16_fp32_backward": [_CTX] + [_T] * 13,
     "hk_bias_add": [_CTX, _T, _T, _T, _T],
     "hk_bias_add_backward": [_CTX, _T, _T],
     "hk_nll_loss": [_CTX, _T, _T, _T, _i32, ctypes.c_int64, _T, _T],

@@ -328,6 +328,25 @@ def embedding(weight: torch.Tensor, ids: torch.Tensor, padding_idx=None, scale_g
     return _Embedding.apply(weight.contiguous(), ids.contiguous(), padding_idx, bool(scale_grad_by_freq))
 
 
+class _SwigluBf16Fp32(torch.autograd.Function):
+    """The composition below as one node: X is rounded once, gate and up are one product each way and
+    the element-wise passes write the next product's BF16 operand. Saves the BF16 snapshots of X, the
+    weights and the activation, and gate and up in F32, as the composition's nodes do."""
+
+    @staticmethod
+    def forward(ctx, x, gate, up, down):
+        y, *saved = HipRuntime.swiglu_bf16_fp32(x, gate, up, down)
+        ctx.save_for_backward(*saved)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        dy = dy.contiguous().float()
+        if dy.data_ptr() % 16:
+            dy = dy.clone()
+        return HipRuntime.swiglu_bf16_fp32_backward(dy, *ctx.saved_tensors)
+
+
 def swiglu_bf16_fp32(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor) -> torch.Tensor:
     """(SiLU(x gate^T) * (x up^T)) down^T with F32 storage and BF16 linear compute.
     Reference: nn::swiglu_bf16_fp32 (src/nn/feed_forward.rs:24-42): gate/up [H,K], down [N,H],
@@ -339,7 +358,11 @@ def swiglu_bf16_fp32(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down
         raise ValueError("SwiGLU requires aligned X[M,K], gate/up[H,K] and down[N,H]")
     if any(t.dtype != torch.float32 for t in (x, gate, up, down)):
         raise ValueError("SwiGLU requires FP32 input and weights")
-    g = linear_bf16_fp32(x, gate)
+    tensors = [t.contiguous() for t in (x, gate, up, down)]
+    if 2 * h * max(k, m) < 1 << 29 and n * max(h, m) < 1 << 29 and m * k < 1 << 29 and \
+            all(t.data_ptr() % 16 == 0 for t in tensors):
+        return _SwigluBf16Fp32.apply(*tensors)
+    g = linear_bf16_fp32(x, gate)  # operands past the fused call's 32-bit offsets or off its alignment
     u = linear_bf16_fp32(x, up)
     return linear_bf16_fp32(silu_mul(g, u), down)
 

@@ -473,6 +473,29 @@ class HipRuntime:
         _call("hk_silu_mul_backward", desc(gate), desc(up), desc(grad), desc(dg), desc(du))
         return dg, du
 
+    @staticmethod
+    def swiglu_bf16_fp32(x, gate, up, down):
+        """[F32 Y, and what the backward reads: BF16 X, gate|up weights and down, F32 gate|up, BF16 act] of
+        the FP32 SwiGLU block (nn::swiglu_bf16_fp32, src/nn/feed_forward.rs:24-42) in one call."""
+        (m, k), (h, _), n = x.shape, gate.shape, down.shape[0]
+        bf = torch.bfloat16
+        y, gu = _empty((m, n), torch.float32, x), _empty((m, 2 * h), torch.float32, x)
+        xb, wb, db, act = _empty((m, k), bf, x), _empty((2 * h, k), bf, x), _empty((n, h), bf, x), _empty((m, h), bf, x)
+        _call("hk_swiglu_bf16_fp32", desc(x), desc(gate), desc(up), desc(down), desc(y), desc(xb), desc(wb), desc(db),
+              desc(gu), desc(act))
+        return y, xb, wb, db, gu, act
+
+    @staticmethod
+    def swiglu_bf16_fp32_backward(grad, x_bf16, gu_bf16, down_bf16, gu, act_bf16):
+        """[F32 dX, dgate, dup, ddown] of the FP32 SwiGLU block."""
+        (m, k), n, h = x_bf16.shape, down_bf16.shape[0], down_bf16.shape[1]
+        f32, bf = torch.float32, torch.bfloat16
+        dyb, dm, dgu = _empty((m, n), bf, grad), _empty((m, h), f32, grad), _empty((m, 2 * h), bf, grad)
+        dx, dg, du, dd = (_empty(s, f32, grad) for s in ((m, k), (h, k), (h, k), (n, h)))
+        _call("hk_swiglu_bf16_fp32_backward", desc(grad), desc(x_bf16), desc(gu_bf16), desc(down_bf16), desc(gu),
+              desc(act_bf16), desc(dyb), desc(dm), desc(dgu), desc(dx), desc(dg), desc(du), desc(dd))
+        return dx, dg, du, dd
+
     # ---------------------------------------------------------------- bias and residual add
 
     @staticmethod
