@@ -1684,48 +1684,58 @@ attn_bwd_dkdv(BwdArgs a) {
     }
 }
 
-// The splits' F32 partial dK (scaled) and dV of 128 keys of one (batch, KV head), added in split
-// order and stored by dkdv_store (BF16/F32 planes or rows output; scale 1, the partials carry it)
-// in the dK/dV kernel's lane layout: the result is what that kernel stores unsplit, up to the
-// order of the F32 additions.
+// The splits' F32 partial dK (scaled) and dV, added in split order and stored as the unsplit kernel
+// stores them (BF16/F32 planes or the rows output with RoPE's transpose on dK; each value rounded to
+// BF16 before its rotation), up to the order of the F32 additions. A thread takes 4 values at d and
+// the 4 at d + D / 2 (a split-half pair's other member) of one gradient row, D / 8 threads a row, so the
+// planes are read in whole lines by as many workgroups as they hold (one workgroup per 128 keys, each
+// lane walking a row of its own: B1 Hkv4 N512 D128, 4 splits 24 us; now, 8 splits, 6).
 template <int D>
 __global__ void __launch_bounds__(kThreads)
-attn_bwd_dkdv_reduce(BwdArgs a) {
-    constexpr int DP = D < 32 ? 32 : D;
-    constexpr int DT = DP / 32;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lq = lane & 31, lg = lane >> 5;
-    const int bkv = blockIdx.x / a.blocks, nb = blockIdx.x % a.blocks;
-    const int64_t b = bkv / a.kv_heads, kvh = bkv % a.kv_heads;
-    const int64_t my_key = static_cast<int64_t>(nb) * kKBlock + wave * 32 + lq;
-    if (my_key >= a.n) return;
-    const int64_t nkv = a.n * static_cast<int64_t>(gridDim.x / a.blocks);
-    f32x16_t dk[DT], dv[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) dk[dt][v] = dv[dt][v] = 0.0f;
+attn_bwd_dkdv_reduce(BwdArgs a, int64_t nkv) {
+    constexpr int kPer = D / 8;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    const int d = static_cast<int>(i % kPer) * 4;
+    const int64_t key = i / kPer % nkv;           // (b Hkv + kv head) n + key
+    const int which = static_cast<int>(i / kPer / nkv);  // 0: dK, 1: dV
+    if (which > 1) return;
+    float x[4] = {0.0f, 0.0f, 0.0f, 0.0f}, y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int sp = 0; sp < a.splits; ++sp) {
-        const float* pk = a.partial + ((static_cast<int64_t>(sp) * 2) * nkv + static_cast<int64_t>(bkv) * a.n + my_key) * D;
-        const float* pv = pk + nkv * D;
+        const float* p = a.partial + ((static_cast<int64_t>(sp) * 2 + which) * nkv + key) * D + d;
+        const f32x4_t u = *reinterpret_cast<const f32x4_t*>(p), v = *reinterpret_cast<const f32x4_t*>(p + D / 2);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int e = 0; e < 4; ++e) x[e] += u[e], y[e] += v[e];
+    }
+    if constexpr (D >= 64) {
+        if (a.rows != nullptr) {
+            const int64_t bkv = key / a.n, s = key - bkv * a.n, b = bkv / a.kv_heads, kvh = bkv % a.kv_heads;
+            const int64_t head = which == 0 ? a.heads + kvh : a.heads + a.kv_heads + kvh;
+            uint16_t* row = a.rows + (b * a.m + s) * a.row_w + head * D + d;
+            if (which == 0) {
+                const float* ct = a.rope_cos + s * (D / 2);
+                const float* st = a.rope_sin + s * (D / 2);
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int d = 32 * dt + 8 * g4 + 4 * lg;
-                if (d >= D) continue;
-                const f32x4_t k4 = *reinterpret_cast<const f32x4_t*>(pk + d);
-                const f32x4_t v4 = *reinterpret_cast<const f32x4_t*>(pv + d);
+                for (int e = 0; e < 4; ++e) x[e] = round_bf16(x[e]), y[e] = round_bf16(y[e]);
+                if (a.rope_layout == 1) {  // pairs (d + e, d + e + D / 2)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    dk[dt][4 * g4 + e] += k4[e];
-                    dv[dt][4 * g4 + e] += v4[e];
+                    for (int e = 0; e < 4; ++e) rope_rotate<true>(x[e], y[e], ct[d + e], st[d + e], x[e], y[e]);
+                } else {  // pairs (d, d + 1) and (d + 2, d + 3) of each half
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        const int t = (d + e) / 2;
+                        rope_rotate<true>(x[e], x[e + 1], ct[t], st[t], x[e], x[e + 1]);
+                        rope_rotate<true>(y[e], y[e + 1], ct[t + D / 4], st[t + D / 4], y[e], y[e + 1]);
+                    }
                 }
             }
+            *reinterpret_cast<u32x2_t*>(row) = u32x2_t{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+            *reinterpret_cast<u32x2_t*>(row + D / 2) = u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+            return;
+        }
     }
-    BwdArgs ra = a;
-    ra.scale = 1.0f;
-    dkdv_store<D, DT>(ra, b, kvh, bkv, my_key, lg, dk, dv);
+    void* out = which == 0 ? a.dk : a.dv;
+    store_row4<D>(out, a.dkv_bf16, key, d, x);
+    store_row4<D>(out, a.dkv_bf16, key, d + D / 2, y);
 }
 
 // dQ of 128 queries of one (batch, head), looping over 64-key tiles up to the diagonal:
@@ -2104,7 +2114,7 @@ size_t stat_bytes(const AttnShape& sh) {  // row statistic and lse2, rounded to 
 // Workgroups per dK/dV key block: causal key blocks near the start of the sequence see every
 // query and those near its end few of them, so a grid of one round of workgroups (C5: 256 key
 // blocks on 256 CUs) takes as long as its heaviest block, ~1.9x the average at C5. Splitting
-// every block's steps s ways (s = 2 or 4) lets the dispatcher fill the CUs evenly: s is the
+// every block's steps s ways (s = 2, 4 or 8) lets the dispatcher fill the CUs evenly: s is the
 // smallest whose heaviest share is at most the average work per CU, i.e. ratio = heaviest block x
 // CUs / all blocks' work <= s (1 when the ratio is at most 1: C4's four rounds already balance).
 // The environment variable HK_ATTN_DKV_SPLITS (1, 2 or 4) overrides the choice.
@@ -2125,7 +2135,10 @@ int dkv_splits_for(const AttnShape& sh, int num_cus) {
     work *= sh.batch * sh.kv_heads;
     if (work == 0) return 1;
     const double ratio = static_cast<double>(heaviest) * num_cus / static_cast<double>(work);
-    return ratio <= 1.0 ? 1 : (ratio <= 2.0 ? 2 : 4);
+    // 8 where the heaviest block is above 8 average shares (B1 Hq16 Hkv4 512 tokens D128, 16 key blocks: this
+    // kernel 34 -> 24 us against 4 splits); a split takes a query step at least
+    const int splits = ratio <= 1.0 ? 1 : (ratio <= 2.0 ? 2 : (ratio <= 8.0 ? 4 : 8));
+    return splits == 8 && qsteps < 8 ? 4 : splits;
 }
 size_t partial_bytes(const AttnShape& sh) {  // the split's F32 dK and dV partial sums
     return sh.dkv_splits > 1 ? static_cast<size_t>(sh.dkv_splits) * 2 * sh.batch * sh.kv_heads * sh.n * sh.d * 4 : 0;
@@ -2179,8 +2192,9 @@ hipError_t launch_bwd(const AttnShape& sh, const void* q, const void* k, const v
     const dim3 dkdv_grid(static_cast<unsigned>(sh.batch * sh.kv_heads * a.blocks * a.splits));
     if (a.splits > 1) {
         hipLaunchKernelGGL((attn_bwd_dkdv<D, true>), dkdv_grid, dim3(kThreads), 0, s, a);
-        hipLaunchKernelGGL((attn_bwd_dkdv_reduce<D>), dim3(static_cast<unsigned>(sh.batch * sh.kv_heads * a.blocks)),
-                           dim3(kThreads), 0, s, a);
+        const int64_t nkv = sh.batch * sh.kv_heads * sh.n;
+        hipLaunchKernelGGL((attn_bwd_dkdv_reduce<D>), dim3(static_cast<unsigned>((nkv * 2 * (D / 8) + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, s, a, nkv);
     } else {
         hipLaunchKernelGGL((attn_bwd_dkdv<D, false>), dkdv_grid, dim3(kThreads), 0, s, a);
     }
