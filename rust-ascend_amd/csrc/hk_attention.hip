@@ -44,7 +44,6 @@ constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kBlockM = 128;  // query rows per forward workgroup (4 waves x 32)
 constexpr int kBlockN = 64;   // keys per K/V tile
 constexpr int kThreads = 256;
-constexpr int kXcds = 8;     // accelerator complex dies; workgroups are dispatched round-robin over them
 
 
 // 16-byte chunk swizzle of a tile row (XOR applied to the chunk index). gfx950's LDS has 64
@@ -115,15 +114,6 @@ __device__ __forceinline__ void settle(bf16x8_t (&v)[N]) {
     for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
 }
 __device__ __forceinline__ void settle(float& v) { asm volatile("" : "+v"(v)); }
-
-// Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2. Renumbering
-// blockIdx so that each XCD runs one contiguous range of a logical order lets a kernel place
-// the workgroups that share operands on the same XCD.
-__device__ __forceinline__ int xcd_logical() {
-    const int nwg = static_cast<int>(gridDim.x), id = static_cast<int>(blockIdx.x);
-    const int xcd = id % kXcds, per_xcd = nwg / kXcds, extra = nwg % kXcds;
-    return xcd * per_xcd + (xcd < extra ? xcd : extra) + id / kXcds;
-}
 
 struct FwdArgs {
     const uint16_t* q;

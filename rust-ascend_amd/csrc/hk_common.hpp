@@ -286,6 +286,16 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2. Renumbering
+// blockIdx so that each XCD runs one contiguous range of a logical order lets a kernel place
+// the workgroups that share operands on the same XCD.
+constexpr int kXcds = 8;  // accelerator complex dies
+__device__ __forceinline__ int xcd_logical() {
+    const int nwg = static_cast<int>(gridDim.x), id = static_cast<int>(blockIdx.x);
+    const int xcd = id % kXcds, per_xcd = nwg / kXcds, extra = nwg % kXcds;
+    return xcd * per_xcd + (xcd < extra ? xcd : extra) + id / kXcds;
+}
+
 // ---- global->LDS loads (buffer_load ... lds)
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));

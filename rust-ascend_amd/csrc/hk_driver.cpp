@@ -3002,12 +3002,26 @@ hk_status ensure_planned(Ctx* c, const std::function<void(Carve&, hipError_t*, C
     return st;
 }
 
-// BF16 operand: `t` itself when BF16, else its RNE rounding into the workspace.
-const void* bf16_operand(const hk_tensor* t, Carve& w, hipError_t* e, hipStream_t s) {
-    if (t->dtype == HK_BF16) return t->data;
-    void* p = w.take(static_cast<size_t>(numel(t)) * 2);
-    if (w.base && *e == hipSuccess) *e = hk::cast_apply(1, t->data, p, numel(t), s);
-    return p;
+// BF16 operands: a tensor itself when BF16, else its RNE rounding into the workspace (one launch for all).
+struct Operands {
+    hk::CastJob jobs[4];
+    int count = 0;
+    const void* add(const hk_tensor* t, Carve& w) {
+        if (t->dtype == HK_BF16) return t->data;
+        void* p = w.take(static_cast<size_t>(numel(t)) * 2);
+        jobs[count++] = {static_cast<const float*>(t->data), p, numel(t)};
+        return p;
+    }
+    void cast(hipError_t* e, hipStream_t s) const {
+        if (*e == hipSuccess) *e = hk::cast_many(jobs, count, s);
+    }
+};
+
+// K or V's fragments for the kernels that hold the scores in registers, in the workspace.
+hk::PackJob packed(const hk_tensor* t, const ComposedShape& sh, bool transposed, Carve& w) {
+    hk::PackJob j{t->data, nullptr, static_cast<int>(t->shape[t->rank - 1]), t->dtype == HK_BF16, transposed};
+    j.out = static_cast<uint16_t*>(w.take(hk::packed_bytes(j, sh.groups(), sh.n)));
+    return j;
 }
 
 // The scores bf16(Q) bf16(K)^T, F32 [B*Hkv, rows, N].
@@ -3058,17 +3072,30 @@ hk_status hk_attention_masked_forward(hk_context* h, const hk_tensor* q, const h
     const bool aligned = aligned16({q->data, k->data, v->data, o->data});
     const float* mask_data = mask ? static_cast<const float*>(mask->data) : nullptr;
     const bool fused = hk::masked_softmax_applies(sh.n, mask_data, nullptr);
+    const bool direct = aligned && aligned16({mask_data}) && hk::masked_attention_applies(G, R, sh.n, sh.d, sh.dv);
     bool lean = false;
     auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
-        const void* qb = bf16_operand(q, w, e, c ? c->stream : nullptr);
-        const void* kb = bf16_operand(k, w, e, c ? c->stream : nullptr);
-        const void* vb = bf16_operand(v, w, e, c ? c->stream : nullptr);
+        Operands ops;
+        const void* qb = ops.add(q, w);
+        if (direct) {
+            hk::PackJob jobs[] = {packed(k, sh, false, w), packed(v, sh, true, w)};
+            if (!c) return;
+            ops.cast(e, c->stream);
+            if (*e == hipSuccess) *e = hk::pack_attention_operands(jobs, 2, G, sh.n, c->stream);
+            if (*e == hipSuccess)
+                *e = hk::masked_attention_forward(qb, jobs[0].out, jobs[1].out, mask_data, scale, o->data,
+                                                  o->dtype == HK_BF16, G, R, sh.n, sh.d, sh.dv, c->stream);
+            return;
+        }
+        const void* kb = ops.add(k, w);
+        const void* vb = ops.add(v, w);
         float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));
         float* p = fused ? nullptr : static_cast<float*>(w.take(sh.scores() * 4));
         void* pb = w.take(sh.scores() * 2);
         const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
         void* gws = w.take(gb);
         if (!c) return;
+        ops.cast(e, c->stream);
         composed_scores(sh, qb, kb, sbuf, gws, gb, cus, c->stream, e);
         if (fused) {
             if (*e == hipSuccess) *e = hk::masked_softmax(sbuf, mask_data, scale, pb, G * R, sh.n, c->stream);
@@ -3086,7 +3113,7 @@ hk_status hk_attention_masked_forward(hk_context* h, const hk_tensor* q, const h
     if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
     plan(w, &e, g.c, g.c->num_cus);
-    return complete(g.c, e, "attention_masked_forward", fused ? 4 : 6);
+    return complete(g.c, e, "attention_masked_forward", direct ? 3 : (fused ? 4 : 6));
 }
 
 hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const hk_tensor* k, const hk_tensor* v,
@@ -3124,13 +3151,34 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
     const float* mask_data = mask ? static_cast<const float*>(mask->data) : nullptr;
     float* dmask_data = dmask ? static_cast<float*>(dmask->data) : nullptr;
     const bool fused = hk::masked_softmax_applies(sh.n, mask_data, dmask_data);
+    const bool direct = aligned && aligned16({mask_data, dmask_data}) &&
+                        hk::masked_attention_applies(G, R, sh.n, sh.d, sh.dv);
     bool lean = false;
     auto plan = [&](Carve& w, hipError_t* e, Ctx* c, int cus) {
         hipStream_t s = c ? c->stream : nullptr;
-        const void* qb = bf16_operand(q, w, e, s);
-        const void* kb = bf16_operand(k, w, e, s);
-        const void* vb = bf16_operand(v, w, e, s);
-        const void* dob = bf16_operand(dout, w, e, s);
+        Operands ops;
+        const void* qb = ops.add(q, w);
+        const void* dob = ops.add(dout, w);
+        if (direct) {
+            hk::PackJob jobs[] = {packed(k, sh, false, w), packed(v, sh, false, w), packed(k, sh, true, w)};
+            void* p = w.take(sh.scores() * 2);   // bf16(P)
+            void* ds = w.take(sh.scores() * 2);  // bf16(scale * dS)
+            const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
+            void* gws = w.take(gb);
+            if (!c) return;
+            ops.cast(e, s);
+            if (*e == hipSuccess) *e = hk::pack_attention_operands(jobs, 3, G, sh.n, s);
+            if (*e == hipSuccess)
+                *e = hk::masked_attention_backward(qb, jobs[0].out, jobs[1].out, jobs[2].out, dob, mask_data, scale, p, ds,
+                                                   dmask_data, dq->data, dq->dtype == HK_BF16, G, R, sh.n, sh.d, sh.dv, s);
+            if (*e == hipSuccess)
+                *e = hk::gemm_bf16(ds, qb, dk->data, dk->dtype == HK_BF16, G, sh.n, sh.d, R, HK_YES, HK_NO, gws, gb, cus, s);
+            if (*e == hipSuccess)
+                *e = hk::gemm_bf16(p, dob, dv->data, dv->dtype == HK_BF16, G, sh.n, sh.dv, R, HK_YES, HK_NO, gws, gb, cus, s);
+            return;
+        }
+        const void* kb = ops.add(k, w);
+        const void* vb = ops.add(v, w);
         float* sbuf = static_cast<float*>(w.take(sh.scores() * 4));  // scores (not fused: then dP)
         // fused: dP, in dMask's buffer when there is one; otherwise P
         float* f32 = fused && dmask_data ? dmask_data : static_cast<float*>(w.take(sh.scores() * 4));
@@ -3141,6 +3189,7 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
         const size_t gb = composed_gemm_ws(sh, aligned, lean, cus);
         void* gws = w.take(gb);
         if (!c) return;
+        ops.cast(e, s);
         // P is recomputed (the reference keeps it in its autodiff graph); dP = bf16(dO) bf16(V)^T;
         // dS = P * (dP - rowsum(P * dP)) (softmax_backward); dMask = dS
         composed_scores(sh, qb, kb, sbuf, gws, gb, cus, s, e);
@@ -3170,7 +3219,7 @@ hk_status hk_attention_masked_backward(hk_context* h, const hk_tensor* q, const 
     if ((st = ensure_planned(g.c, plan, &lean)) != HK_OK) return st;
     Carve w{static_cast<char*>(g.c->workspace)};
     plan(w, &e, g.c, g.c->num_cus);
-    return complete(g.c, e, "attention_masked_backward", fused ? 8 : 11);
+    return complete(g.c, e, "attention_masked_backward", direct ? 5 : (fused ? 8 : 11));
 }
 
 }  // extern "C"

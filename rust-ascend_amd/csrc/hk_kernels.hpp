@@ -221,6 +221,29 @@ hipError_t masked_softmax(const float* scores, const float* mask, float scale, v
 hipError_t masked_softmax_backward(const float* scores, const float* mask, const float* dp, float scale, void* p, void* dsb,
                                    float* ds, int64_t rows, int64_t width, hipStream_t s);
 
+// The materialized attention with its scores in registers (hk_attention_masked.hip): `groups` KV heads of
+// `rows` query rows, n keys, head width d, value width dv; Q and dO are BF16 rows, mask [groups][rows][n]
+// F32 or null. K and V come as BF16 fragments that pack_attention_operands makes (one launch for up to
+// three): ks, vs for the score products, vt, kt for the products with P and dS. The backward writes p =
+// bf16(P), ds = bf16(scale dS), dQ and, when given, dmask = dS in F32. Applies up to 2304 keys; every
+// pointer is 16-byte aligned.
+struct PackJob {
+    const void* in;  // [groups][n][w] F32 or BF16
+    uint16_t* out;
+    int w;
+    int bf16, transposed;
+};
+size_t packed_bytes(const PackJob& j, int64_t groups, int64_t n);
+hipError_t pack_attention_operands(const PackJob* jobs, int count, int64_t groups, int64_t n, hipStream_t s);
+bool masked_attention_applies(int64_t groups, int64_t rows, int64_t n, int64_t d, int64_t dv);
+hipError_t masked_attention_forward(const void* q, const void* ks, const void* vt, const float* mask, float scale, void* o,
+                                    bool out_bf16, int64_t groups, int64_t rows, int64_t n, int64_t d, int64_t dv,
+                                    hipStream_t s);
+hipError_t masked_attention_backward(const void* q, const void* ks, const void* vs, const void* kt, const void* dout,
+                                     const float* mask, float scale, void* p, void* ds, float* dmask, void* dq,
+                                     bool dq_bf16, int64_t groups, int64_t rows, int64_t n, int64_t d, int64_t dv,
+                                     hipStream_t s);
+
 // Composed-attention compatibility kernels (hk_heads.hip); F32, contiguous.
 hipError_t causal_mask(float* out, int64_t batch, int64_t queries, int64_t keys, uint64_t query_start,
                        uint64_t key_start, hipStream_t s);
