@@ -496,6 +496,25 @@ hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* 
     return hipGetLastError();
 }
 
+bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, int64_t m, int64_t n, int64_t k, int ta,
+                       int tb, int64_t rows, int64_t cols, size_t ws_bytes, int num_cus, hipStream_t s, hipError_t* e) {
+    if (!in_place_applies(m, n, k, aligned16({a, b}))) return false;
+    const GemmChoice ch = choose_gemm(batch, m, n, k, ta != 0, false, ws_bytes, num_cus);
+    if (ch.splits > 1) return false;
+    GemmArgs p{};
+    p.a = static_cast<const uint16_t*>(a);
+    p.b = static_cast<const uint16_t*>(b);
+    p.c = c;
+    p.m = static_cast<int>(m);
+    p.n = static_cast<int>(n);
+    p.k = static_cast<int>(k);
+    p.crop_m = static_cast<int>(rows);
+    p.crop_n = static_cast<int>(cols);
+    launch_choice(ch, p, batch, false, ta != 0, tb == 0, nullptr, s);
+    *e = hipGetLastError();
+    return true;
+}
+
 bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k) { return in_place_applies(m, n, k, true); }
 
 bool epi_applies(int64_t m, int64_t n, int64_t k) {

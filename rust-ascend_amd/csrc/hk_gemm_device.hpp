@@ -24,6 +24,9 @@ struct GemmArgs {
     // F32 outputs: rows from m_split on go to c2 (c2 + m n is row m's place), null: all rows to c.
     void* c2;
     int m_split;
+    // F32 outputs: only rows below crop_m and columns below crop_n are wanted, c is [batch][crop_m][crop_n]
+    // of any alignment (crop_n 0: all of them, as [batch][m][n]).
+    int crop_m, crop_n;
     // 4-wave kernel tile order: 0 = bands of 4 M-tile rows per XCD, else bands of this many
     // N-tile columns.
     int band_n;
@@ -72,6 +75,19 @@ __device__ __forceinline__ const uint16_t* weight_slice(const GemmArgs& p, int r
 // Base of row m of an F32 output.
 __device__ __forceinline__ float* out_f32(const GemmArgs& p, int m) {
     return static_cast<float*>(p.c2 != nullptr && m >= p.m_split ? p.c2 : p.c);
+}
+// Columns n..n + 3 of row m of batch g of a cropped output.
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void store_cropped(const GemmArgs& p, int64_t g, int m, int n, const f32x4_t& v) {
+    if (m >= p.crop_m) return;
+    float* out = static_cast<float*>(p.c) + (g * p.crop_m + m) * p.crop_n + n;
+    if (n + 4 <= p.crop_n) {
+        *reinterpret_cast<f32x4_any_t*>(out) = v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (n + e < p.crop_n) out[e] = v[e];
+    }
 }
 
 // The compiler may not move instructions across this point.
@@ -544,6 +560,17 @@ __device__ __forceinline__ void gemm_m16_tile(Args p) {
             }
         }
         return;
+    }
+    if constexpr (!OUT_BF16) {
+        if (p.crop_n != 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    store_cropped(p, g, tm * kPPTile + 128 * wm + 16 * i + l16, tn * kTileN + kWaveN * wn + 16 * j + 4 * lg,
+                                  acc[i][j]);
+            return;
+        }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {

@@ -223,6 +223,15 @@ gemm_mid_kernel(MidArgs p) {
         }
         return;
     }
+    if constexpr (!OUT_BF16) {
+        if (p.crop_n != 0) {  // never split
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) store_cropped(p, g, m0 + 16 * i, n0 + 16 * j + 4 * lg, acc[i][j]);
+            return;
+        }
+    }
     // partial planes: [split][batch][m][n] F32
     const int64_t plane = p.splits > 1 ? static_cast<int64_t>(split) * gridDim.z + g : g;
 #pragma unroll

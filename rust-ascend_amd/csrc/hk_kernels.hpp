@@ -106,6 +106,11 @@ hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_
 // 16-byte aligned tensors, M, N, K that gemm_reads_in_place takes. No workspace.
 hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* c2, int64_t m_split, int64_t m, int64_t n,
                                  int64_t k, int ta, int tb, int num_cus, hipStream_t s);
+// A product of which only rows x cols of the m x n outputs are wanted, written to c [batch][rows][cols]
+// (any alignment). False, with nothing launched, for the products that only gemm_bf16 runs (operands
+// that it transposes, K splits in ws_bytes).
+bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, int64_t m, int64_t n, int64_t k, int ta,
+                       int tb, int64_t rows, int64_t cols, size_t ws_bytes, int num_cus, hipStream_t s, hipError_t* e);
 bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k);
 // M-grouped NT GEMM: C[i, :] = A[i, :] W[g(i)]^T with A [m, k], W [groups, n, k], C [m, n];
 // g(i) = block_group[i / 256] (group ends are multiples of 256). No workspace.
@@ -155,6 +160,12 @@ hipError_t nll_loss_backward(int dtype, int id_bytes, const void* grad, const vo
 hipError_t pad_bf16(int src_bf16, const void* src, void* dst, int64_t batch, int64_t rows, int64_t cols, int64_t R,
                     int64_t C, hipStream_t s);
 // dst [batch, rows, cols] = the leading window of src [batch, R, C] (F32).
+struct PadJob {
+    const void* src;  // F32 [batch, rows, cols]
+    void* dst;        // [batch, R, C]
+    int64_t rows, cols, R, C;
+};
+hipError_t pad_bf16_two(const PadJob& a, const PadJob& b, int64_t batch, hipStream_t s);
 hipError_t crop_f32(const float* src, float* dst, int64_t batch, int64_t rows, int64_t cols, int64_t R, int64_t C,
                     hipStream_t s);
 

@@ -57,47 +57,59 @@ crop_f32_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t 
     }
 }
 
-// pad_bf16_kernel's result, row by row: destination row rb of [batch, R, C] (its batch and row
-// from one division per row), thread j its 8 columns 8j .. 8j+7 as one 16-byte store. Where all 8
-// exist in the source and vec_src (the source rows are 16-byte aligned), one 16-byte (BF16) or two
-// (F32) loads; else per element, zero outside the source. BF16 is copied bit for bit, F32 rounded
-// as pad_bf16_kernel rounds it.
+// pad_bf16_kernel's result, row by row, of up to two matrices in one launch: destination row rb of [batch,
+// R, C] (its batch and row from one division per row), thread j its 8 columns 8j .. 8j+7 as one
+// 16-byte store. Where all 8 exist in the source, F32 loads them as two vectors of any 4-byte
+// alignment (rows of odd length: with eight strided loads a thread, 1777 x 2001, 3003 x 2001 and 1777 x
+// 3003 took 47 us in three launches, so 19 in two; 90 MB) and BF16 as one where vec says that its rows are 16-byte aligned; else per element, zero outside the
+// source. BF16 is copied bit for bit, F32 rounded as pad_bf16_kernel rounds it.
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+struct PadRows {
+    const void* src;
+    uint16_t* dst;
+    int64_t rows, cols, R, C, nrows;
+    int vec;
+};
+
+template <typename T>
+__device__ __forceinline__ void pad_row(const PadRows& p, int64_t rb) {
+    const int64_t b = rb / p.R, r = rb - b * p.R;
+    const T* srow = static_cast<const T*>(p.src) + (b * p.rows + r) * p.cols;  // read only for r < rows
+    uint16_t* drow = p.dst + rb * p.C;
+    for (int64_t j = threadIdx.x; j < p.C / 8; j += kPadThreads) {  // C is a multiple of 16
+        const int64_t c0 = 8 * j;
+        u32x4_t w;
+        if ((sizeof(T) == 4 || p.vec) && r < p.rows && c0 + 8 <= p.cols) {
+            if constexpr (sizeof(T) == 2) {
+                w = *reinterpret_cast<const u32x4_t*>(srow + c0);
+            } else {
+                const f32x4_any_t u = *reinterpret_cast<const f32x4_any_t*>(srow + c0);
+                const f32x4_any_t v = *reinterpret_cast<const f32x4_any_t*>(srow + c0 + 4);
+                w = u32x4_t{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+        } else {
+            uint16_t h[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                h[e] = 0;
+                if (r < p.rows && c0 + e < p.cols) {
+                    if constexpr (sizeof(T) == 4) h[e] = f32_to_bf16(srow[c0 + e]);
+                    else h[e] = srow[c0 + e];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = static_cast<uint32_t>(h[2 * i]) | (static_cast<uint32_t>(h[2 * i + 1]) << 16);
+        }
+        *reinterpret_cast<u32x4_t*>(drow + c0) = w;
+    }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kPadThreads)
-pad_rows_kernel(const T* __restrict__ src, uint16_t* __restrict__ dst, int64_t rows, int64_t cols, int64_t R,
-                int64_t C, int64_t nrows, int vec_src) {
-    const int64_t chunks = C / 8;  // C is a multiple of 16
-    for (int64_t rb = blockIdx.x; rb < nrows; rb += gridDim.x) {
-        const int64_t b = rb / R, r = rb - b * R;
-        const T* srow = src + (b * rows + r) * cols;  // read only for r < rows
-        uint16_t* drow = dst + rb * C;
-        for (int64_t j = threadIdx.x; j < chunks; j += kPadThreads) {
-            const int64_t c0 = 8 * j;
-            u32x4_t w;
-            if (vec_src && r < rows && c0 + 8 <= cols) {
-                if constexpr (sizeof(T) == 2) {
-                    w = *reinterpret_cast<const u32x4_t*>(srow + c0);
-                } else {
-                    float v[8];
-                    load8(srow + c0, v);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-                }
-            } else {
-                uint16_t h[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    h[e] = 0;
-                    if (r < rows && c0 + e < cols) {
-                        if constexpr (sizeof(T) == 4) h[e] = f32_to_bf16(srow[c0 + e]);
-                        else h[e] = srow[c0 + e];
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) w[i] = static_cast<uint32_t>(h[2 * i]) | (static_cast<uint32_t>(h[2 * i + 1]) << 16);
-            }
-            *reinterpret_cast<u32x4_t*>(drow + c0) = w;
-        }
+pad_rows_kernel(PadRows p, PadRows q) {
+    for (int64_t rb = blockIdx.x; rb < p.nrows + q.nrows; rb += gridDim.x) {
+        if (rb < p.nrows) pad_row<T>(p, rb);
+        else pad_row<T>(q, rb - p.nrows);
     }
 }
 
@@ -123,6 +135,13 @@ crop_rows_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t
 unsigned blocks_for(int64_t work) { return flat_blocks(work, kPadThreads); }
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+template <typename T>
+void launch_pad_rows(const PadRows& p, const PadRows& q, hipStream_t s) {
+    const int64_t nrows = p.nrows + q.nrows;
+    hipLaunchKernelGGL(pad_rows_kernel<T>, dim3(static_cast<unsigned>(nrows < kMaxFlatBlocks ? nrows : kMaxFlatBlocks)),
+                       dim3(kPadThreads), 0, s, p, q);
+}
+
 }  // namespace
 
 hipError_t pad_bf16(int src_bf16, const void* src, void* dst, int64_t batch, int64_t rows, int64_t cols, int64_t R,
@@ -130,15 +149,9 @@ hipError_t pad_bf16(int src_bf16, const void* src, void* dst, int64_t batch, int
     const int64_t pairs = batch * R * C / 2;
     if (pairs == 0) return hipSuccess;
     if (C >= 512 && aligned16(dst)) {
-        const int64_t nrows = batch * R;
-        const int vec = aligned16(src) && cols % (src_bf16 ? 8 : 4) == 0;
-        const dim3 grid(static_cast<unsigned>(nrows < kMaxFlatBlocks ? nrows : kMaxFlatBlocks));
-        if (src_bf16)
-            hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, grid, dim3(kPadThreads), 0, s, static_cast<const uint16_t*>(src),
-                               static_cast<uint16_t*>(dst), rows, cols, R, C, nrows, vec);
-        else
-            hipLaunchKernelGGL(pad_rows_kernel<float>, grid, dim3(kPadThreads), 0, s, static_cast<const float*>(src),
-                               static_cast<uint16_t*>(dst), rows, cols, R, C, nrows, vec);
+        const PadRows p{src, static_cast<uint16_t*>(dst), rows, cols, R, C, batch * R, aligned16(src) && cols % 8 == 0};
+        if (src_bf16) launch_pad_rows<uint16_t>(p, PadRows{}, s);
+        else launch_pad_rows<float>(p, PadRows{}, s);
         return hipGetLastError();
     }
     if (src_bf16)
@@ -148,6 +161,18 @@ hipError_t pad_bf16(int src_bf16, const void* src, void* dst, int64_t batch, int
         hipLaunchKernelGGL(pad_bf16_kernel<float>, dim3(blocks_for(pairs)), dim3(kPadThreads), 0, s,
                            static_cast<const float*>(src), static_cast<uint16_t*>(dst), rows, cols, R, C, pairs);
     return hipGetLastError();
+}
+
+hipError_t pad_bf16_two(const PadJob& a, const PadJob& b, int64_t batch, hipStream_t s) {
+    if (a.C >= 512 && b.C >= 512 && aligned16(a.dst) && aligned16(b.dst)) {
+        auto rows = [&](const PadJob& j) {
+            return PadRows{j.src, static_cast<uint16_t*>(j.dst), j.rows, j.cols, j.R, j.C, batch * j.R, 0};
+        };
+        launch_pad_rows<float>(rows(a), rows(b), s);
+        return hipGetLastError();
+    }
+    const hipError_t e = pad_bf16(0, a.src, a.dst, batch, a.rows, a.cols, a.R, a.C, s);
+    return e != hipSuccess ? e : pad_bf16(0, b.src, b.dst, batch, b.rows, b.cols, b.R, b.C, s);
 }
 
 hipError_t crop_f32(const float* src, float* dst, int64_t batch, int64_t rows, int64_t cols, int64_t R, int64_t C,
