@@ -531,7 +531,7 @@ namespace {
 // The tile of a fused-epilogue product (K is never split: the epilogue needs the whole sum): the
 // 256x256 kernel for full grids as choose_gemm has it, else the least estimated time of those built.
 // The products of a 512-token layer of hidden 2048 made 16-88 workgroups of 256x256; with these tiles
-// its two residual projections take 46 us instead of 187, gate/up 49 (66), the SwiGLU backward 28 (66)
+// its two residual projections take 46 us instead of 187, gate/up 44 (66; 50 on 128x128 pairs), the SwiGLU backward 28 (66)
 // and the QKV projection 20 (63).
 int pick_epi_tile(int64_t m, int64_t n, int64_t k, std::initializer_list<int> built, int num_cus) {
     const GemmChoice full = choose_gemm(1, m, n, k, false, true, 0, num_cus);
@@ -568,7 +568,8 @@ hipError_t launch_epi(GemmEpiArgs p, int num_cus, hipStream_t s) {
             default: break;
         }
     } else {
-        switch (pick_epi_tile(p.m, p.n, p.k, {kT128Pair, kT64x128, kT64}, num_cus)) {
+        switch (pick_epi_tile(p.m, p.n, p.k, {kT256x128, kT128Pair, kT64x128, kT64}, num_cus)) {
+            case kT256x128: launch_epi_mid<2, 2, 8, 4, 3, 1, EPI, B_MN>(p, s); return hipGetLastError();
             case kT128Pair: launch_epi_mid<2, 2, 4, 4, 2, 2, EPI, B_MN>(p, s); return hipGetLastError();
             case kT64x128: launch_epi_mid<2, 2, 2, 4, 3, 2, EPI, B_MN>(p, s); return hipGetLastError();
             case kT64: launch_epi_mid<2, 2, 2, 2, 4, 2, EPI, B_MN>(p, s); return hipGetLastError();
