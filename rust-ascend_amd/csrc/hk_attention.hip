@@ -2104,9 +2104,13 @@ size_t stat_bytes(const AttnShape& sh) {  // row statistic and lse2, rounded to 
 // Workgroups per dK/dV key block: causal key blocks near the start of the sequence see every
 // query and those near its end few of them, so a grid of one round of workgroups (C5: 256 key
 // blocks on 256 CUs) takes as long as its heaviest block, ~1.9x the average at C5. Splitting
-// every block's steps s ways (s = 2, 4 or 8) lets the dispatcher fill the CUs evenly: s is the
-// smallest whose heaviest share is at most the average work per CU, i.e. ratio = heaviest block x
-// CUs / all blocks' work <= s (1 when the ratio is at most 1: C4's four rounds already balance).
+// every block's steps s ways (s = 2, 4 or 8) lets the dispatcher fill the CUs evenly: by ratio = heaviest
+// block x CUs / all blocks' work, about the smallest s >= ratio (1 when the ratio is at most 1: C4's four
+// rounds already balance). Whole backward, us, with 1, 2, 4 and 8 (2.75 leaves the partial sums' traffic of 4 to those
+// that gain by it):
+//   B2 Hq8 Hkv8 1747 D64     ratio 2.13    83  74  88 114      B2 Hq32 Hkv8 1024 D128   ratio 3.56   211 142 129 162
+//   B1 Hq32 Hkv8 3000 D128   ratio 2.61   573 369 371 409      B2 Hq8 Hkv2 1900 D128    ratio 8.0    352 206 138 141
+//   B1 Hq16 Hkv4 2048 D128   ratio 7.53   375 219 141 146      B4 Hq8 Hkv2 512 D128     ratio 12.8   108  74  56  46
 // The environment variable HK_ATTN_DKV_SPLITS (1, 2 or 4) overrides the choice.
 int dkv_splits_for(const AttnShape& sh, int num_cus) {
     if (const char* env = std::getenv("HK_ATTN_DKV_SPLITS")) {
@@ -2125,9 +2129,8 @@ int dkv_splits_for(const AttnShape& sh, int num_cus) {
     work *= sh.batch * sh.kv_heads;
     if (work == 0) return 1;
     const double ratio = static_cast<double>(heaviest) * num_cus / static_cast<double>(work);
-    // 8 where the heaviest block is above 8 average shares (B1 Hq16 Hkv4 512 tokens D128, 16 key blocks: this
-    // kernel 34 -> 24 us against 4 splits); a split takes a query step at least
-    const int splits = ratio <= 1.0 ? 1 : (ratio <= 2.0 ? 2 : (ratio <= 8.0 ? 4 : 8));
+    // a split takes a query step at least
+    const int splits = ratio <= 1.0 ? 1 : (ratio <= 2.75 ? 2 : (ratio <= 8.0 ? 4 : 8));
     return splits == 8 && qsteps < 8 ? 4 : splits;
 }
 size_t partial_bytes(const AttnShape& sh) {  // the split's F32 dK and dV partial sums
