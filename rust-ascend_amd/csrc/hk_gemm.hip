@@ -496,11 +496,30 @@ hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* 
     return hipGetLastError();
 }
 
+bool gemm_bf16_pair(const void* a, const void* b, float* c, float* c2, int64_t batch, int64_t m, int64_t n, int64_t k,
+                    int ta, int tb, int num_cus, hipStream_t s, hipError_t* e) {
+    if (!in_place_applies(m, n, k, aligned16({a, b, c, c2}))) return false;
+    const GemmChoice ch = choose_gemm(2 * batch, m, n, k, ta != 0, false, 0, num_cus);
+    if (ch.tile <= kT256x192) return false;
+    GemmArgs p{};
+    p.a = static_cast<const uint16_t*>(a);
+    p.b = static_cast<const uint16_t*>(b);
+    p.c = c;
+    p.c2 = reinterpret_cast<void*>(reinterpret_cast<uintptr_t>(c2) - static_cast<uintptr_t>(batch * m * n) * sizeof(float));
+    p.m_split = p.g_split = static_cast<int>(batch);
+    p.m = static_cast<int>(m);
+    p.n = static_cast<int>(n);
+    p.k = static_cast<int>(k);
+    launch_choice(ch, p, 2 * batch, false, ta != 0, tb == 0, nullptr, s);
+    *e = hipGetLastError();
+    return true;
+}
+
 bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, int64_t m, int64_t n, int64_t k, int ta,
                        int tb, int64_t rows, int64_t cols, size_t ws_bytes, int num_cus, hipStream_t s, hipError_t* e) {
     if (!in_place_applies(m, n, k, aligned16({a, b}))) return false;
     const GemmChoice ch = choose_gemm(batch, m, n, k, ta != 0, false, ws_bytes, num_cus);
-    if (ch.splits > 1) return false;
+    if (ch.splits > 1 || ch.tile <= kT256x192) return false;
     GemmArgs p{};
     p.a = static_cast<const uint16_t*>(a);
     p.b = static_cast<const uint16_t*>(b);

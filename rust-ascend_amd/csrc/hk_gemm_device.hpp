@@ -24,9 +24,10 @@ struct GemmArgs {
     // F32 outputs: rows from m_split on go to c2 (c2 + m n is row m's place), null: all rows to c.
     void* c2;
     int m_split;
-    // F32 outputs: only rows below crop_m and columns below crop_n are wanted, c is [batch][crop_m][crop_n]
-    // of any alignment (crop_n 0: all of them, as [batch][m][n]).
-    int crop_m, crop_n;
+    // F32 outputs of the tiles below 256x256 (there these stores cost the largest products 0.3%): batches from
+    // g_split on go to c2; only rows below crop_m and columns below crop_n are wanted, c is [batch][crop_m][crop_n]
+    // of any alignment (0: all of them, as [batch][m][n]).
+    int g_split, crop_m, crop_n;
     // 4-wave kernel tile order: 0 = bands of 4 M-tile rows per XCD, else bands of this many
     // N-tile columns.
     int band_n;
@@ -560,17 +561,6 @@ __device__ __forceinline__ void gemm_m16_tile(Args p) {
             }
         }
         return;
-    }
-    if constexpr (!OUT_BF16) {
-        if (p.crop_n != 0) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    store_cropped(p, g, tm * kPPTile + 128 * wm + 16 * i + l16, tn * kTileN + kWaveN * wn + 16 * j + 4 * lg,
-                                  acc[i][j]);
-            return;
-        }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {

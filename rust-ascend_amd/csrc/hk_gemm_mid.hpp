@@ -247,7 +247,7 @@ gemm_mid_kernel(MidArgs p) {
                 u32x2_t w = {pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
                 *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(p.c) + off) = w;
             } else {
-                *reinterpret_cast<f32x4_t*>((p.splits > 1 ? p.partial : out_f32(p, m)) + off) = acc[i][j];
+                *reinterpret_cast<f32x4_t*>((p.splits > 1 ? p.partial : out_f32(p, p.g_split != 0 ? static_cast<int>(g) : m)) + off) = acc[i][j];
             }
         }
     }

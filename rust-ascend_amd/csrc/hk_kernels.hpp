@@ -106,9 +106,14 @@ hipError_t gemm_bf16(const void* a, const void* b, void* c, int out_bf16, int64_
 // 16-byte aligned tensors, M, N, K that gemm_reads_in_place takes. No workspace.
 hipError_t gemm_bf16_two_outputs(const void* a, const void* b, float* c, float* c2, int64_t m_split, int64_t m, int64_t n,
                                  int64_t k, int ta, int tb, int num_cus, hipStream_t s);
+// Two products of one shape in one launch: a and b hold 2 batch matrices each, the first half's F32 products
+// go to c and the second's to c2. False, with nothing launched, for products on 256-wide tiles or with operands
+// that gemm_bf16 transposes.
+bool gemm_bf16_pair(const void* a, const void* b, float* c, float* c2, int64_t batch, int64_t m, int64_t n, int64_t k,
+                    int ta, int tb, int num_cus, hipStream_t s, hipError_t* e);
 // A product of which only rows x cols of the m x n outputs are wanted, written to c [batch][rows][cols]
 // (any alignment). False, with nothing launched, for the products that only gemm_bf16 runs (operands
-// that it transposes, K splits in ws_bytes).
+// that it transposes, K splits in ws_bytes, 256-wide tiles).
 bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, int64_t m, int64_t n, int64_t k, int ta,
                        int tb, int64_t rows, int64_t cols, size_t ws_bytes, int num_cus, hipStream_t s, hipError_t* e);
 bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k);
