@@ -9,7 +9,7 @@
 // A GEMM per score matrix and a row pass over them wrote and read 4 bytes a score two (forward) or
 // five (backward) times; here a score exists only as an accumulator, so what is left is the mask's 4
 // bytes (and the backward's 2 + 2 bytes of P and dS, 4 of a mask gradient). 32 heads of 1040 x 1056
-// scores, D = Dv = 64: forward 126 -> 55 us, backward 285 -> 156 (92 of them this kernel; the mask and
+// scores, D = Dv = 64: forward 126 -> 55 us, backward 285 -> 140 (92 of them this kernel; the mask and
 // the stores would take 26 and 52 at 5.5 TB/s). What bounds them besides is the address unit (16 clocks
 // for a 1 KB operand load, 36 of them per wave and 32 columns) and the arithmetic of 20 instructions a
 // score, both overlapped with the traffic by two workgroups on a CU.
