@@ -117,7 +117,13 @@ hk_status hk_get_stats(hk_context* ctx, hk_stats* out);
  * a backward whose dS buffer cannot be allocated falls back to the recompute form). No
  * reference counterpart: the reference allocates per call (runtime/matrix.rs:33-44).
  * hk_workspace_size reports its size in bytes; hk_trim_workspace frees it, after the queued
- * work, when it holds more than keep_bytes (0: always). */
+ * work, when it holds more than keep_bytes (0: always).
+ * Stream capture: the F32 partial sums of split GEMMs, F32 matmuls and few-query attention forwards
+ * are optional scratch, and on a capturing stream these calls run unsplit without it, so a graph of
+ * them holds no workspace address. Scratch that an op cannot do without (operand rounding and
+ * staging, transposes, softmax and loss rows, the attention backward) is recorded by address: replays
+ * of such a graph must be ordered with the work on the context's stream, and the workspace must be
+ * neither grown (warm it with the largest call first) nor trimmed while the graph is in use. */
 hk_status hk_workspace_size(hk_context* ctx, uint64_t* bytes);
 hk_status hk_trim_workspace(hk_context* ctx, uint64_t keep_bytes);
 /* Thread-local message of the last failure; reference: Display for CannError. */

@@ -268,9 +268,20 @@ hk_status ensure_workspace(Ctx* c, size_t bytes) {
     return HK_OK;
 }
 
-// Workspace of an op that takes `fixed` bytes and then scratch shared by its products: grows to what
-// they want, or, where that cannot be had (the workspace limit, device memory, a capturing stream,
-// on which nothing may be allocated), to what they need. *scratch_bytes: the scratch they may use.
+// Whether work queued on the context's stream goes into a graph (a stream that cannot be asked counts as one).
+bool capturing(const Ctx* c) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // or the next launch wrapper reports it
+    return true;
+}
+
+// Workspace of an op that takes `fixed` bytes and then scratch shared by its products: what they want,
+// or what they need where the rest cannot be had (the workspace limit, device memory) and always on a
+// capturing stream: a graph keeps the workspace's address, and a later call that grows or trims the
+// workspace frees it under the replays, so optional scratch never gets into one. *scratch_bytes is exactly
+// one of the two, whatever the workspace happens to hold: a call's splits, and with them the bits of
+// its result, do not depend on the calls before it.
 hk_status ensure_scratch(Ctx* c, size_t fixed, std::initializer_list<hk::Scratch> products,
                          size_t* scratch_bytes) {
     size_t need = 0, want = 0;
@@ -278,17 +289,13 @@ hk_status ensure_scratch(Ctx* c, size_t fixed, std::initializer_list<hk::Scratch
         need = std::max(need, w.need);
         want = std::max(want, w.want);
     }
-    hk_status st = HK_OK;
-    if (fixed + want > c->ws_bytes) {
-        bool grow = want == need;
-        if (!grow) {
-            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-            grow = hipStreamIsCapturing(c->stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
-        }
-        st = grow ? ensure_workspace(c, fixed + want) : HK_HIP_ERROR;
-        if (st == HK_HIP_ERROR && want > need) st = ensure_workspace(c, fixed + need);
+    bool optional = want > need && !capturing(c);
+    hk_status st = ensure_workspace(c, fixed + (optional ? want : need));
+    if (st == HK_HIP_ERROR && optional) {
+        optional = false;
+        st = ensure_workspace(c, fixed + need);
     }
-    *scratch_bytes = st == HK_OK ? c->ws_bytes - fixed : 0;
+    *scratch_bytes = st != HK_OK ? 0 : (optional ? want : need);
     return st;
 }
 

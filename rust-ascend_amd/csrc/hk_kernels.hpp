@@ -308,8 +308,8 @@ inline int64_t attention_diag(const AttnShape& sh) {
     const uint64_t cap = static_cast<uint64_t>(sh.m + sh.n + 1);
     return -static_cast<int64_t>(d > cap ? cap : d);
 }
-// Scratch that a forward of a few queries wants for splitting its keys over workgroups (0: none); with
-// less it runs with fewer splits.
+// Scratch that a forward of a few queries wants for splitting its keys over workgroups (0: none); without
+// it the keys are not split.
 size_t attention_fwd_workspace_bytes(const AttnShape& sh, int num_cus);
 hipError_t attention_forward(const AttnShape& sh, const void* q, const void* k, const void* v, void* o,
                              float* lse, void* workspace, size_t ws_bytes, int num_cus, hipStream_t s);
