@@ -411,7 +411,9 @@ hk_status hk_silu_mul_backward(hk_context* ctx, const hk_tensor* gate, const hk_
  * operands to BF16, FP32 sums, the gate in F32). x [M,K], gate/up [H,K], down [N,H] F32, every dimension a
  * positive multiple of 16, 16-byte aligned; what the backward reads is written to x_bf16 [M,K],
  * gu_bf16 [2H,K] (gate rows, then up rows), down_bf16 [N,H], gu [M,2H] F32 (gate | up) and act_bf16
- * [M,H]. Operands below 2^30 elements; past that use the separate calls. */
+ * [M,H]. hk_swiglu_bf16_fp32_applies: 1 if the call and its backward take the dimensions (no operand,
+ * its contraction rounded up to 64, past 32-bit byte offsets), else 0: then use the separate calls. */
+int32_t hk_swiglu_bf16_fp32_applies(int64_t m, int64_t k, int64_t h, int64_t n);
 hk_status hk_swiglu_bf16_fp32(hk_context* ctx, const hk_tensor* x, const hk_tensor* gate, const hk_tensor* up,
                               const hk_tensor* down, hk_tensor* y, hk_tensor* x_bf16, hk_tensor* gu_bf16,
                               hk_tensor* down_bf16, hk_tensor* gu, hk_tensor* act_bf16);

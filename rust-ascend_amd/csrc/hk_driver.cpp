@@ -1845,20 +1845,31 @@ hk_status hk_silu_mul(hk_context* h, const hk_tensor* gate, const hk_tensor* up,
 namespace {
 // The FP32 SwiGLU block's tensors: X [M,K], gate/up [H,K], down [N,H] (F32 in the forward, their BF16
 // snapshots in the backward), every dimension a positive multiple of 16, products read in place.
-hk_status swiglu_fp32_dims(int64_t m, int64_t k, int64_t hid, int64_t n) {
+bool swiglu_fp32_aligned(int64_t m, int64_t k, int64_t hid, int64_t n) {
     for (int64_t x : {m, k, hid, n})
-        if (x <= 0 || x % 16 != 0 || x > INT32_MAX)
-            return fail(HK_INVALID_ARGUMENT, "SwiGLU requires aligned X[M,K], gate/up[H,K] and down[N,H]");
-    // the six products: (M, 2H, K), (M, N, H), (M, H, N), (N, H, M), (M, K, 2H), (2H, K, M)
-    if (!hk::gemm_reads_in_place(m, 2 * hid, k) || !hk::gemm_reads_in_place(m, n, hid) || !hk::gemm_reads_in_place(m, hid, n) ||
-        !hk::gemm_reads_in_place(n, hid, m) || !hk::gemm_reads_in_place(m, k, 2 * hid) || !hk::gemm_reads_in_place(2 * hid, k, m))
-        return fail(HK_INVALID_ARGUMENT, "fused SwiGLU operands must stay below 2^30 elements (use the composition)");
+        if (x <= 0 || x % 16 != 0 || x > INT32_MAX) return false;
+    return true;
+}
+// the six products: (M, 2H, K), (M, N, H), (M, H, N), (N, H, M), (M, K, 2H), (2H, K, M)
+bool swiglu_fp32_in_place(int64_t m, int64_t k, int64_t hid, int64_t n) {
+    return hk::gemm_reads_in_place(m, 2 * hid, k) && hk::gemm_reads_in_place(m, n, hid) && hk::gemm_reads_in_place(m, hid, n) &&
+           hk::gemm_reads_in_place(n, hid, m) && hk::gemm_reads_in_place(m, k, 2 * hid) && hk::gemm_reads_in_place(2 * hid, k, m);
+}
+hk_status swiglu_fp32_dims(int64_t m, int64_t k, int64_t hid, int64_t n) {
+    if (!swiglu_fp32_aligned(m, k, hid, n))
+        return fail(HK_INVALID_ARGUMENT, "SwiGLU requires aligned X[M,K], gate/up[H,K] and down[N,H]");
+    if (!swiglu_fp32_in_place(m, k, hid, n))
+        return fail(HK_INVALID_ARGUMENT, "fused SwiGLU operands are past 32-bit offsets (use the composition)");
     return HK_OK;
 }
 bool matrix_of(const hk_tensor* t, int32_t dtype, int64_t rows, int64_t cols) {
     return t && t->dtype == dtype && t->rank == 2 && t->shape[0] == rows && t->shape[1] == cols && aligned16({t->data}) && t->data;
 }
 }  // namespace
+
+int32_t hk_swiglu_bf16_fp32_applies(int64_t m, int64_t k, int64_t h, int64_t n) {
+    return swiglu_fp32_aligned(m, k, h, n) && swiglu_fp32_in_place(m, k, h, n) ? 1 : 0;
+}
 
 hk_status hk_swiglu_bf16_fp32(hk_context* h, const hk_tensor* x, const hk_tensor* gate, const hk_tensor* up,
                               const hk_tensor* down, hk_tensor* y, hk_tensor* x_bf16, hk_tensor* gu_bf16,

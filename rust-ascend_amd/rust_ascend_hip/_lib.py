@@ -124,6 +124,7 @@ SIGNATURES = {
     "hk_cast_into": [_CTX, _T, _T],
     "hk_silu_mul": [_CTX, _T, _T, _T],
     "hk_silu_mul_backward": [_CTX, _T, _T, _T, _T, _T],
+    "hk_swiglu_bf16_fp32_applies": [ctypes.c_int64] * 4,
     "hk_swiglu_bf16_fp32": [_CTX] + [_T] * 10,
     "hk_swiglu_bf16_fp32_backward": [_CTX] + [_T] * 13,
     "hk_bias_add": [_CTX, _T, _T, _T, _T],

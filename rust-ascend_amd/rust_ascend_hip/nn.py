@@ -359,8 +359,7 @@ def swiglu_bf16_fp32(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down
     if any(t.dtype != torch.float32 for t in (x, gate, up, down)):
         raise ValueError("SwiGLU requires FP32 input and weights")
     tensors = [t.contiguous() for t in (x, gate, up, down)]
-    if 2 * h * max(k, m) < 1 << 29 and n * max(h, m) < 1 << 29 and m * k < 1 << 29 and \
-            all(t.data_ptr() % 16 == 0 for t in tensors):
+    if _lib.load().hk_swiglu_bf16_fp32_applies(m, k, h, n) and all(t.data_ptr() % 16 == 0 for t in tensors):
         return _SwigluBf16Fp32.apply(*tensors)
     g = linear_bf16_fp32(x, gate)  # operands past the fused call's 32-bit offsets or off its alignment
     u = linear_bf16_fp32(x, up)

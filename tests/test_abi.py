@@ -367,3 +367,33 @@ def test_integration_extern_blocks_match_the_exports():
     assert declared - exported == set(), declared - exported
     assert exported - declared == set(), exported - declared
     assert exported == set(declared_functions())
+
+
+def test_fused_swiglu_takes_what_the_library_says():
+    """The Python guard of the one-call FP32 SwiGLU is the library's own rule, which counts a contraction
+    rounded up to 64: at K = M = 16 and H = 2^23 the product over gate|up (H doubled) is past 32-bit byte
+    offsets although its 2^28 elements are not, and so is the last row tile of a [16, 2^23] operand."""
+    lib = _lib.load()
+    for dims, want in [((16, 16, 16, 16), 1), ((2000, 2048, 5632, 2048), 1), ((16, 16, (1 << 22) - 64, 16), 1),
+                       ((16, 16, 1 << 23, 16), 0), ((16, 1 << 23, 16, 16), 0), ((16, 16, 16, 1 << 24), 0),
+                       ((1 << 24, 16, 16, 16), 0), ((16, 16, 24, 16), 0), ((0, 16, 16, 16), 0)]:
+        assert lib.hk_swiglu_bf16_fp32_applies(*dims) == want, dims
+
+
+def test_swiglu_past_the_fused_offsets_takes_the_composition(monkeypatch):
+    import torch
+
+    from rust_ascend_hip import nn
+    taken = []
+    monkeypatch.setattr(nn._SwigluBf16Fp32, "apply", staticmethod(lambda *a: taken.append("fused")))
+    monkeypatch.setattr(nn, "linear_bf16_fp32", lambda x, w: taken.append("linear") or torch.empty((x.shape[0], w.shape[0])))
+    monkeypatch.setattr(nn, "silu_mul", lambda g, u: taken.append("silu") or g)
+    wide = 1 << 23
+    for shapes, want in [(((16, 16), (32, 16), (32, 16), (16, 32)), ["fused"]),
+                         (((16, 16), (wide, 16), (wide, 16), (16, wide)), ["linear", "linear", "silu", "linear"])]:
+        x, gate, up, down = (torch.empty(s) for s in shapes)
+        if any(t.data_ptr() % 16 for t in (x, gate, up, down)):
+            pytest.skip("the host allocator returned memory off 16-byte alignment")
+        taken.clear()
+        nn.swiglu_bf16_fp32(x, gate, up, down)
+        assert taken == want
