@@ -69,10 +69,14 @@ gemm_mid_kernel(MidArgs p) {
     static_assert((NS - 2) * kLoads < 64, "vmcnt range");
     __shared__ __attribute__((aligned(1024))) uint16_t ring[NS][kStage];
 
-    // XCD-contiguous ranges of (split, tile), bands of 8 tile rows within a split
+    // XCD-contiguous ranges of (split, tile), bands of 8 tile rows within a split; where the grid is no multiple
+    // of 8, only for the two to eight row tiles of one matrix, which in dispatch order lie on different XCDs
+    // and each read their column tile of the weight into its own L2 (64 x 8112 x 4096 NT, 254 tiles of 32x64:
+    // 36 us, 19 in this order; one row tile, many or a batch lose up to 30% by it: 5 x 704 x 208 x 2032 14, 18).
     const int tiles = p.tiles_m * p.tiles_n, all = tiles * p.splits;
     int bid = blockIdx.x;
     if ((all & 7) == 0) bid = (bid & 7) * (all >> 3) + (bid >> 3);
+    else if (p.tiles_m > 1 && p.tiles_m <= 8 && gridDim.z == 1) bid = xcd_logical();
     const int split = bid / tiles;
     bid -= split * tiles;
     constexpr int GROUP = 8;
