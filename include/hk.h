@@ -153,6 +153,13 @@ hk_status hk_gemm_plan_check(const hk_tensor* a, const hk_tensor* b, int32_t ta,
 hk_status hk_gemm_into(hk_context* ctx, const hk_tensor* a, const hk_tensor* b,
                        int32_t ta, int32_t tb, hk_tensor* out);
 
+/* The kernel that hk_gemm_into runs for 16-byte aligned tensors on a GPU of num_cus compute units with
+ * scratch_bytes of workspace (no context; for tests and tuning): tile + 256 * K splits, the tile (rows x
+ * columns) 0 256x256, 1 256x192, 2 256x128, 3 128x128, 4 128x128 two to a CU, 5 64x128, 6 128x64, 7 64x64,
+ * 8 32x64; -1: operands that are not read in place. */
+int32_t hk_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int32_t ta, int32_t out_dtype,
+                      uint64_t scratch_bytes, int32_t num_cus);
+
 /* Linear backward for Y = X W^T: dX = dY W (BF16), dW = dY^T X (F32).
  * Reference: AscendRuntime::linear_nt_backward, runtime/mod.rs:357-362 (matrix.rs:60-74). */
 hk_status hk_linear_nt_backward(hk_context* ctx, const hk_tensor* x, const hk_tensor* w,

@@ -1367,6 +1367,11 @@ hk_status hk_attention_scores_backward(hk_context* h, const hk_tensor* s, const 
     return complete(g.c, e, "attention_scores_backward", dbias ? 2 : 1);
 }
 
+int32_t hk_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int32_t ta, int32_t out_dtype, uint64_t scratch_bytes,
+                      int32_t num_cus) {
+    return hk::gemm_route(batch, m, n, k, ta, out_dtype == HK_BF16, static_cast<size_t>(scratch_bytes), num_cus);
+}
+
 hk_status hk_linear_nt_backward(hk_context* h, const hk_tensor* x, const hk_tensor* w, const hk_tensor* dy,
                                 hk_tensor* dx, hk_tensor* dw) {
     // Reference: matrix.rs:60-74.

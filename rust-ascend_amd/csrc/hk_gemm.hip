@@ -361,6 +361,17 @@ GemmChoice choose_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_mn
         c.tile = k % kPK == 0 && pick_tile_nj(batch, m, n, num_cus) == 6 ? kT256x192 : kT256;
         return c;
     }
+    // One row tile against a weight past the caches, whose column tiles of 64 alone fill 3/4 of the CUs or more, in one
+    // round: its stream is what counts, and a split only adds its planes and a launch. The estimates tie there, with
+    // errors either way. 64 x 14336 x 4096: 25.6 us unsplit on rotating weights, 20.0 on one, 29.0 and 24.5 with K
+    // in two on 128x128; 32 x 12320 x 11488: 65 and 58 against 72 and 63.
+    const int64_t columns = (n + 63) / 64;
+    if (batch == 1 && m <= 64 && n * k * 2 > 64000000 && 4 * columns >= 3 * num_cus && columns <= num_cus) {
+        GemmChoice c;
+        c.tile = m <= 32 && !a_mn ? kT32x64 : kT64;
+        c.us = tile_time(kTileCost[c.tile], batch, m, n, k, out_bf16, 1, num_cus);
+        return c;
+    }
     return pick_gemm(batch, m, n, k, a_mn, out_bf16, ws_bytes, num_cus);
 }
 
@@ -532,6 +543,15 @@ bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, in
     launch_choice(ch, p, batch, false, ta != 0, tb == 0, nullptr, s);
     *e = hipGetLastError();
     return true;
+}
+
+int gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, bool out_bf16, size_t ws_bytes, int num_cus) {
+    if (!in_place_applies(m, n, k, true)) return -1;
+    const GemmChoice c = choose_gemm(batch, m, n, k, ta != 0, out_bf16, ws_bytes, num_cus);
+    MidArgs p{};
+    p.k = static_cast<int>(k);
+    set_splits(p, c.splits);
+    return c.tile + 256 * p.splits;
 }
 
 bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k) { return in_place_applies(m, n, k, true); }

@@ -117,6 +117,8 @@ bool gemm_bf16_pair(const void* a, const void* b, float* c, float* c2, int64_t b
 bool gemm_bf16_cropped(const void* a, const void* b, float* c, int64_t batch, int64_t m, int64_t n, int64_t k, int ta,
                        int tb, int64_t rows, int64_t cols, size_t ws_bytes, int num_cus, hipStream_t s, hipError_t* e);
 bool gemm_reads_in_place(int64_t m, int64_t n, int64_t k);
+// Tile index + 256 x K splits of the product gemm_bf16 runs for 16-byte aligned tensors; -1: not read in place.
+int gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int ta, bool out_bf16, size_t ws_bytes, int num_cus);
 // M-grouped NT GEMM: C[i, :] = A[i, :] W[g(i)]^T with A [m, k], W [groups, n, k], C [m, n];
 // g(i) = block_group[i / 256] (group ends are multiples of 256). No workspace.
 hipError_t gemm_bf16_grouped_nt(const void* a, const void* w, void* c, int out_bf16, int64_t m, int64_t n,
