@@ -1077,11 +1077,6 @@ attn_decode_combine(DecodeArgs a) {
     if (lane == 0) a.lse[row] = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
 }
 
-// The decode kernel takes the shapes whose query rows per KV head fit its 64 (and D = 64 or 128).
-bool decode_applies(const AttnShape& sh) {
-    return (sh.d == 64 || sh.d == 128) && sh.heads / sh.kv_heads * sh.m <= kDecodeMaxRows;
-}
-
 // 32-key tiles up to the last key that some query sees.
 int decode_tiles(const AttnShape& sh) {
     int64_t keys = sh.n;
@@ -1090,6 +1085,25 @@ int decode_tiles(const AttnShape& sh) {
         keys = seen < 0 ? 0 : (seen < keys ? seen : keys);
     }
     return static_cast<int>((keys + 31) / 32);
+}
+
+// The decode kernel takes the shapes whose query rows per KV head fit its 64 (and D = 64 or 128). Up to 32
+// rows it is the faster kernel at every length. With 33 to 64 (four row blocks: the merge and the registers of
+// 64 rows cost each workgroup 4 us) it pays where it reads K and V less often, that is where a workgroup per
+// query head takes more rounds of the CUs than one per KV head, or where the keys are many. Kernel us, ping-pong
+// against decode, 64 rows of one head, by B x H and keys:
+//   D 128   32: n 64 8.5 13.5, n 384 16.2 18.3, n 512 19.6 19.1, n 1024 31 22;   256: n 512 21.8 24.6, n 768 28.1 29.3, n 1024 37 34
+//           1024: n 64 30 48, n 512 86 98, n 768 118 123, n 1024 148 145
+//   D 64    32: n 64 6.7 8.1, n 128 8.1 8.6, n 256 10.6 9.9;   1024: n 64 21 26, n 256 37 40, n 384 47 49, n 512 58 57
+//   32 rows, D 128, 1024: n 64 29.5 18;   two heads of 32 rows, 512 KV heads: n 64 28 25, n 512 78 47
+bool decode_applies(const AttnShape& sh, int num_cus) {
+    const int64_t rows = sh.heads / sh.kv_heads * sh.m;
+    if ((sh.d != 64 && sh.d != 128) || rows > kDecodeMaxRows) return false;
+    if (rows <= 32) return true;
+    const int64_t q_rounds = (sh.batch * sh.heads + num_cus - 1) / num_cus;
+    const int64_t kv_rounds = (sh.batch * sh.kv_heads + num_cus - 1) / num_cus;
+    const int one_round = sh.d == 64 ? 192 : 512;
+    return q_rounds > kv_rounds || 32 * decode_tiles(sh) > (q_rounds == 1 ? one_round : (sh.d == 64 ? 384 : 768));
 }
 
 size_t decode_split_bytes(const AttnShape& sh, int splits) {
@@ -1149,7 +1163,7 @@ hipError_t launch_fwd(const AttnShape& sh, const void* q, const void* k, const v
     a.scale_log2 = sh.scale * kLog2e;
     a.causal = sh.causal;
     if constexpr (D >= 64) {
-        if (decode_applies(sh)) {
+        if (decode_applies(sh, num_cus)) {
             a.tiles = decode_tiles(sh);
             a.splits = decode_splits(sh, ws_bytes, num_cus);
             a.split_tiles = (a.tiles + a.splits - 1) / a.splits;
@@ -2224,7 +2238,7 @@ size_t attention_bwd_workspace_bytes(const AttnShape& sh) {
 }
 
 size_t attention_fwd_workspace_bytes(const AttnShape& sh, int num_cus) {
-    return decode_applies(sh) ? decode_split_bytes(sh, decode_splits(sh, SIZE_MAX, num_cus)) : 0;
+    return decode_applies(sh, num_cus) ? decode_split_bytes(sh, decode_splits(sh, SIZE_MAX, num_cus)) : 0;
 }
 
 hipError_t attention_forward(const AttnShape& sh, const void* q, const void* k, const void* v, void* o, float* lse,

@@ -54,6 +54,21 @@ def test_decode_attention(b, hq, hkv, m, n, d):
         check(o, lse, q, k, v, d ** -0.5, causal, qs, ks)
 
 
+# 33 to 64 query rows on either side of the line between the two kernels, told apart by the workspace: the
+# split decode keeps its partials there, the ping-pong kernel takes none
+@pytest.mark.parametrize("hq,hkv,m,n,d,decodes", [(4, 4, 64, 512, 128, False), (4, 4, 64, 520, 128, True), (4, 4, 33, 192, 64, False),
+                                                  (4, 4, 33, 200, 64, None), (8, 4, 24, 384, 128, False), (4, 4, 32, 512, 128, True),
+                                                  (4, 4, 64, 2048, 64, True), (8, 4, 32, 2000, 128, True)])
+def test_rows_where_the_query_kernel_is_faster(hq, hkv, m, n, d, decodes):
+    q, k, v = inputs(2, hq, hkv, m, n, d)
+    HipRuntime.trim_workspace()
+    print(f"rows {hq}/{hkv} m{m} n{n} d{d}", flush=True)
+    o, lse = HipRuntime.attention_forward(q, k, v, d ** -0.5, True, n - m, 0)
+    if decodes is not None:
+        assert (HipRuntime.workspace_size() > 0) == decodes
+    check(o, lse, q, k, v, d ** -0.5, True, n - m, 0)
+
+
 def test_decode_attention_f32_surface_and_negative_scale():
     q, k, v = (t.float() for t in inputs(2, 8, 2, 1, 700, 128))
     o, lse = HipRuntime.attention_forward(q, k, v, -0.1, True, 699, 0, out_dtype=torch.float32)
