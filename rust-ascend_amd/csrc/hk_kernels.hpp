@@ -220,8 +220,8 @@ hipError_t softmax_backward(const float* y, const float* dy, float* dx, int64_t 
 
 // Cross entropy's passes over the logits (hk_softmax.hip). y = log_softmax(x) with each row's NLL term
 // -weight[t] y[t] and counted weight (weight null: 1), and the gradient of the summed terms through
-// the log-softmax from its output. The forward applies to 16-byte aligned x and y of widths up to
-// 65536; out (null, or [rows]) receives the terms themselves.
+// the log-softmax from its output. The forward applies to 16-byte aligned x and y of widths from 257 (a
+// multiple of 4: 772) to 65536; out (null, or [rows]) receives the terms themselves.
 bool log_softmax_nll_applies(int64_t width, const float* x, const float* y);
 hipError_t log_softmax_nll(const float* x, float* y, int64_t rows, int64_t width, const void* target, int id_bytes,
                            const float* weight, int64_t ignore, float* row_v, float* row_w, float* out, hipStream_t s);

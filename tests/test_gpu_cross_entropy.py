@@ -82,3 +82,24 @@ def test_unaligned_logits_and_bad_labels():
         nn.cross_entropy(x, t)
     with pytest.raises(HkError):
         nn.cross_entropy(x[0:1], t)
+
+
+# the last widths of the two passes and the first of the one, on either row alignment
+@pytest.mark.parametrize("classes,two_passes", [(3, True), (100, True), (255, True), (256, True), (257, False), (300, True),
+                                                (768, True), (769, False), (772, False)])
+def test_narrow_rows_take_the_faster_passes(classes, two_passes):
+    """Rows too narrow for the one-pass kernel run the log-softmax and the NLL one after the other: the bits of
+    that composition (the widths past the line agree with it as above)."""
+    x, t, w = inputs(67, classes)
+    a, b = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    fused, want = nn.weighted_cross_entropy(a, t, w), composed(b, t, w, LossReduction.Mean, None)
+    _, y, _ = HipRuntime.cross_entropy(x, t, w)
+    logp = nn.log_softmax(x)
+    if two_passes:
+        assert torch.equal(y, logp) and torch.equal(fused, want)
+    assert bool(((y - logp).abs() <= 2 ** -20 * logp.abs().max()).all())
+    assert abs((fused - want).item()) <= 2 ** -20 * abs(want.item())
+    (da,), (db,) = torch.autograd.grad(fused, [a]), torch.autograd.grad(want, [b])
+    assert ((da - db).norm() / db.norm()).item() <= 2 ** -20
+    x64 = torch.log_softmax(x.double(), -1)
+    assert ((logp.double() - x64).norm() / x64.norm()).item() <= 1e-6
