@@ -23,6 +23,8 @@
 #include "hk_common.hpp"
 #include "hk_kernels.hpp"
 
+#include <type_traits>
+
 namespace hk {
 
 namespace {
@@ -31,7 +33,8 @@ constexpr int kRowsPerWg = 16;
 constexpr int kMaxBlocks = 9;   // 32-key blocks a wave holds: 72 registers of scores, of dP and of operands each
 constexpr int kChunk = 128;     // output columns summed over the waves at a time
 constexpr int kPastEnd = 0x7ffffff0;  // a byte offset past every buffer: loads of it return 0
-constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = 1.925963033500e-8f;  // log2(e) = their sum
+constexpr float kLn2 = 0.6931471805599453f;
 
 struct MaskedArgs {
     const uint16_t* q;     // [groups][rows][d]
@@ -140,6 +143,17 @@ __device__ __forceinline__ int bf16_slot(int row, int c) { return (row * 4 + (c 
 
 constexpr int kBatch = 4;  // blocks in a wave's LDS at a time
 
+// e^x for x <= 0 within an ulp or two: 2^t of the rounded product t = x log2(e), whose rounding (up to |t| / 2 ulps of
+// the result: 2e-6 of it at x = -60) is taken back in first order. Where t is -inf (x as well, or near the type's lowest
+// value) the remainder is a NaN or infinite, which the median bounds, and r is 0; x = NaN makes r one. For dMask, the
+// one result that holds the weights in F32; where they only go on in BF16 (2^-9) the plain power is the same.
+__device__ __forceinline__ float exp_f32(float x) {
+    const float t = x * kLog2e;
+    const float rest = __builtin_amdgcn_fmed3f(fmaf(x, kLog2eLow, fmaf(x, kLog2e, -t)), -1.0f, 1.0f);
+    const float r = __builtin_amdgcn_exp2f(t);
+    return fmaf(r * rest, kLn2, r);
+}
+
 // f[b]: rows lane / 8 (+ 8) in memory order -> query r, keys 8 g + 4 t
 template <int MAXB>
 __device__ __forceinline__ void rows_to_queries(Pairs<MAXB>& f, uint32_t* lds, int lane) {
@@ -237,17 +251,23 @@ masked_attention(MaskedArgs a) {
 
     f32x4_t dp[BWD ? MAXB : 1][2];
     if constexpr (BWD) scores<MAXB>(dv, dp, d0, f, [&](int b, int t) { return f[b][t]; });  // no registers for K^T yet
+    // The sums join a tile's four terms before the running sum: with one term at a time its rounding (72 terms a
+    // lane) showed in every weight of the row, dMask 1-4% further from float64 than by the row kernels.
     float sum = 0.0f, dot = 0.0f;
+    auto weigh = [&](auto exact) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < MAXB; ++b)
+        for (int b = 0; b < MAXB; ++b)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < 2; ++t) {
+                f32x4_t& w = s[b][t];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                s[b][t][e] = __builtin_amdgcn_exp2f((s[b][t][e] - m) * kLog2e);
-                sum += s[b][t][e];
-                if constexpr (BWD) dot += s[b][t][e] * dp[b][t][e];
+                for (int e = 0; e < 4; ++e) w[e] = decltype(exact)::value ? exp_f32(w[e] - m) : __builtin_amdgcn_exp2f((w[e] - m) * kLog2e);
+                sum += (w[0] + w[1]) + (w[2] + w[3]);
+                if constexpr (BWD) dot += (w[0] * dp[b][t][0] + w[1] * dp[b][t][1]) + (w[2] * dp[b][t][2] + w[3] * dp[b][t][3]);
             }
+    };
+    if (BWD && a.dmask != nullptr) weigh(std::true_type{});
+    else weigh(std::false_type{});
     const float inv = 1.0f / over_waves<false, W>(sum, stat[1], wave, lane);
     if constexpr (BWD) dot = over_waves<false, W>(dot, stat[2], wave, lane) * inv;
 

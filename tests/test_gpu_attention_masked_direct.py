@@ -63,3 +63,26 @@ def test_extreme_values():
     assert rel(o[ok], want[ok]) <= 2 ** -7
     dq, dk, dv, dmask = HipRuntime.attention_masked_backward(q, k, v, mask, dy, 0.2, mask_grad=True)
     assert torch.equal(torch.isnan(dq).any(-1), nan_rows) and torch.equal(torch.isnan(dmask).any(-1), nan_rows)
+
+
+def test_small_probabilities_keep_f32_accuracy():
+    """dMask of keys far below the row's maximum, element by element. The scores are 0 and the maximum is 0, so the
+    exponents are the mask's values, exactly; dP is small whole numbers, exact too. What is left is the
+    exponential (1.5 ulp), the row's sum and reciprocal, dP - rowsum(P dP) (at least 1 here, values up to 8) and
+    two products: 8 roundings of 2^-24, 5e-7 of each element. An exponent rounded once more, at 2^-24 of up
+    to 115, would be off by 2e-6."""
+    m, n, d = 32, 96, 16
+    q = torch.zeros((1, 2, m, d), device=DEV)
+    k, v = (torch.zeros((1, 1, n, d), device=DEV) for _ in range(2))
+    dy = torch.zeros((1, 2, m, d), device=DEV)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(2)
+    dy[..., 0] = 1.0
+    v[..., 0] = torch.randint(2, 7, (n,), generator=g, device=DEV).float()
+    v[0, 0, 0, 0] = 0.0  # the one heavy key: rowsum(P dP) stays near 0
+    mask = -80 + 60 * torch.rand((1, 2, m, n), generator=g, device=DEV)
+    mask[..., 0] = 0.0
+    got = HipRuntime.attention_masked_backward(q, k, v, mask, dy, 1.0, mask_grad=True)[3].double()
+    want = reference(q, k, v, dy, mask, 1.0)[4]
+    far = ((got - want).abs() / want.abs())[..., 1:]
+    assert far.max().item() <= 5e-7
