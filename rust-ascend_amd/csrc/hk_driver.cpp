@@ -2894,6 +2894,11 @@ hk_status attention_backward_common(hk_context* h, const hk_tensor* q, const hk_
     hk::attention_bwd_plan(sh, g.c->num_cus);
     size_t stat_bytes = ws_round(hk::attention_bwd_workspace_bytes(sh));
     st = ensure_workspace(g.c, stat_bytes + staging);
+    if (st == HK_HIP_ERROR && sh.dkv_splits > 4) {  // half the partial sums before the slower form
+        sh.dkv_splits = 4;
+        stat_bytes = ws_round(hk::attention_bwd_workspace_bytes(sh));
+        st = ensure_workspace(g.c, stat_bytes + staging);
+    }
     if (st == HK_HIP_ERROR && (sh.store_ds || sh.dkv_splits > 1)) {
         // the stored-dS buffer or the split's partial sums do not fit in free device memory (or
         // the workspace limit): the recompute form of dQ, unsplit, needs only the row statistics

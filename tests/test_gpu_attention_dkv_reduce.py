@@ -54,3 +54,24 @@ def test_rows_output_bit_exact_with_merge(shape, layout, splits, monkeypatch):
     rows = HipRuntime.attention_backward_qkv_rows(*args, cos, sin, d ** -0.5, True, layout=RotaryLayout(layout))
     dq, dk, dv = HipRuntime.attention_backward(*args, d ** -0.5, True, grad_dtype=torch.bfloat16)
     assert torch.equal(rows, HipRuntime.qkv_rope_merge(dq, dk, dv, cos, sin, RotaryLayout(layout)))
+
+
+def test_eight_splits_past_the_workspace_limit_become_four(monkeypatch):
+    """A limit that holds the partial sums of four splits but not of eight: four, with the stored dS, not the
+    unsplit recompute form."""
+    shape = SHAPES[0]
+    d = shape[-1]
+    args = inputs(*shape)
+
+    def run(splits=None, limit=None):
+        for name, value in (("HK_ATTN_DKV_SPLITS", splits), ("HK_WORKSPACE_LIMIT", limit)):
+            monkeypatch.delenv(name, raising=False) if value is None else monkeypatch.setenv(name, str(value))
+        HipRuntime.trim_workspace()
+        return HipRuntime.attention_backward(*args, d ** -0.5, True, grad_dtype=torch.float32), HipRuntime.workspace_size()
+    _, eight = run()
+    four, limit = run(splits=4)
+    assert limit < eight
+    got, held = run(limit=limit)
+    assert held == limit
+    for a, b in zip(got, four):
+        assert torch.equal(a, b)
