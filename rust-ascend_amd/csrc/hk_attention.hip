@@ -2125,11 +2125,11 @@ size_t stat_bytes(const AttnShape& sh) {  // row statistic and lse2, rounded to 
 //   B2 Hq8 Hkv8 1747 D64     ratio 2.13    83  74  88 114      B2 Hq32 Hkv8 1024 D128   ratio 3.56   211 142 129 162
 //   B1 Hq32 Hkv8 3000 D128   ratio 2.61   573 369 371 409      B2 Hq8 Hkv2 1900 D128    ratio 8.0    352 206 138 141
 //   B1 Hq16 Hkv4 2048 D128   ratio 7.53   375 219 141 146      B4 Hq8 Hkv2 512 D128     ratio 12.8   108  74  56  46
-// The environment variable HK_ATTN_DKV_SPLITS (1, 2 or 4) overrides the choice.
+// The environment variable HK_ATTN_DKV_SPLITS (1, 2, 4 or 8) overrides the choice.
 int dkv_splits_for(const AttnShape& sh, int num_cus) {
     if (const char* env = std::getenv("HK_ATTN_DKV_SPLITS")) {
         const int v = std::atoi(env);
-        if (v == 1 || v == 2 || v == 4) return v;
+        if (v == 1 || v == 2 || v == 4 || v == 8) return v;
     }
     const int64_t blocks = (sh.n + kKBlock - 1) / kKBlock, qsteps = (sh.m + kQStep - 1) / kQStep;
     const int64_t group = sh.heads / sh.kv_heads, diag = attention_diag(sh);

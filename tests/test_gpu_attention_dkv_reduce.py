@@ -75,3 +75,23 @@ def test_eight_splits_past_the_workspace_limit_become_four(monkeypatch):
     assert held == limit
     for a, b in zip(got, four):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(2, 4, 4, 300, 64)], ids=lambda s: "x".join(map(str, s)))
+def test_eight_splits_forced(shape, monkeypatch):
+    """HK_ATTN_DKV_SPLITS=8: the choice of the small grids, and five query steps over eight splits (empty shares)."""
+    d = shape[-1]
+    args = inputs(*shape)
+    monkeypatch.delenv("HK_ATTN_DKV_SPLITS", raising=False)
+    own = HipRuntime.attention_backward(*args, d ** -0.5, True, grad_dtype=torch.float32)
+    held = {}
+    for splits in ("4", "8"):
+        monkeypatch.setenv("HK_ATTN_DKV_SPLITS", splits)
+        HipRuntime.trim_workspace()
+        got = HipRuntime.attention_backward(*args, d ** -0.5, True, grad_dtype=torch.float32)
+        held[splits] = HipRuntime.workspace_size()
+    assert held["8"] > held["4"]
+    for a, b in zip(got, own):
+        err = (a - b).reshape(-1, d).norm(dim=1) / b.reshape(-1, d).norm(dim=1).clamp_min(1e-30)
+        assert float(err.max()) <= 1e-5
+        assert shape not in SHAPES or torch.equal(a, b)
