@@ -159,6 +159,13 @@ hk_status hk_gemm_into(hk_context* ctx, const hk_tensor* a, const hk_tensor* b,
  * 8 32x64; -1: operands that are not read in place. */
 int32_t hk_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int32_t ta, int32_t out_dtype,
                       uint64_t scratch_bytes, int32_t num_cus);
+/* The same for a fused-epilogue product of m x n outputs (qkv_rope 1: hk_qkv_projection_rope, 0: the others,
+ * n = 2 F for hk_swiglu_projection): the tile index, -1 if it does not apply. */
+int32_t hk_epilogue_route(int64_t m, int64_t n, int64_t k, int32_t qkv_rope, int32_t num_cus);
+/* The same for hk_tensor_matmul (which 0) and its gradients dA (1) and dB (2) in F32: the tile's edge, 64 or
+ * 128, + 1024 * K splits; -1: gathered operands (F16 and BF16, and F32 past 32-bit offsets). */
+int32_t hk_tensor_matmul_route(const hk_tensor* a, const hk_tensor* b, int32_t which, uint64_t scratch_bytes,
+                               int32_t num_cus);
 
 /* Linear backward for Y = X W^T: dX = dY W (BF16), dW = dY^T X (F32).
  * Reference: AscendRuntime::linear_nt_backward, runtime/mod.rs:357-362 (matrix.rs:60-74). */

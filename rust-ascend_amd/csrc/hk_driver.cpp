@@ -1204,6 +1204,13 @@ hk_status hk_matmul_layout(const hk_tensor* a, const hk_tensor* b, hk_tensor* ou
     return HK_OK;
 }
 
+int32_t hk_tensor_matmul_route(const hk_tensor* a, const hk_tensor* b, int32_t which, uint64_t scratch_bytes, int32_t num_cus) {
+    hk::MatmulSpec s;
+    hk_tensor layout{};
+    if (which < 0 || which > 2 || matmul_spec(a, b, &s, &layout) != HK_OK) return -1;
+    return hk::matmul_f32_route(s, which, static_cast<size_t>(scratch_bytes), num_cus);
+}
+
 hk_status hk_tensor_matmul(hk_context* h, const hk_tensor* a, const hk_tensor* b, hk_tensor* out) {
     // Reference: AscendRuntime::tensor_matmul (runtime/mod.rs:156-158) -> generic_matrix::matmul
     // (generic_matrix.rs:17-54) -> AscendState::tensor_matmul (worker.rs:128-162): KEEP_DTYPE.
@@ -1370,6 +1377,10 @@ hk_status hk_attention_scores_backward(hk_context* h, const hk_tensor* s, const 
 int32_t hk_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int32_t ta, int32_t out_dtype, uint64_t scratch_bytes,
                       int32_t num_cus) {
     return hk::gemm_route(batch, m, n, k, ta, out_dtype == HK_BF16, static_cast<size_t>(scratch_bytes), num_cus);
+}
+
+int32_t hk_epilogue_route(int64_t m, int64_t n, int64_t k, int32_t qkv_rope, int32_t num_cus) {
+    return hk::epilogue_route(m, n, k, qkv_rope != 0, num_cus);
 }
 
 hk_status hk_linear_nt_backward(hk_context* h, const hk_tensor* x, const hk_tensor* w, const hk_tensor* dy,

@@ -584,6 +584,12 @@ int pick_epi_tile(int64_t m, int64_t n, int64_t k, std::initializer_list<int> bu
     return best;
 }
 
+template <int EPI>
+int epi_tile(int64_t m, int64_t n, int64_t k, int num_cus) {
+    if constexpr (EPI == kEpiQkvRope) return pick_epi_tile(m, n, k, {kT128Pair, kT64x128}, num_cus);
+    else return pick_epi_tile(m, n, k, {kT256x128, kT128Pair, kT64x128, kT64}, num_cus);
+}
+
 template <int WM, int WN, int NI, int NJ, int NS, int PER_CU, int EPI, bool B_MN>
 void launch_epi_mid(const GemmEpiArgs& a, hipStream_t s) {
     MidArgs p{};
@@ -601,13 +607,13 @@ void launch_epi_mid(const GemmEpiArgs& a, hipStream_t s) {
 template <int EPI, bool B_MN>
 hipError_t launch_epi(GemmEpiArgs p, int num_cus, hipStream_t s) {
     if constexpr (EPI == kEpiQkvRope) {
-        switch (pick_epi_tile(p.m, p.n, p.k, {kT128Pair, kT64x128}, num_cus)) {
+        switch (epi_tile<EPI>(p.m, p.n, p.k, num_cus)) {
             case kT128Pair: launch_epi_mid<4, 1, 2, 8, 2, 2, EPI, B_MN>(p, s); return hipGetLastError();
             case kT64x128: launch_epi_mid<4, 1, 1, 8, 3, 2, EPI, B_MN>(p, s); return hipGetLastError();
             default: break;
         }
     } else {
-        switch (pick_epi_tile(p.m, p.n, p.k, {kT256x128, kT128Pair, kT64x128, kT64}, num_cus)) {
+        switch (epi_tile<EPI>(p.m, p.n, p.k, num_cus)) {
             case kT256x128: launch_epi_mid<2, 2, 8, 4, 3, 1, EPI, B_MN>(p, s); return hipGetLastError();
             case kT128Pair: launch_epi_mid<2, 2, 4, 4, 2, 2, EPI, B_MN>(p, s); return hipGetLastError();
             case kT64x128: launch_epi_mid<2, 2, 2, 4, 3, 2, EPI, B_MN>(p, s); return hipGetLastError();
@@ -635,6 +641,11 @@ GemmEpiArgs epi_args(const void* a, const void* b, void* c, int64_t m, int64_t n
     return p;
 }
 }  // namespace
+
+int epilogue_route(int64_t m, int64_t n, int64_t k, bool qkv_rope, int num_cus) {
+    if (!epi_applies(m, n, k)) return -1;
+    return qkv_rope ? epi_tile<kEpiQkvRope>(m, n, k, num_cus) : epi_tile<kEpiResidual>(m, n, k, num_cus);
+}
 
 hipError_t gemm_qkv_rope(const void* x, const void* w, int64_t tokens, int64_t hidden, int64_t seq, int64_t hq,
                          int64_t hkv, const float* cos_t, const float* sin_t, int layout, void* q, void* k, void* v,

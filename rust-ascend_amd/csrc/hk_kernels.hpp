@@ -76,6 +76,8 @@ struct MatmulSpec {
     MatmulBatch batch, a_batch, b_batch;  // output batch shape; A's and B's strides over it
 };
 Scratch matmul_workspace(const MatmulSpec& s, int num_cus);
+// Tile edge (64 or 128) + 1024 x K splits of an F32 product read in place (which: 0 the product, 1 dA, 2 dB); -1: gathered.
+int matmul_f32_route(const MatmulSpec& s, int which, size_t ws_bytes, int num_cus);
 hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, size_t ws_bytes,
                   int num_cus, hipStream_t st);
 // Module attention's score transform (hk_attention_module.hip) over F32 scores [B, H, Sq, Sk]:
@@ -134,6 +136,8 @@ hipError_t gemm_qkv_rope(const void* x, const void* w, int64_t tokens, int64_t h
 // The other fused-epilogue GEMMs of a decoder layer (BF16, any M and N; they apply
 // when K % 8 == 0 and M K, N K stay below 2^30 elements, K rounded up to 64):
 bool epi_applies(int64_t m, int64_t n, int64_t k);
+// Tile index (gemm_route) of a fused-epilogue product of m x n outputs; -1: it does not apply.
+int epilogue_route(int64_t m, int64_t n, int64_t k, bool qkv_rope, int num_cus);
 // y [m, n] = res + x [m, k] W [n, k]^T (the product rounded to BF16 before the add)
 hipError_t gemm_residual(const void* x, const void* w, const void* res, void* y, int64_t m, int64_t n, int64_t k,
                          int num_cus, hipStream_t s);

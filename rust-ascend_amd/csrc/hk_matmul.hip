@@ -735,6 +735,17 @@ Scratch matmul_backward_workspace(const MatmulSpec& s, int num_cus) {
     return {bytes, bytes};
 }
 
+int matmul_f32_route(const MatmulSpec& s, int which, size_t ws_bytes, int num_cus) {
+    if (s.dtype != 0 || s.batch.count * s.m * s.n * s.k == 0) return -1;
+    const F32Product xa = f32_grad_a(s, nullptr, nullptr), xb = f32_grad_b(s, nullptr, nullptr);
+    const F32Product x = which == 0 ? f32_forward(s, nullptr, nullptr) : (which == 1 ? xa : xb);
+    if (which == 0 ? !f32_fits(x) : !f32_fits(xa) || !f32_fits(xb)) return -1;
+    const size_t slices = which == 0 ? 0 : f32_slice_bytes(x, operand_shape(s.batch, which == 1 ? s.a_batch : s.b_batch));
+    const F32Choice c = f32_choose(x, num_cus, ws_bytes > slices ? ws_bytes - slices : 0);
+    const int64_t steps = (x.k + kFK - 1) / kFK, per = (steps + c.splits - 1) / c.splits;
+    return (c.big ? 128 : 64) + 1024 * static_cast<int>((steps + per - 1) / per);
+}
+
 hipError_t matmul(const MatmulSpec& s, const void* a, const void* b, void* out, void* workspace, size_t ws_bytes,
                   int num_cus, hipStream_t st) {
     const int64_t G = s.batch.count;

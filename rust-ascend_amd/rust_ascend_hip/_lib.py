@@ -111,6 +111,8 @@ SIGNATURES = {
     "hk_gemm_grouped_plan_check": [_T, _T, ctypes.POINTER(_i32), _i32, _i32, ctypes.POINTER(HkGemmPlan)],
     "hk_gemm_grouped_nt_into": [_CTX, _T, _T, ctypes.c_void_p, _T],
     "hk_gemm_route": [ctypes.c_int64] * 4 + [_i32, _i32, _u64, _i32],
+    "hk_epilogue_route": [ctypes.c_int64] * 3 + [_i32, _i32],
+    "hk_tensor_matmul_route": [_T, _T, _i32, _u64, _i32],
     "hk_linear_nt_backward": [_CTX, _T, _T, _T, _T, _T],
     "hk_gemm_bf16_fp32": [_CTX, _T, _T, _i32, _i32, _T, _T, _T],
     "hk_gemm_bf16_fp32_backward": [_CTX, _T, _T, _T, _i32, _i32, _T, _T],

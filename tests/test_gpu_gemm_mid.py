@@ -1,5 +1,6 @@
-"""GPU parity of the GEMMs that 256x256 tiles cannot fill: every tile shape from 256x128 to 32x64, K
-split over workgroups or not, every transpose read in place, at edges of tiles and of K stages.
+"""GPU parity of the GEMMs that 256x256 tiles cannot fill, over small and ragged shapes: K split over
+workgroups or not, every transpose read in place, at edges of tiles and of K stages (each tile shape in each
+of its forms: test_gpu_gemm_tiles.py).
 
 Against float64 products of the same BF16 values. F32 outputs: a sum of K products rounded to F32 at
 each of K steps in the worst order has a relative 2-norm error of at most about sqrt(K) 2^-24 against
@@ -15,7 +16,7 @@ from rust_ascend_hip import HipRuntime, runtime
 
 pytestmark = pytest.mark.gpu
 
-# batch, M, N, K: one row tile and skinny weights (32x64 tiles, split K), tails of every tile shape,
+# batch, M, N, K: one row tile and skinny weights (32x64 tiles, split K), tails of several tile shapes,
 # a K tail (K % 64 != 0), K of one stage, many small batches, grids around one tile per CU
 SHAPES = [(1, 16, 64, 16), (1, 16, 4096, 2048), (1, 48, 1056, 7312), (1, 144, 272, 336), (1, 272, 400, 1040),
           (1, 512, 2048, 704), (1, 784, 2288, 592), (1, 848, 1264, 3952), (1, 1120, 5360, 1152), (1, 2000, 2048, 80),

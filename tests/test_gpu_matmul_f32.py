@@ -45,7 +45,8 @@ def check(a, b):
         assert rel(got, ref) <= 4 * terms ** 0.5 * 2 ** -24
 
 
-# edges of 64 and 128 tiles and of a 16-step, one element, odd strides, split K, full grids of each tile
+# edges of tiles and of a 16-step, one element, odd strides, split K (all of these on 64x64 tiles; the 128x128
+# ones are in test_gpu_gemm_tiles.py)
 @pytest.mark.parametrize("a,b", [((1, 1), (1, 1)), ((3, 5), (5, 7)), ((64, 16), (16, 64)), ((65, 17), (17, 129)), ((130, 1001), (1001, 67)), ((130, 1001), (1001, 68)), ((130, 1004), (1004, 67)),
                                  ((31, 4097), (4097, 33)), ((2050, 70), (70, 1999)), ((1100, 64), (64, 4099)),
                                  ((4, 77, 130), (130, 95)), ((3, 2, 40, 33), (33, 20)), ((6, 50, 64), (6, 64, 70)),

@@ -1,6 +1,6 @@
 """GPU parity: padded linear products whose GEMM stores only the logical rows and columns, at every
-remainder of the columns modulo 4, on the small, the split, the ragged and the 256x256 tiles, with K off its
-stages; and row padding of odd lengths. Against float64 on the BF16-rounded operands: F32 accumulation
+remainder of the columns modulo 4, on 32x64 and 64x64 tiles, split, and on the 256x256 tiles (the tiles
+between: test_gpu_gemm_tiles.py), with K off its stages; and row padding of odd lengths. Against float64 on the BF16-rounded operands: F32 accumulation
 over K terms, so 1e-5 of the norm; nothing outside the logical output is written."""
 import pytest
 import torch
