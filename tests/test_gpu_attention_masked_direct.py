@@ -4,7 +4,7 @@ widths (a half column step, more than one chunk of output columns, an odd tile, 
 the next), with BF16 operands and results, and off 16-byte alignment, against float64.
 
 P, dS and the operands are BF16 in the products: relative 2-norm errors below 2^-7, as for the row passes;
-a BF16 result adds its own rounding of 2^-9, inside the same bound."""
+a BF16 result adds its own rounding of 2^-9, inside the same bound. dMask is F32 throughout: 1e-5, as there."""
 import pytest
 import torch
 
@@ -27,7 +27,7 @@ def test_edges(n, d, dv, mask_grad):
     got = (o,) + tuple(HipRuntime.attention_masked_backward(q, k, v, mask, dy, d ** -0.5, mask_grad=mask_grad))
     for name, a, b in zip(NAMES, got, reference(q, k, v, dy, mask, d ** -0.5)):
         if a is not None:
-            assert rel(a, b) <= 2 ** -7, name
+            assert rel(a, b) <= (1e-5 if name == "dmask" else 2 ** -7), name
 
 
 @pytest.mark.parametrize("shift", [0, 1])

@@ -2,7 +2,9 @@
 rounding in one kernel each up to 4096 keys, one kernel per step above) against float64.
 
 P, dS and the operands are BF16 in the GEMMs: relative 2-norm errors below 2^-7 (two or three roundings of
-2^-9 each). dMask is dS in F32 from a BF16-operand dP: the same bound."""
+2^-9 each). dMask is dS in F32 and both sides round its operands alike: what is left is F32 arithmetic, of
+which an exponent of up to 16 matters most (its 2^-24 a dozen times over, in the scores' sum, the scale and
+mask, the maximum and the exponential): 1e-5."""
 import pytest
 import torch
 
@@ -50,7 +52,7 @@ def test_masked_rows(n, with_mask, mask_grad):
     got = (o,) + tuple(HipRuntime.attention_masked_backward(q, k, v, mask, dy, 0.2, mask_grad=mask_grad))
     for name, a, b in zip(("o", "dq", "dk", "dv", "dmask"), got, reference(q, k, v, dy, mask, 0.2)):
         if a is not None:
-            assert rel(a, b) <= 2 ** -7, name
+            assert rel(a, b) <= (1e-5 if name == "dmask" else 2 ** -7), name
 
 
 @pytest.mark.parametrize("n", [64, 4128])
