@@ -20,7 +20,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -3031,7 +3030,9 @@ struct Carve {
 
 // Workspace for a plan(carve, error, context or null, CUs): what it takes with the scratch its
 // products want, else (no memory, the limit, a capturing stream) with what they need (*lean set).
-hk_status ensure_planned(Ctx* c, const std::function<void(Carve&, hipError_t*, Ctx*, int)>& plan, bool* lean) {
+extern "C++" {
+template <class Plan>
+hk_status ensure_planned(Ctx* c, const Plan& plan, bool* lean) {
     hipError_t e = hipSuccess;
     size_t bytes[2];
     for (int i = 0; i < 2; ++i) {
@@ -3045,6 +3046,7 @@ hk_status ensure_planned(Ctx* c, const std::function<void(Carve&, hipError_t*, C
     *lean = granted < bytes[0];
     return st;
 }
+}  // extern "C++" (a template)
 
 // BF16 operands: a tensor itself when BF16, else its RNE rounding into the workspace (one launch for all).
 struct Operands {
