@@ -1088,14 +1088,15 @@ int decode_tiles(const AttnShape& sh) {
 }
 
 // The decode kernel takes the shapes whose query rows per KV head fit its 64 (and D = 64 or 128). Up to 32
-// rows it is the faster kernel at every length. With 33 to 64 (four row blocks: the merge and the registers of
+// rows it is the faster kernel, or level with the other, at every length. With 33 to 64 (four row blocks: the merge and the registers of
 // 64 rows cost each workgroup 4 us) it pays where it reads K and V less often, that is where a workgroup per
 // query head takes more rounds of the CUs than one per KV head, or where the keys are many. Kernel us, ping-pong
 // against decode, 64 rows of one head, by B x H and keys:
 //   D 128   32: n 64 8.5 13.5, n 384 16.2 18.3, n 512 19.6 19.1, n 1024 31 22;   256: n 512 21.8 24.6, n 768 28.1 29.3, n 1024 37 34
 //           1024: n 64 30 48, n 512 86 98, n 768 118 123, n 1024 148 145
 //   D 64    32: n 64 6.7 8.1, n 128 8.1 8.6, n 256 10.6 9.9;   1024: n 64 21 26, n 256 37 40, n 384 47 49, n 512 58 57
-//   32 rows, D 128, 1024: n 64 29.5 18;   two heads of 32 rows, 512 KV heads: n 64 28 25, n 512 78 47
+//   32 rows, D 128, 1024: n 16 28.5 26.1, n 64 29.2 28.8, n 128 35.0 35.6 (not causal 27.2 28.9 at n 64, where it is worst)
+//   two heads of 32 rows, D 128, 512 KV heads: n 64 28 25, n 512 78 47
 bool decode_applies(const AttnShape& sh, int num_cus) {
     const int64_t rows = sh.heads / sh.kv_heads * sh.m;
     if ((sh.d != 64 && sh.d != 128) || rows > kDecodeMaxRows) return false;
